@@ -589,6 +589,53 @@ __device__ __forceinline__ uint32_t wave_min_u32(uint32_t v) {
   return v;
 }
 
+// ---- passes over the slots of a finished table ----
+// The scans that append what they find (dump, Inchworm's seeds) take tiles of
+// 4,096 slots per block of 512 threads, four 16-byte loads in flight per
+// thread, and reserve a tile's output with one atomic on the cursor: with one
+// per wavefront of 64 slots the memory side, which serializes atomics on one
+// address (about 19 ns each), set the pace.  Grids are a few blocks per CU for
+// the same reason (each block ends in at most one more atomic).
+constexpr int kScanThreads = 512;
+constexpr int kScanLoads = 4;  // ulonglong2 per thread and tile
+constexpr uint64_t kScanPairs = (uint64_t)kScanThreads * kScanLoads;
+
+// First output position of this wavefront's `wtot` items of the block's tile.
+// Every thread of the block (kScanThreads) calls it.
+__device__ __forceinline__ uint64_t tile_reserve(uint32_t wtot, unsigned long long* cursor) {
+  __shared__ uint32_t s_w[kScanThreads / 64];
+  __shared__ unsigned long long s_base;
+  const int wv = threadIdx.x >> 6;
+  if ((threadIdx.x & 63) == 0) s_w[wv] = wtot;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    uint32_t tot = 0;
+    for (int i = 0; i < kScanThreads / 64; i++) tot += s_w[i];
+    s_base = tot ? atomicAdd(cursor, (unsigned long long)tot) : 0ull;
+  }
+  __syncthreads();
+  uint64_t at = s_base;
+  for (int i = 0; i < wv; i++) at += s_w[i];
+  __syncthreads();  // s_w and s_base are read before the next tile writes them
+  return at;
+}
+
+// Slot pair u of this thread in the tile at pair `tile` (zeros past the end).
+__device__ __forceinline__ ulonglong2 tile_pair(const uint64_t* slots, uint64_t tile, int u, uint64_t n2) {
+  const uint64_t i = tile + (uint64_t)u * kScanThreads + threadIdx.x;
+  return i < n2 ? reinterpret_cast<const ulonglong2*>(slots)[i] : make_ulonglong2(0ull, 0ull);
+}
+
+// Numbers of A, C and G in a k-mer.
+__device__ __forceinline__ void composition(uint64_t key, int k, int& a, int& c, int& g) {
+  const uint64_t M = 0x5555555555555555ULL & ((1ull << (2 * k)) - 1);  // k <= 31
+  const uint64_t lo = key & M, hi = (key >> 1) & M;
+  const int nt = __popcll(hi & lo);
+  g = __popcll(hi & ~lo & M);
+  c = __popcll(~hi & lo & M);
+  a = k - nt - g - c;
+}
+
 // Bit g of the result is set when nibble g (lanes 4g..4g+3) of x is non-zero.
 __device__ __forceinline__ uint32_t nibble_bits(uint64_t x) {
   x |= x >> 1;

@@ -132,6 +132,9 @@ int select_check(tk_ctx* c, const tk_read_stat* dl, const tk_read_stat* dr, uint
 int select_run(tk_ctx* c, const tk_read_stat* dl, const tk_read_stat* dr, uint64_t n, int max_cov,
                int min_cov, uint8_t* dsel, uint32_t* consumes, uint32_t* idx, void* scan_temp,
                size_t scan_bytes, uint32_t* flags, uint64_t* n_selected);
+// Blocks of a pass over n_slots table slots: four per CU (every thread slot)
+// or one per tile.
+uint32_t scan_grid(const tk_ctx* ctx, uint64_t n_slots);
 // Launch bracket for per-kernel timing on ctx->stream.
 void timing_begin(tk_ctx* ctx, hipEvent_t* a);
 void timing_end(tk_ctx* ctx, const char* name, hipEvent_t a);

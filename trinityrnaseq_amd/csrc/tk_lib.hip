@@ -217,6 +217,13 @@ int collect_timing(tk_ctx* ctx) {
   return TK_OK;
 }
 
+static inline uint64_t ceil_div(uint64_t a, uint64_t b) { return (a + b - 1) / b; }
+
+uint32_t scan_grid(const tk_ctx* ctx, uint64_t n_slots) {
+  const uint64_t tiles = ceil_div(n_slots, 2 * kScanPairs);
+  return (uint32_t)std::max<uint64_t>(1, std::min<uint64_t>(tiles, (uint64_t)std::max(ctx->num_cu, 1) * 4));
+}
+
 #define TK_LAUNCH(ctx, name, grid, block, shmem, kernel, ...)            \
   do {                                                                   \
     hipEvent_t _a;                                                       \
@@ -228,7 +235,6 @@ int collect_timing(tk_ctx* ctx) {
     if (_le != hipSuccess) return ::tk::hip_fail(_le, "launch " name);   \
   } while (0)
 
-static inline uint64_t ceil_div(uint64_t a, uint64_t b) { return (a + b - 1) / b; }
 static inline uint64_t next_pow2(uint64_t x) {
   uint64_t p = 1;
   while (p < x) p <<= 1;
@@ -440,7 +446,7 @@ static int reads_build(tk_ctx* ctx, const char* d_seq, const uint64_t* d_off, ui
     hipError_t e = hipMemsetAsync(ctx->d_flags, 0, 64 * 4, ctx->stream);
     if (e != hipSuccess) { rc = hip_fail(e, "memset flags"); break; }
     {
-      uint64_t grid = std::min<uint64_t>(ceil_div(n + 1, 256), (uint64_t)std::max(ctx->num_cu, 1) * 8);
+      uint64_t grid = std::min<uint64_t>(ceil_div(n + 1, 256), (uint64_t)std::max(ctx->num_cu, 1) * 4);
       hipEvent_t a;
       timing_begin(ctx, &a);
       hipLaunchKernelGGL(k_read_words, dim3(grid), dim3(256), 0, ctx->stream, d_off, n,
@@ -579,7 +585,9 @@ static int reads_windows(tk_ctx* ctx, const tk_reads* rc_, int k, uint64_t* tota
   unsigned long long* d = reinterpret_cast<unsigned long long*>(ctx->d_flags + 8);
   TK_HIP(hipMemsetAsync(d, 0, 8, ctx->stream));
   if (r->n_reads) {
-    uint64_t grid = std::min<uint64_t>(ceil_div(r->n_reads, 256), 4096);
+    // one atomic on the total per block, which the memory side serializes:
+    // four blocks per CU (4,096 blocks took 54 us whatever the read count)
+    uint64_t grid = std::min<uint64_t>(ceil_div(r->n_reads, 256), (uint64_t)std::max(ctx->num_cu, 1) * 4);
     TK_LAUNCH(ctx, "windows", grid, 256, 0, k_windows, r->d_len, r->n_reads, k, d);
   }
   uint64_t h = 0;
@@ -1333,50 +1341,65 @@ __global__ void k_load(const uint64_t* __restrict__ keys, const uint32_t* __rest
 // =====================================================================
 // Dump / histo / prune / lookup over a finalised table
 // =====================================================================
-__global__ void k_dump_count(TableView t, uint64_t n_slots, uint64_t lo, uint64_t hi,
-                             unsigned long long* __restrict__ out) {
+// Count as the tools print it: saturated at 2^32 - 1.
+__device__ __forceinline__ uint64_t slot_count32(const TableView& t, uint64_t s) {
+  const uint64_t v = slot_count(t, s);
+  return v > 0xFFFFFFFFull ? 0xFFFFFFFFull : v;
+}
+
+__global__ __launch_bounds__(kScanThreads) void k_dump_count(TableView t, uint64_t n_slots, uint64_t lo, uint64_t hi,
+                                                             unsigned long long* __restrict__ out) {
+  const uint64_t n2 = n_slots / 2;
   uint64_t c = 0;
-  for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n_slots;
-       i += (uint64_t)gridDim.x * blockDim.x) {
-    const uint64_t s = t.slots[i];
-    if (!s || (s >> t.cshift) == 0) continue;
-    uint64_t v = slot_count(t, s);
-    v = v > 0xFFFFFFFFull ? 0xFFFFFFFFull : v;  // counts print saturated at 2^32-1
-    c += (v >= lo && v <= hi);
+  for (uint64_t tile = blockIdx.x * kScanPairs; tile < n2; tile += gridDim.x * kScanPairs) {
+    ulonglong2 v[kScanLoads];
+#pragma unroll
+    for (int u = 0; u < kScanLoads; u++) v[u] = tile_pair(t.slots, tile, u, n2);
+#pragma unroll
+    for (int u = 0; u < 2 * kScanLoads; u++) {
+      const uint64_t s = u & 1 ? v[u >> 1].y : v[u >> 1].x;
+      if (!s || (s >> t.cshift) == 0) continue;
+      const uint64_t n = slot_count32(t, s);
+      c += (n >= lo && n <= hi);
+    }
   }
   block_sum_add(c, out);
 }
 
-// Keys with count in [lo, hi] and key in [klo, khi] appended at *cursor.
-__global__ void k_dump(TableView t, uint64_t n_slots, uint64_t lo, uint64_t hi, uint64_t klo, uint64_t khi,
-                       uint64_t* __restrict__ keys, uint32_t* __restrict__ counts,
-                       uint64_t cap, unsigned long long* __restrict__ cursor) {
-  const int lane = threadIdx.x & 63;
-  for (uint64_t base = (uint64_t)blockIdx.x * blockDim.x; base < n_slots;
-       base += (uint64_t)gridDim.x * blockDim.x) {
-    const uint64_t i = base + threadIdx.x;
-    bool take = false;
-    uint64_t key = 0, v = 0;
-    if (i < n_slots) {
-      const uint64_t s = t.slots[i];
-      if (s && (s >> t.cshift) != 0) {
-        v = slot_count(t, s);
-        v = v > 0xFFFFFFFFull ? 0xFFFFFFFFull : v;
-        key = s & (t.occ - 1);
-        take = v >= lo && v <= hi && key >= klo && key <= khi;
-      }
+// Keys with count in [lo, hi] and key in [klo, khi] appended at *cursor
+// (1 M strand-specific 125-nt reads' table: 17.7 ms with an atomic per
+// wavefront, 0.33 ms now; its k_dump_count 0.81 -> 0.13 ms, k_prune on 120 k
+// reads 255 -> 31 us).
+__global__ __launch_bounds__(kScanThreads) void k_dump(TableView t, uint64_t n_slots, uint64_t lo, uint64_t hi,
+                                                       uint64_t klo, uint64_t khi, uint64_t* __restrict__ keys,
+                                                       uint32_t* __restrict__ counts, uint64_t cap,
+                                                       unsigned long long* __restrict__ cursor) {
+  const uint64_t n2 = n_slots / 2;
+  const uint64_t below = (1ull << (threadIdx.x & 63)) - 1;
+  for (uint64_t tile = blockIdx.x * kScanPairs; tile < n2; tile += gridDim.x * kScanPairs) {
+    ulonglong2 v[kScanLoads];
+    uint32_t n[2 * kScanLoads];
+    uint64_t m[2 * kScanLoads];
+#pragma unroll
+    for (int u = 0; u < kScanLoads; u++) v[u] = tile_pair(t.slots, tile, u, n2);
+    uint32_t wtot = 0;
+#pragma unroll
+    for (int u = 0; u < 2 * kScanLoads; u++) {
+      const uint64_t s = u & 1 ? v[u >> 1].y : v[u >> 1].x;
+      const uint64_t key = s & (t.occ - 1);
+      n[u] = s && (s >> t.cshift) != 0 ? (uint32_t)slot_count32(t, s) : 0u;
+      m[u] = __ballot(n[u] && n[u] >= lo && n[u] <= hi && key >= klo && key <= khi);
+      wtot += (uint32_t)__popcll(m[u]);
     }
-    const uint64_t m = __ballot(take);
-    if (!m) continue;
-    unsigned long long start = 0;
-    if (lane == 0) start = atomicAdd(cursor, (unsigned long long)__popcll(m));
-    start = __shfl(start, 0);
-    if (take) {
-      const uint64_t pos = start + __popcll(m & ((1ull << lane) - 1));
-      if (pos < cap) {
-        keys[pos] = key;
-        counts[pos] = v > 0xFFFFFFFFull ? 0xFFFFFFFFu : (uint32_t)v;
+    uint64_t at = tile_reserve(wtot, cursor);
+#pragma unroll
+    for (int u = 0; u < 2 * kScanLoads; u++) {
+      const uint64_t pos = at + (uint32_t)__popcll(m[u] & below);
+      if (((m[u] >> (threadIdx.x & 63)) & 1ull) && pos < cap) {
+        keys[pos] = (u & 1 ? v[u >> 1].y : v[u >> 1].x) & (t.occ - 1);
+        counts[pos] = n[u];
       }
+      at += (uint32_t)__popcll(m[u]);
     }
   }
 }
@@ -1416,7 +1439,7 @@ __global__ __launch_bounds__(256) void k_dump_bins(TableView t, uint64_t n_slots
 // 10,001 bins fit) are LDS counters, flushed once per block; only bins from
 // `nl` on, counts past 15,359 steps, go to device memory one by one.
 // Persistent blocks of 1,024 threads, two per CU (60 KB of LDS each at most),
-// two 16-byte loads in flight per thread.
+// two 16-byte loads in flight per thread (0.23 ms).
 constexpr uint32_t kHistoBins = 15360;
 
 __global__ __launch_bounds__(1024) void k_histo(TableView t, uint64_t n_slots, uint64_t base, uint64_t ceil_,
@@ -1449,41 +1472,41 @@ __global__ __launch_bounds__(1024) void k_histo(TableView t, uint64_t n_slots, u
     if (s_hist[i]) atomicAdd(&bins[i], (unsigned long long)s_hist[i]);
 }
 
-__device__ __forceinline__ void composition(uint64_t key, int k, int& a, int& c, int& g) {
-  const uint64_t M = (k == 32) ? 0x5555555555555555ULL
-                               : (0x5555555555555555ULL & ((1ull << (2 * k)) - 1));
-  const uint64_t lo = key & M, hi = (key >> 1) & M;
-  const int nt = __popcll(hi & lo);
-  g = __popcll(hi & ~lo & M);
-  c = __popcll(~hi & lo & M);
-  a = k - nt - g - c;
-}
-
-__global__ void k_prune(TableView t, uint64_t n_slots, int k, uint64_t min_count,
-                        const uint8_t* __restrict__ keep, unsigned long long* __restrict__ kept) {
-  uint64_t nk = 0;
+// Thread per slot pair; the composition table (kt bytes, 0 = keep every key)
+// sits in LDS.
+__global__ __launch_bounds__(kScanThreads) void k_prune(TableView t, uint64_t n_slots, int k, uint64_t min_count,
+                                                        const uint8_t* __restrict__ keep, uint32_t kt,
+                                                        unsigned long long* __restrict__ kept) {
+  extern __shared__ uint8_t s_keep[];
+  for (uint32_t i = threadIdx.x; i < kt; i += blockDim.x) s_keep[i] = keep[i];
+  __syncthreads();
+  const uint64_t n2 = n_slots / 2;
   const int K1 = k + 1;
-  for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n_slots;
-       i += (uint64_t)gridDim.x * blockDim.x) {
-    const uint64_t s = t.slots[i];
-    if (!s) continue;
-    const uint64_t f = s >> t.cshift;
-    if (f == 0) continue;
-    const uint64_t v = slot_count(t, s);
-    bool ok = v >= min_count;
-    if (ok && keep) {
-      int a, c, g;
-      composition(s & (t.occ - 1), k, a, c, g);
-      ok = keep[(a * K1 + c) * K1 + g] != 0;
-    }
-    if (ok) {
-      nk++;
-    } else {
-      if (f == t.cmax) {
-        uint64_t* o = ovf_find(t, s & t.kmo);
-        if (o) *o = 0;
+  uint64_t nk = 0;
+  for (uint64_t tile = blockIdx.x * kScanPairs; tile < n2; tile += gridDim.x * kScanPairs) {
+    ulonglong2 v[kScanLoads];
+#pragma unroll
+    for (int u = 0; u < kScanLoads; u++) v[u] = tile_pair(t.slots, tile, u, n2);
+#pragma unroll
+    for (int u = 0; u < 2 * kScanLoads; u++) {
+      const uint64_t s = u & 1 ? v[u >> 1].y : v[u >> 1].x;
+      const uint64_t f = s >> t.cshift;
+      if (f == 0) continue;
+      bool ok = slot_count(t, s) >= min_count;
+      if (ok && kt) {
+        int a, c, g;
+        composition(s & (t.occ - 1), k, a, c, g);
+        ok = s_keep[(a * K1 + c) * K1 + g] != 0;
       }
-      t.slots[i] = s & t.kmo;
+      if (ok) {
+        nk++;
+      } else {
+        if (f == t.cmax) {
+          uint64_t* o = ovf_find(t, s & t.kmo);
+          if (o) *o = 0;
+        }
+        t.slots[2 * (tile + (uint64_t)(u >> 1) * kScanThreads + threadIdx.x) + (u & 1)] = s & t.kmo;
+      }
     }
   }
   block_sum_add(nk, kept);
@@ -3073,8 +3096,7 @@ int tk_table_dump_size(tk_ctx* c, tk_table* t, uint32_t lo, uint32_t hi, uint64_
   TK_HIP(hipMemsetAsync(d, 0, 8, c->stream));
   TableView v = table_view(t);
   uint64_t ns = t->nb * 8;
-  TK_LAUNCH(c, "dump_count", std::min<uint64_t>(ceil_div(ns, 256), 65536), 256, 0, k_dump_count,
-            v, ns, (uint64_t)lo, (uint64_t)hi, d);
+  TK_LAUNCH(c, "dump_count", scan_grid(c, ns), kScanThreads, 0, k_dump_count, v, ns, (uint64_t)lo, (uint64_t)hi, d);
   uint64_t h = 0;
   TK_HIP(hipMemcpyAsync(&h, d, 8, hipMemcpyDeviceToHost, c->stream));
   TK_HIP(hipStreamSynchronize(c->stream));
@@ -3108,8 +3130,8 @@ static int dump_range(tk_ctx* c, tk_table* t, uint32_t lo, uint32_t hi, uint64_t
   TK_HIP(hipMemsetAsync(cur, 0, 8, c->stream));
   TableView v = table_view(t);
   const uint64_t ns = t->nb * 8;
-  TK_LAUNCH(c, "dump", std::min<uint64_t>(ceil_div(ns, 256), 65536), 256, 0, k_dump, v, ns, (uint64_t)lo,
-            (uint64_t)hi, klo, khi, dk, dc, n, cur);
+  TK_LAUNCH(c, "dump", scan_grid(c, ns), kScanThreads, 0, k_dump, v, ns, (uint64_t)lo, (uint64_t)hi, klo, khi, dk, dc,
+            n, cur);
   uint64_t got = 0;
   TK_HIP(hipMemcpyAsync(&got, cur, 8, hipMemcpyDeviceToHost, c->stream));
   TK_HIP(hipStreamSynchronize(c->stream));
@@ -3163,7 +3185,7 @@ int tk_table_dump(tk_ctx* c, tk_table* t, uint32_t lo, uint32_t hi, uint64_t* ke
     TK_HIP(hipMemsetAsync(pbins, 0, nb * 8, c->stream));
     TableView v = table_view(t);
     const uint64_t ns = t->nb * 8;
-    TK_LAUNCH(c, "dump_bins", std::min<uint64_t>(ceil_div(ns, 256), 65536), 256, 0, k_dump_bins, v, ns,
+    TK_LAUNCH(c, "dump_bins", std::min<uint64_t>(ceil_div(ns, 256), (uint64_t)std::max(c->num_cu, 1) * 8), 256, 0, k_dump_bins, v, ns,
               (uint64_t)lo, (uint64_t)hi, r.klo, r.khi, shift, (unsigned long long*)pbins);
     TK_HIP(hipMemcpyAsync(bins.data(), pbins, nb * 8, hipMemcpyDeviceToHost, c->stream));
     TK_HIP(hipStreamSynchronize(c->stream));
@@ -3258,8 +3280,8 @@ int tk_table_prune(tk_ctx* c, tk_table* t, uint32_t min_count, const uint8_t* ke
   TK_HIP(hipMemsetAsync(d, 0, 8, c->stream));
   TableView v = table_view(t);
   uint64_t ns = t->nb * 8;
-  TK_LAUNCH(c, "prune", std::min<uint64_t>(ceil_div(ns, 256), 65536), 256, 0, k_prune, v, ns, t->k,
-            (uint64_t)min_count, dkeep, d);
+  const uint32_t kt32 = keep ? (uint32_t)kt : 0;  // at most 32^3 bytes
+  TK_LAUNCH(c, "prune", scan_grid(c, ns), kScanThreads, kt32, k_prune, v, ns, t->k, (uint64_t)min_count, dkeep, kt32, d);
   uint64_t h = 0;
   TK_HIP(hipMemcpyAsync(&h, d, 8, hipMemcpyDeviceToHost, c->stream));
   TK_HIP(hipStreamSynchronize(c->stream));
