@@ -1,0 +1,86 @@
+"""Per-read passes at the read lengths where their runs end (64, 128 and 256
+windows), with counts on both sides of the 32-bit sums, against the oracle (GPU)."""
+from __future__ import annotations
+
+import numpy as np
+import pytest
+
+from data import concat
+from oracle import oracle as O
+
+pytestmark = pytest.mark.gpu
+
+WINDOWS = [0, 1, 2, 31, 32, 33, 63, 64, 65, 96, 126, 127, 128, 129, 160, 191, 192, 193, 254, 255, 256, 257, 400]
+LARGE = [5792, 5793, 4095, 4096, 8190, 8191, 8192, 2**20, 2**31, 2**32 - 1]
+
+
+@pytest.fixture(scope="module")
+def api():
+    from trinityrnaseq_amd import api as A
+    return A
+
+
+def _reads(k, longest, n_rate, seed):
+    """Three reads of every window count up to `longest` (and some shorter than k), the longest last."""
+    rng = np.random.default_rng(seed)
+    out = ["", "ACGT"]
+    for w in sorted(WINDOWS):
+        if w > longest:
+            continue
+        for _ in range(3):
+            s = rng.choice(list("ACGT"), size=w + k - 1 if w else k - 1)
+            s[rng.random(len(s)) < n_rate] = "N"
+            out.append("".join(s))
+    return out
+
+
+@pytest.mark.parametrize("pipe", ["1", "0"])
+@pytest.mark.parametrize("k,canonical", [(25, True), (25, False), (31, True), (13, True), (16, True)])
+@pytest.mark.parametrize("longest", [64, 128, 256, 400])
+def test_stats_run_ends(api, ctx, monkeypatch, longest, k, canonical, pipe):
+    print("stats_run_ends", longest, k, canonical, pipe, flush=True)
+    monkeypatch.setenv("TK_STATS_PIPE", pipe)
+    seqs = _reads(k, longest, 0.004, 11 + longest)
+    seq, off = concat(seqs)
+    keys, counts = O.count(seq, off, k, canonical)
+    rng = np.random.default_rng(3)
+    reads = api.Reads(ctx, seq, off)
+    for large in (False, True):
+        c = rng.choice([1, 2, 3, 7, 50, 5792, 4095] if not large else [1, 2, 9] + LARGE, size=len(keys)).astype(np.uint32)
+        here = rng.random(len(keys)) < 0.8
+        t = api.Table(ctx, k, canonical, len(keys), 0.7)
+        t.load(keys[here], c[here])
+        for nwin, med in [(0, 0), (1, 1), (0, 2)]:
+            got = api.read_cov_stats(ctx, t, reads, min_count=2, nwin_policy=nwin, median_policy=med)
+            want = O.read_stats(seq, off, keys[here], c[here], k, canonical, 2, 1, nwin, med)
+            assert np.array_equal(got, want.astype(got.dtype)), (large, nwin, med)
+        t.free()
+    reads.free()
+
+
+@pytest.mark.parametrize("pipe", ["1", "0"])
+@pytest.mark.parametrize("k,canonical", [(25, True), (25, False), (31, True), (13, True)])
+@pytest.mark.parametrize("longest", [64, 128, 400])
+def test_vote_run_ends(api, ctx, monkeypatch, longest, k, canonical, pipe):
+    """Each read's windows spread over several components, ties among them."""
+    print("vote_run_ends", longest, k, canonical, pipe, flush=True)
+    monkeypatch.setenv("TK_VOTE_PIPE", pipe)
+    seqs = _reads(k, longest, 0.004, 5 + longest)
+    rng = np.random.default_rng(4)
+    pieces, comps = [], []
+    for s in seqs:
+        for a in range(0, len(s) - k + 1, 9):
+            if rng.random() < 0.7:
+                pieces.append(s[a:a + k + 5])
+                comps.append(int(rng.choice([0, 1, 2, 7, 2**32 - 2])))
+    comps = np.array(comps, np.uint32)
+    seq, off = concat(seqs)
+    cseq, coff = concat(pieces)
+    reads, bundles = api.Reads(ctx, seq, off), api.Reads(ctx, cseq, coff)
+    ct = api.CTable(ctx, bundles, comps, k, canonical)
+    bk, bc = O.r2t_build(cseq, coff, comps, k, canonical)
+    got = ct.vote(reads)
+    want = O.r2t_vote(seq, off, bk, bc, k, canonical)
+    assert np.array_equal(got, want.astype(got.dtype))
+    for o in (ct, bundles, reads):
+        o.free()

@@ -319,7 +319,7 @@ __global__ __launch_bounds__(256) void k_batch_vote(ReadsView rv, const uint32_t
   const int wv = threadIdx.x >> 6;
   const uint64_t wpb = blockDim.x >> 6;
   uint32_t* hits = s_dyn + (uint64_t)wv * slab;
-  uint32_t* tmp = s_dyn + wpb * slab + wv * 64;
+  uint64_t* tmp = reinterpret_cast<uint64_t*>(s_dyn + wpb * slab) + wv * kLookupScratch;
   for (uint64_t r = (uint64_t)blockIdx.x * wpb + wv; r < rv.n_reads; r += (uint64_t)gridDim.x * wpb) {
     const CompLayout L = lay[read_comp[r]];
     vote_read<kPacked>(rv, r, k, canonical, ct, L.ct_boff, L.ct_mask, hits, tmp, lane, out + r);
@@ -532,7 +532,7 @@ static int batch_enqueue(tk_ctx* c, tk_batch* b, const tk_stats_opts* o, tk_read
   if (d_votes && rv.n_reads) {
     hipLaunchKernelGGL(k_fill_zero, dim3(grid(b->n_ct_words, 256)), dim3(256), 0, c->stream, b->d_ct, b->n_ct_words);
     const ReadsView cv = rview(b->contigs);
-    const size_t vlds = (size_t)slab * 4 * wpb + (size_t)wpb * 256;
+    const size_t vlds = ((size_t)slab * 4 + 8 * kLookupScratch) * wpb;
     if (b->n_ct_lds && b->ct_packed)
       hipLaunchKernelGGL(k_batch_ctable_lds<true>, dim3((unsigned)b->n_ct_lds), dim3(256), b->ct_lds_bytes, c->stream,
                          cv, b->d_ct_lds, b->d_contig_off, b->d_lay, b->k, b->canonical, b->d_ct, c->d_flags);

@@ -5,8 +5,9 @@
 //   nmask[w]  : 32-bit word, bit 31-i set when base i of codes[w] is not ACGT
 //   word_off[r]: first word of read r (each read starts on a fresh word)
 //   len[r]    : bases in read r
-// One zero padding word follows the last read, so a window extractor may
-// always read words w and w+1.
+// kWordPad padding words (code 0, every base invalid) follow the last read, so
+// a window extractor may always read words w and w+1, and a lane of a
+// per-read kernel the four words from its own on (lane_words).
 //
 // Count table (tk_table): open addressing over 64-byte buckets of eight
 // 64-bit slots.  A slot packs
@@ -31,7 +32,9 @@ namespace tk {
 
 constexpr int kWave = 64;
 constexpr int kBucketSlots = 8;
-// u64 entries of LDS lookup scratch per wavefront (coop4_get with two keys per lane)
+constexpr int kWordPad = 16;
+// u64 entries of LDS lookup scratch per wavefront (coop_lookup: 64 two-word
+// entries, then up to 128 values)
 constexpr int kLookupScratch = 128;
 
 __host__ __device__ __forceinline__ uint64_t mix64(uint64_t x) {
@@ -43,13 +46,11 @@ __host__ __device__ __forceinline__ uint64_t mix64(uint64_t x) {
   return x;
 }
 
-// Reverse complement of a k-mer held in the low 2k bits.
+// Reverse complement of a k-mer held in the low 2k bits: the bits reversed
+// (bases reversed, the two bits of each swapped), the pairs swapped back.
 __device__ __forceinline__ uint64_t revcomp(uint64_t v, int k) {
-  uint64_t x = ~v;
-  x = ((x >> 2) & 0x3333333333333333ULL) | ((x & 0x3333333333333333ULL) << 2);
-  x = ((x >> 4) & 0x0F0F0F0F0F0F0F0FULL) | ((x & 0x0F0F0F0F0F0F0F0FULL) << 4);
-  x = __builtin_bswap64(x);
-  return x >> (64 - 2 * k);
+  const uint64_t x = __builtin_bitreverse64(~v);
+  return (((x >> 1) & 0x5555555555555555ULL) | ((x & 0x5555555555555555ULL) << 1)) >> (64 - 2 * k);
 }
 
 struct ReadsView {
@@ -125,7 +126,7 @@ struct TicketStream {
   __device__ __forceinline__ uint32_t next() {
     if (cb == ce) {
       if (done) return n;
-      const uint32_t s = __shfl(tk, 0);
+      const uint32_t s = __builtin_amdgcn_readfirstlane(tk);
       if (s >= n) {
         done = true;
         return n;
@@ -170,19 +171,33 @@ __device__ __forceinline__ void window_at_mask(const ReadsView& rv, uint64_t wba
   nmask = m >> (32 - k);
 }
 
-// window_at over a read whose words are spread over the wave: lane j holds
-// code word j of the read (cw) and its mask word (mw), for j up to the word
-// after the read's last.  pos < 128, so words 0..4 are read.
-__device__ __forceinline__ void window_lanes(uint64_t cw, uint32_t mw, uint32_t pos, int k, uint64_t& fwd,
-                                             bool& valid) {
-  const int w = (int)(pos >> 5);
-  const uint32_t o = pos & 31u;
-  const uint64_t hi = __shfl(cw, w);
-  const uint64_t lo = __shfl(cw, w + 1);
-  const uint32_t mhi = __shfl(mw, w);
-  const uint32_t mlo = __shfl(mw, w + 1);
-  const uint64_t x = o ? ((hi << (2 * o)) | (lo >> (64 - 2 * o))) : hi;
-  const uint32_t m = o ? ((mhi << o) | (mlo >> (32 - o))) : mhi;
+// The words a lane needs for its two windows of a run of 128 (windows lane and
+// 64 + lane of a read whose words start at wb): words lane/32 .. lane/32 + 3.
+// Every lane loads its own (three 16-byte loads, one or two lines per wave),
+// which replaced words spread over the lanes and fetched with six shuffles per
+// window.  Words are 8-byte aligned, masks 4-byte: the vector types say so.
+typedef uint64_t words2 __attribute__((ext_vector_type(2), aligned(8)));
+typedef uint32_t masks4 __attribute__((ext_vector_type(4), aligned(4)));
+
+struct LaneWords {
+  words2 a, b;  // words 0-1 and 2-3
+  masks4 m;
+};
+
+__device__ __forceinline__ LaneWords lane_words(const ReadsView& rv, uint64_t wb, int lane) {
+  const uint32_t j = (uint32_t)lane >> 5;
+  LaneWords w;
+  w.a = *reinterpret_cast<const words2*>(rv.codes + wb + j);
+  w.b = *reinterpret_cast<const words2*>(rv.codes + wb + j + 2);
+  w.m = *reinterpret_cast<const masks4*>(rv.nmask + wb + j);
+  return w;
+}
+
+// Forward k-mer at base o (< 32) of the word pair (hi, lo) with masks (mhi, mlo).
+__device__ __forceinline__ void pair_window(uint64_t hi, uint64_t lo, uint32_t mhi, uint32_t mlo, uint32_t o, int k,
+                                            uint64_t& fwd, bool& valid) {
+  const uint64_t x = (hi << (2 * o)) | ((lo >> 1) >> (63 - 2 * o));
+  const uint32_t m = (mhi << o) | ((mlo >> 1) >> (31 - o));
   fwd = x >> (64 - 2 * k);
   valid = (m >> (32 - k)) == 0u;
 }
@@ -209,8 +224,17 @@ struct TableView {
   uint32_t max_probe; // buckets probed before giving up
 };
 
+// High 64 bits of h * n.  n (a table's buckets) is the same for every lane
+// and below 2^32 but for tables of 256 GB, so half of the product's four
+// quarter-rate 32-bit multiplies go, behind a scalar branch.
+__device__ __forceinline__ uint64_t mulhi_n(uint64_t h, uint64_t n) {
+  if (n >> 32) return __umul64hi(h, n);
+  const uint32_t n32 = (uint32_t)n;
+  return ((uint64_t)(uint32_t)(h >> 32) * n32 + __umulhi((uint32_t)h, n32)) >> 32;
+}
+
 __device__ __forceinline__ uint64_t bucket0(const TableView& t, uint64_t key) {
-  return t.boff + __umul64hi(mix64(key), t.nb);
+  return t.boff + mulhi_n(mix64(key), t.nb);
 }
 __device__ __forceinline__ uint64_t bucket_next(const TableView& t, uint64_t b) {
   const uint64_t r = b - t.boff;
@@ -567,26 +591,31 @@ __device__ __forceinline__ void block_sum_add(uint64_t v, unsigned long long* ou
     if (tot) atomicAdd(out, (unsigned long long)tot);
   }
 }
+// Wave reductions of 32-bit values on the DPP row shifts and row broadcasts
+// (one VALU instruction per step; a shuffle is an address, an LDS permute and
+// a wait).  All 64 lanes must be active; the result is wave-uniform.
+template <int kCtrl, int kRows>
+__device__ __forceinline__ uint32_t dpp_u32(uint32_t identity, uint32_t v) {
+  return (uint32_t)__builtin_amdgcn_update_dpp((int)identity, (int)v, kCtrl, kRows, 0xF, false);
+}
+template <class Op>
+__device__ __forceinline__ uint32_t wave_reduce_u32(uint32_t v, uint32_t identity, Op op) {
+  v = op(v, dpp_u32<0x111, 0xF>(identity, v));  // row_shr:1
+  v = op(v, dpp_u32<0x112, 0xF>(identity, v));  // row_shr:2
+  v = op(v, dpp_u32<0x114, 0xF>(identity, v));  // row_shr:4
+  v = op(v, dpp_u32<0x118, 0xF>(identity, v));  // row_shr:8: lane 15 of a row holds the row's result
+  v = op(v, dpp_u32<0x142, 0xA>(identity, v));  // row_bcast:15 into rows 1 and 3
+  v = op(v, dpp_u32<0x143, 0xC>(identity, v));  // row_bcast:31 into rows 2 and 3
+  return (uint32_t)__builtin_amdgcn_readlane((int)v, 63);
+}
 __device__ __forceinline__ uint32_t wave_sum_u32(uint32_t v) {
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o);
-  return v;
+  return wave_reduce_u32(v, 0u, [](uint32_t a, uint32_t b) { return a + b; });
 }
 __device__ __forceinline__ uint32_t wave_max_u32(uint32_t v) {
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) {
-    uint32_t w = __shfl_xor(v, o);
-    v = w > v ? w : v;
-  }
-  return v;
+  return wave_reduce_u32(v, 0u, [](uint32_t a, uint32_t b) { return a > b ? a : b; });
 }
 __device__ __forceinline__ uint32_t wave_min_u32(uint32_t v) {
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) {
-    uint32_t w = __shfl_xor(v, o);
-    v = w < v ? w : v;
-  }
-  return v;
+  return wave_reduce_u32(v, 0xFFFFFFFFu, [](uint32_t a, uint32_t b) { return a < b ? a : b; });
 }
 
 // ---- passes over the slots of a finished table ----
@@ -649,67 +678,130 @@ __device__ __forceinline__ uint32_t nibble_bits(uint64_t x) {
 
 // Cooperative lookup of 64*NK keys, NK per lane (key i of a lane is key
 // number 64*i + lane), four lanes per key.  In round q the lanes 4g..4g+3
-// read the 64-byte home bucket of key 16q+g, sixteen bytes (two slots) each:
-// one coalesced request per key, as with eight lanes, but half the load,
-// shuffle and compare instructions.  All 4*NK loads of a lane are issued
-// before any is inspected.  Whether the bucket matched or held an empty slot
-// reaches the key's own lane through the round's ballots; the matching lane
-// passes the raw count field through `val` (64*NK x u64, LDS).  A key whose
-// home bucket is full without a match continues with a full probe.  out[i]
-// is the count of key i (0 = absent or pruned); lanes with want[i] = false
-// take part in the rounds (their bucket is not read) and get 0.
-template <int NK>
-__device__ __forceinline__ void coop4_get(const TableView& t, const uint64_t (&key)[NK],
-                                          const bool (&want)[NK], uint64_t* val, int lane,
-                                          uint64_t (&out)[NK]) {
+// read the 64-byte home bucket of key 16q+g, sixteen bytes each: one
+// coalesced request per key.  All 4*NK loads of a lane are issued before any
+// is inspected.
+//
+// The kernels that call this are bound by instruction issue as much as by
+// their misses (the scoring pass issued vector instructions in 76% of its
+// cycles), so the exchange between a key's lane and its group goes through
+// LDS: the lane writes {bucket offset, tagged key} once and the group reads
+// both with one broadcast 16-byte read per round (five shuffles before).  The
+// matching lane writes the key's value back; a group whose bucket is full
+// (its last lane sees no empty slot; occupied slots are a prefix) first
+// leaves kLookupFull there, which a match overwrites (the LDS operations of a
+// wave execute in order), and the key's lane then probes on alone.
+//
+// off[i]: byte offset of the home bucket from `slots`.  Layout L: match(slots,
+// tag, value) for the lane's sixteen bytes, full(slots) for the bucket's last
+// sixteen, kNone the value of an absent key.  A lane without a key asks for
+// bucket 0 with tag 0 (no branch around the loads) and ignores its value.
+// scratch: kLookupScratch u64.
+constexpr uint64_t kLookupFull = ~0ull;
+
+template <int NK, class L>
+__device__ __forceinline__ void coop_lookup(const uint64_t* slots, const L& lay, const uint64_t (&off)[NK],
+                                            const uint64_t (&tag)[NK], uint64_t* scratch, int lane,
+                                            uint64_t (&out)[NK]) {
   constexpr int R = 4 * NK;
+  static_assert(64 * NK <= kLookupScratch, "scratch holds one value per key");
   const int g = lane >> 2, sl = lane & 3;
-  uint64_t b[NK], tg[NK];
-#pragma unroll
-  for (int i = 0; i < NK; i++) {
-    b[i] = bucket0(t, key[i]);
-    tg[i] = key[i] | t.occ;
-  }
+  ulonglong2* ent = reinterpret_cast<ulonglong2*>(scratch);
+  const char* base = reinterpret_cast<const char*>(slots) + 16 * sl;
   ulonglong2 sv[R];
-#pragma unroll
-  for (int q = 0; q < R; q++) {
-    const uint64_t bq = __shfl(b[q >> 2], (q & 3) * 16 + g);
-    const int wq = __shfl((int)want[q >> 2], (q & 3) * 16 + g);
-    sv[q] = wq ? reinterpret_cast<const ulonglong2*>(t.slots + (bq << 3))[sl] : make_ulonglong2(0, 0);
-  }
-  uint64_t mbs[R], ebs[R];
-#pragma unroll
-  for (int q = 0; q < R; q++) {
-    const uint64_t tq = __shfl(tg[q >> 2], (q & 3) * 16 + g);
-    const bool m0 = (sv[q].x & t.kmo) == tq;
-    const bool m1 = (sv[q].y & t.kmo) == tq;
-    if (m0 | m1) val[16 * q + g] = (m0 ? sv[q].x : sv[q].y) >> t.cshift;
-    mbs[q] = __ballot(m0 | m1);
-    ebs[q] = __ballot((sv[q].x == 0) | (sv[q].y == 0));
-  }
-  wave_sync();
-  const int qq = lane >> 4, sh = (lane & 15) * 4;
+  uint64_t tq[R];
 #pragma unroll
   for (int i = 0; i < NK; i++) {
-    const uint64_t mq = qq == 0 ? mbs[4 * i] : qq == 1 ? mbs[4 * i + 1] : qq == 2 ? mbs[4 * i + 2] : mbs[4 * i + 3];
-    const uint64_t eq = qq == 0 ? ebs[4 * i] : qq == 1 ? ebs[4 * i + 1] : qq == 2 ? ebs[4 * i + 2] : ebs[4 * i + 3];
-    const bool hit = (mq >> sh) & 0xFull;
-    const bool empty = (eq >> sh) & 0xFull;
-    uint64_t f = 0;
-    if (want[i]) {
-      if (hit) {
-        f = val[64 * i + lane];
-        if (f == t.cmax) {
-          const uint64_t* o = ovf_find(t, tg[i]);
-          f = o ? *o : f;
-        }
-      } else if (!empty) {
-        f = table_get(t, key[i]);
-      }
+    ent[lane] = make_ulonglong2(off[i], tag[i]);
+    wave_sync();
+#pragma unroll
+    for (int q = 4 * i; q < 4 * i + 4; q++) {
+      const ulonglong2 e = ent[(q & 3) * 16 + g];
+      tq[q] = e.y;
+      sv[q] = *reinterpret_cast<const ulonglong2*>(base + e.x);
     }
-    out[i] = f;
+    wave_sync();
+  }
+#pragma unroll
+  for (int i = 0; i < NK; i++) scratch[64 * i + lane] = L::kNone;
+  wave_sync();
+#pragma unroll
+  for (int q = 0; q < R; q++)
+    if (sl == 3 && L::full(sv[q])) scratch[16 * q + g] = kLookupFull;
+  wave_sync();
+#pragma unroll
+  for (int q = 0; q < R; q++) {
+    uint64_t v;
+    if (lay.match(sv[q], tq[q], v)) scratch[16 * q + g] = v;
   }
   wave_sync();
+#pragma unroll
+  for (int i = 0; i < NK; i++) out[i] = scratch[64 * i + lane];
+  wave_sync();
+}
+
+// The count table's slots: the value is the raw count field.
+struct CountLayout {
+  static constexpr uint64_t kNone = 0;
+  uint64_t kmo;
+  uint32_t cshift;
+  __device__ __forceinline__ bool match(const ulonglong2& s, uint64_t tag, uint64_t& v) const {
+    const bool m0 = (s.x & kmo) == tag, m1 = (s.y & kmo) == tag;
+    v = (m0 ? s.x : s.y) >> cshift;
+    return m0 | m1;
+  }
+  static __device__ __forceinline__ bool full(const ulonglong2& s) { return s.y != 0; }
+};
+
+// Raw count field of a key whose home bucket is full and does not hold it (0 =
+// absent): the buckets after it, each read whole, its slots compared without
+// branches (about one absent key in twenty comes here at load 0.5).
+__device__ __forceinline__ uint64_t table_field_after(const TableView& t, uint64_t tagged) {
+  uint64_t b = bucket0(t, tagged & (t.occ - 1));
+  for (uint32_t p = 1; p < t.max_probe; p++) {
+    b = bucket_next(t, b);
+    const ulonglong2* l2 = reinterpret_cast<const ulonglong2*>(t.slots + (b << 3));
+    const ulonglong2 v[4] = {l2[0], l2[1], l2[2], l2[3]};
+    uint64_t hit = 0;
+#pragma unroll
+    for (int j = 0; j < 4; j++) {
+      hit = (v[j].x & t.kmo) == tagged ? v[j].x : hit;
+      hit = (v[j].y & t.kmo) == tagged ? v[j].y : hit;
+    }
+    if (hit) return hit >> t.cshift;
+    if (v[3].y == 0) return 0;
+  }
+  return 0;
+}
+
+// Counts of the keys (0 = absent or pruned; want[i] = false: 0).
+template <int NK>
+__device__ __forceinline__ void coop4_get(const TableView& t, const uint64_t (&key)[NK], const bool (&want)[NK],
+                                          uint64_t* scratch, int lane, uint64_t (&out)[NK]) {
+  uint64_t off[NK], tag[NK];
+#pragma unroll
+  for (int i = 0; i < NK; i++) {
+    off[i] = want[i] ? bucket0(t, key[i]) << 6 : 0;
+    tag[i] = want[i] ? key[i] | t.occ : 0;
+  }
+  coop_lookup<NK>(t.slots, CountLayout{t.kmo, t.cshift}, off, tag, scratch, lane, out);
+#pragma unroll
+  for (int i = 0; i < NK; i++) {
+    out[i] = want[i] ? out[i] : 0;
+    if (out[i] == kLookupFull) out[i] = table_field_after(t, tag[i]);
+  }
+  // all-ones fields: the count is in the side table
+  bool side = false;
+#pragma unroll
+  for (int i = 0; i < NK; i++) side = side || out[i] == t.cmax;
+  if (side) {
+#pragma unroll
+    for (int i = 0; i < NK; i++)
+      if (out[i] == t.cmax) {
+        const uint64_t* o = ovf_find(t, tag[i]);
+        out[i] = o ? *o : out[i];
+      }
+  }
 }
 
 // Cooperative +1 of the 64 keys held one per lane (want = lane has a key).

@@ -74,8 +74,8 @@ struct tk_reads {
   uint32_t max_len = 0;
   uint32_t* d_len = nullptr;
   uint64_t* d_word_off = nullptr;  // n_reads + 1
-  uint64_t* d_codes = nullptr;     // n_words + 1
-  uint32_t* d_nmask = nullptr;     // n_words + 1
+  uint64_t* d_codes = nullptr;     // n_words + kWordPad
+  uint32_t* d_nmask = nullptr;     // n_words + kWordPad
   std::map<int, uint64_t> windows; // k -> total windows
   std::map<int, double> est;       // 2k + canonical -> distinct estimate of all reads
   uint32_t* d_order = nullptr;     // locality order of the table passes (n_reads)

@@ -462,10 +462,10 @@ static int reads_build(tk_ctx* ctx, const char* d_seq, const uint64_t* d_off, ui
     if (e != hipSuccess) { rc = hip_fail(e, "read words"); break; }
     r->max_len = ctx->h_flags[0];
     r->n_words = nwords;
-    if ((rc = dev_alloc((void**)&r->d_codes, (nwords + 1) * 8))) break;
-    if ((rc = dev_alloc((void**)&r->d_nmask, (nwords + 1) * 4))) break;
-    e = hipMemsetAsync(r->d_codes + nwords, 0, 8, ctx->stream);
-    if (e == hipSuccess) e = hipMemsetAsync(r->d_nmask + nwords, 0xFF, 4, ctx->stream);
+    if ((rc = dev_alloc((void**)&r->d_codes, (nwords + kWordPad) * 8))) break;
+    if ((rc = dev_alloc((void**)&r->d_nmask, (nwords + kWordPad) * 4))) break;
+    e = hipMemsetAsync(r->d_codes + nwords, 0, kWordPad * 8, ctx->stream);
+    if (e == hipSuccess) e = hipMemsetAsync(r->d_nmask + nwords, 0xFF, kWordPad * 4, ctx->stream);
     if (e != hipSuccess) { rc = hip_fail(e, "pad"); break; }
     if (nwords) {
       const uint64_t nblk = ceil_div(nwords, 256);
@@ -486,7 +486,7 @@ static int reads_build(tk_ctx* ctx, const char* d_seq, const uint64_t* d_off, ui
     if (e != hipSuccess) { rc = hip_fail(e, "pack sync"); break; }
   } while (0);
   dev_free(d_nw, nwb);
-  r->bytes = std::max<uint64_t>(n, 1) * 4 + nwb + (r->n_words + 1) * 12;
+  r->bytes = std::max<uint64_t>(n, 1) * 4 + nwb + (r->n_words + kWordPad) * 12;
   if (rc) {
     tk_reads_free(r);
     return rc;
@@ -1571,18 +1571,15 @@ __global__ __launch_bounds__(256) void k_stats_short(ReadsView rv, int k, int ca
   stats_pass<true, kTicket>(rv, k, canonical, t, sp, out, slab, tickets, grab);
 }
 
-// k_stats_short over ticket runs, software-pipelined over each wave's reads:
-// while read j is scored, read j+1's code words (spread over lanes 0-5),
-// read j+2's length and first word and read j+3's index in the order are
-// loaded, so a read's table lookups wait on one memory round trip instead of
-// four dependent ones (order -> length / offset -> codes -> buckets).
-__global__ __launch_bounds__(256) void k_stats_pipe(ReadsView rv, int k, int canonical, TableView t,
-                                                    StatsParams sp, tk_read_stat* __restrict__ out,
-                                                    uint32_t* tickets, uint32_t grab) {
-  extern __shared__ uint64_t s_pipe[];
-  const int lane = threadIdx.x & 63;
-  const int wv = threadIdx.x >> 6;
-  uint64_t* tmp = s_pipe + wv * kLookupScratch;
+// The reads of one XCD's share of a per-read pass, software-pipelined over a
+// wave's ticket runs: while read j is processed, read j+1's code words
+// (lane_words), read j+2's length and first word and read j+3's index in the
+// order are loaded, so a read's table lookups wait on one memory round trip
+// instead of four dependent ones (order -> length / offset -> codes ->
+// buckets).  Values loaded an iteration earlier are made scalar when they are
+// used.  f(read, length, first word, lane's words).
+template <class F>
+__device__ __forceinline__ void piped_reads(const ReadsView& rv, uint32_t* tickets, uint32_t grab, int lane, F&& f) {
   const uint64_t per_xcd = (rv.n_reads + 7) >> 3;
   const uint64_t x = blockIdx.x & 7;
   const uint64_t lo = x * per_xcd;
@@ -1592,8 +1589,9 @@ __global__ __launch_bounds__(256) void k_stats_pipe(ReadsView rv, int k, int can
   TicketStream ts(tickets + x * kTicketStride, n, grab, lane);
   // stage a: index known; b: length and first word known; c: words known
   bool va = false, vb = false, vc = false;
-  uint32_t ra = 0, rb = 0, rc = 0, Lb = 0, Lc = 0, mwc = 0;
-  uint64_t wbb = 0, cwc = 0;
+  uint32_t ra = 0, rb = 0, rc = 0, Lb = 0, Lc = 0;
+  uint64_t wbb = 0, wbc = 0;
+  LaneWords wc{};
   for (;;) {
     const uint32_t p = ts.next();
     const bool vn = p < n;
@@ -1601,31 +1599,22 @@ __global__ __launch_bounds__(256) void k_stats_pipe(ReadsView rv, int k, int can
     if (vn) rn = rv.order ? rv.order[lo + p] : (uint32_t)(lo + p);
     uint32_t La = 0;
     uint64_t wba = 0;
+    ra = __builtin_amdgcn_readfirstlane(ra);
     if (va) {
       La = rv.len[ra];
       wba = rv.word_off[ra];
     }
-    uint64_t cwb = 0;
-    uint32_t mwb = 0;
-    if (vb && lane < 6 && (uint32_t)lane <= ((Lb + 31) >> 5)) {
-      cwb = rv.codes[wbb + lane];
-      mwb = rv.nmask[wbb + lane];
-    }
-    if (vc) {
-      const uint32_t nwin = Lc >= (uint32_t)k ? Lc - k + 1 : 0;
-      uint32_t nn, med;
-      uint64_t sum, sqlo, sqhi;
-      stats_short_core(nwin, k, canonical, t, sp, tmp, lane,
-                       [&](uint32_t pos, uint64_t& f, bool& v) { window_lanes(cwc, mwc, pos, k, f, v); }, nn, med,
-                       sum, sqlo, sqhi);
-      write_stat(lane, med, nn, sum, sqlo, sqhi, out + rc);
-      wave_sync();
-    }
+    LaneWords wn = wc;
+    Lb = __builtin_amdgcn_readfirstlane(Lb);
+    wbb = ((uint64_t)__builtin_amdgcn_readfirstlane((uint32_t)(wbb >> 32)) << 32) |
+          (uint32_t)__builtin_amdgcn_readfirstlane((uint32_t)wbb);
+    if (vb) wn = lane_words(rv, wbb, lane);
+    if (vc) f(rc, Lc, wbc, wc);
     vc = vb;
     rc = rb;
     Lc = Lb;
-    cwc = cwb;
-    mwc = mwb;
+    wbc = wbb;
+    wc = wn;
     vb = va;
     rb = ra;
     Lb = La;
@@ -1634,6 +1623,30 @@ __global__ __launch_bounds__(256) void k_stats_pipe(ReadsView rv, int k, int can
     ra = rn;
     if (!va && !vb && !vc) break;
   }
+}
+
+// The scoring pass for reads of at most 128 * CH windows.  Bound by the table
+// lines that miss L2 (44.7 G/s of the 47-49 G/s such lines reach: 4 M pairs,
+// 670 M of 1,008 M lookups miss) once the reads are many, by instruction issue
+// below that.  Eight lookups in flight per lane: with four and the registers
+// for seven waves per SIMD instead of four, 8.6 instead of 6.75 ms for 2 M
+// pairs.  With values in registers, DPP reductions and the LDS exchange of
+// coop_lookup (before: 1.5x the vector instructions): 200 k 76-nt reads
+// 477 -> 362 us, 2 M pairs 7.31 -> 6.75 ms, 20 M pairs 68.3 -> 66.9 ms.
+template <int CH>
+__global__ __launch_bounds__(256, 4) void k_stats_pipe(ReadsView rv, int k, int canonical, TableView t,
+                                                    StatsParams sp, tk_read_stat* __restrict__ out,
+                                                    uint32_t* tickets, uint32_t grab) {
+  __shared__ ulonglong2 s_pipe[4][kLookupScratch / 2];
+  const int lane = threadIdx.x & 63;
+  uint64_t* tmp = reinterpret_cast<uint64_t*>(s_pipe[threadIdx.x >> 6]);
+  piped_reads(rv, tickets, grab, lane, [&](uint32_t r, uint32_t L, uint64_t wb, const LaneWords& w) {
+    const uint32_t nwin = L >= (uint32_t)k ? L - k + 1 : 0;
+    uint32_t n, med;
+    uint64_t sum, sqlo, sqhi;
+    stats_regs<CH>(rv, wb, w, nwin, k, canonical, t, sp, tmp, lane, n, med, sum, sqlo, sqhi);
+    write_stat(lane, med, n, sum, sqlo, sqhi, out + r);
+  });
 }
 
 // k_stats for ordered reads of at most 128 windows each: every block takes
@@ -1817,7 +1830,7 @@ __global__ __launch_bounds__(256) void k_ctable_build(ReadsView rv, const uint32
 }
 
 template <bool kTicket>
-__global__ __launch_bounds__(256) void k_vote(ReadsView rv, int k, int canonical,
+__global__ __launch_bounds__(256, 4) void k_vote(ReadsView rv, int k, int canonical,
                                               const uint64_t* __restrict__ slots, uint64_t bmask,
                                               tk_r2t_vote* __restrict__ out, uint32_t slab, uint32_t* tickets,
                                               uint32_t grab) {
@@ -1826,7 +1839,7 @@ __global__ __launch_bounds__(256) void k_vote(ReadsView rv, int k, int canonical
   const int wv = threadIdx.x >> 6;
   const uint64_t wpb = blockDim.x >> 6;
   uint32_t* hits = s_dyn + (uint64_t)wv * slab;
-  uint32_t* tmp = s_dyn + wpb * slab + wv * 64;
+  uint64_t* tmp = reinterpret_cast<uint64_t*>(s_dyn + wpb * slab) + wv * kLookupScratch;
   // reads in the locality order, one contiguous range of it per XCD (as k_stats)
   const uint64_t per_xcd = (rv.n_reads + 7) >> 3;
   const uint64_t x = blockIdx.x & 7;
@@ -1841,115 +1854,30 @@ __global__ __launch_bounds__(256) void k_vote(ReadsView rv, int k, int canonical
 }
 
 // k_vote over ticket runs for reads of at most 128 windows (unpacked
-// component table), software-pipelined over each wave's reads as
-// k_stats_pipe: read j+1's code words, read j+2's length and first word and
-// read j+3's index load while read j votes (64 windows per lookup round).
-__global__ __launch_bounds__(256) void k_vote_pipe(ReadsView rv, int k, int canonical,
+// component table), pipelined as the scoring pass.
+__global__ __launch_bounds__(256, 6) void k_vote_pipe(ReadsView rv, int k, int canonical,
                                                    const uint64_t* __restrict__ slots, uint64_t bmask,
                                                    tk_r2t_vote* __restrict__ out, uint32_t* tickets, uint32_t grab) {
-  __shared__ uint32_t s_vote[4][192];  // per wave: 128 hits, 64 lookup scratch
+  __shared__ ulonglong2 s_vote[4][kLookupScratch / 2];
   const int lane = threadIdx.x & 63;
-  const int wv = threadIdx.x >> 6;
-  uint32_t* hits = s_vote[wv];
-  uint32_t* tmp = s_vote[wv] + 128;
-  const uint64_t occ = 1ull << (2 * k);
-  const uint64_t per_xcd = (rv.n_reads + 7) >> 3;
-  const uint64_t x = blockIdx.x & 7;
-  const uint64_t lo = x * per_xcd;
-  const uint64_t hi = lo + per_xcd < rv.n_reads ? lo + per_xcd : rv.n_reads;
-  if (lo >= hi) return;
-  const uint32_t n = (uint32_t)(hi - lo);
-  TicketStream ts(tickets + x * kTicketStride, n, grab, lane);
-  bool va = false, vb = false, vc = false;
-  uint32_t ra = 0, rb = 0, rc = 0, Lb = 0, Lc = 0, mwc = 0;
-  uint64_t wbb = 0, cwc = 0;
-  for (;;) {
-    const uint32_t p = ts.next();
-    const bool vn = p < n;
-    uint32_t rn = 0;
-    if (vn) rn = rv.order ? rv.order[lo + p] : (uint32_t)(lo + p);
-    uint32_t La = 0;
-    uint64_t wba = 0;
-    if (va) {
-      La = rv.len[ra];
-      wba = rv.word_off[ra];
-    }
-    uint64_t cwb = 0;
-    uint32_t mwb = 0;
-    if (vb && lane < 6 && (uint32_t)lane <= ((Lb + 31) >> 5)) {
-      cwb = rv.codes[wbb + lane];
-      mwb = rv.nmask[wbb + lane];
-    }
-    if (vc) {
-      const uint32_t nwin = Lc >= (uint32_t)k ? Lc - k + 1 : 0;
-      uint32_t nh = 0;
-      for (uint32_t base = 0; base < nwin; base += 64) {
-        const uint32_t pos = base + lane;
-        uint64_t f = 0;
-        bool valid = false;
-        window_lanes(cwc, mwc, pos, k, f, valid);
-        valid = valid && pos < nwin;
-        const uint64_t key = valid ? canon_key(f, k, canonical) : 0;
-        const uint32_t cmp = coop_cget64(slots, 0, bmask, occ, key, valid, tmp, lane);
-        const bool has = cmp != 0xFFFFFFFFu;
-        const uint64_t m = __ballot(has);
-        if (has) hits[nh + __popcll(m & ((1ull << lane) - 1))] = cmp;
-        nh += (uint32_t)__popcll(m);
-      }
-      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-      __builtin_amdgcn_wave_barrier();
-      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-      uint32_t best = 0xFFFFFFFFu, bestn = 0;
-      uint64_t prev = 0;
-      bool first = true;
-      while (nh) {
-        uint32_t cand = 0xFFFFFFFFu;
-        for (uint32_t i = lane; i < nh; i += 64) {
-          const uint32_t v = hits[i];
-          if ((first || v > (uint32_t)prev) && v < cand) cand = v;
-        }
-        cand = wave_min_u32(cand);
-        if (cand == 0xFFFFFFFFu) break;
-        uint32_t cnt = 0;
-        for (uint32_t i = lane; i < nh; i += 64) cnt += hits[i] == cand;
-        cnt = wave_sum_u32(cnt);
-        if (cnt > bestn) {
-          bestn = cnt;
-          best = cand;
-        }
-        prev = cand;
-        first = false;
-      }
-      if (lane == 0) {
-        tk_r2t_vote v;
-        v.comp = best;
-        v.hits = bestn;
-        v.nwin = nwin;
-        out[rc] = v;
-      }
-      wave_sync();
-    }
-    vc = vb;
-    rc = rb;
-    Lc = Lb;
-    cwc = cwb;
-    mwc = mwb;
-    vb = va;
-    rb = ra;
-    Lb = La;
-    wbb = wba;
-    va = vn;
-    ra = rn;
-    if (!va && !vb && !vc) break;
-  }
+  uint64_t* scratch = reinterpret_cast<uint64_t*>(s_vote[threadIdx.x >> 6]);
+  piped_reads(rv, tickets, grab, lane, [&](uint32_t r, uint32_t L, uint64_t, const LaneWords& w) {
+    const uint32_t nwin = L >= (uint32_t)k ? L - k + 1 : 0;
+    uint32_t c[2], best, bestn;
+    run_comps<false>(w, 0, nwin, k, canonical, slots, 0, bmask, scratch, lane, c);
+    vote_regs<2>(c, best, bestn);
+    write_vote(lane, best, bestn, nwin, out + r);
+  });
 }
 
-// Grid of the per-read table passes (k_stats, k_vote): at most TK_READ_BLOCKS_PER_CU
-// (default 128, the fastest of 4..128 and unbounded; 0 = one block per wpb
-// reads) blocks per CU.
-static int per_read_grid(tk_ctx* ctx, uint64_t n_reads, int wpb) {
-  const char* e = getenv("TK_READ_BLOCKS_PER_CU");
-  const uint64_t per_cu = e ? strtoull(e, nullptr, 10) : 128;
+// Grid of the per-read table passes: at most TK_READ_BLOCKS_PER_CU (default
+// per_cu; 0 = one block per wpb reads) blocks per CU.  Fewer reads in flight
+// keep a locus' lines in L2, more hide the misses: the passes over reads of at
+// most 128 windows are the same from 4 to 128 (2 M pairs: 6.45 to 6.75 ms; 7.70 at
+// 2), the vote is fastest at 5 (6 M reads: 9.06 ms; 9.40 at 128), reads of
+// 129 to 256 windows at 3 (1.2 M 250-nt reads: 3.48 ms; 3.82 at 4, 4.00 at 128).
+static int per_read_grid(tk_ctx* ctx, uint64_t n_reads, int wpb, uint64_t per_cu = 128) {
+  if (const char* e = getenv("TK_READ_BLOCKS_PER_CU")) per_cu = strtoull(e, nullptr, 10);
   const uint64_t want = ceil_div(n_reads, (uint64_t)wpb);
   const uint64_t cap = per_cu ? (uint64_t)std::max(ctx->num_cu, 1) * per_cu : (uint64_t)0x7FFFFFF0;
   return (int)std::max<uint64_t>(1, std::min<uint64_t>(want, cap));
@@ -1959,8 +1887,8 @@ static int per_read_grid(tk_ctx* ctx, uint64_t n_reads, int wpb) {
 // per-XCD ticket counters of the per-read passes.
 constexpr size_t kFlagBytes = (64 + kTicketWords) * 4;
 
-// Scoring reads of at most 128 windows with the software-pipelined kernel
-// (TK_STATS_PIPE, default 1; 0 = k_stats_short, one read at a time).
+// Scoring reads of at most 256 windows with the software-pipelined kernel
+// (TK_STATS_PIPE, default 1; 0 = k_stats_short or k_stats, one read at a time).
 static bool stats_pipe() {
   const char* e = getenv("TK_STATS_PIPE");
   return !e || e[0] != '0';
@@ -2309,8 +2237,8 @@ int tk_reads_free(tk_reads* r) {
   (void)hipSetDevice(r->device);
   dev_free(r->d_len, std::max<uint64_t>(r->n_reads, 1) * 4);
   dev_free(r->d_word_off, (r->n_reads + 1) * 8);
-  if (r->d_codes) dev_free(r->d_codes, (r->n_words + 1) * 8);
-  if (r->d_nmask) dev_free(r->d_nmask, (r->n_words + 1) * 4);
+  if (r->d_codes) dev_free(r->d_codes, (r->n_words + kWordPad) * 8);
+  if (r->d_nmask) dev_free(r->d_nmask, (r->n_words + kWordPad) * 4);
   if (r->d_order) dev_free(r->d_order, r->n_reads * 4);
   delete r;
   return TK_OK;
@@ -3375,10 +3303,14 @@ int tk_read_cov_stats_d(tk_ctx* c, tk_table* t, const tk_reads* r, const tk_stat
   const uint32_t grab = read_ticket_grab();
   uint32_t* tickets = grab ? c->d_tickets : nullptr;
   if (tickets) TK_LAUNCH(c, "tickets", 1, 256, 0, k_fill_u32, tickets, kTicketWords, 0u);
-  if (max_nwin <= 128 && tickets && stats_pipe()) {
-    const int pgrid = (per_read_grid(c, r->n_reads, 4) + 7) / 8 * 8;
-    TK_LAUNCH(c, "stats", pgrid, 256, 4 * 8 * kLookupScratch, k_stats_pipe, reads_view(r), t->k, t->canonical,
-              table_view(use), sp, d_out, tickets, grab);
+  if (max_nwin <= 256 && tickets && stats_pipe()) {
+    const int pgrid = (per_read_grid(c, r->n_reads, 4, max_nwin <= 128 ? 128 : 3) + 7) / 8 * 8;
+    if (max_nwin <= 128)
+      TK_LAUNCH(c, "stats", pgrid, 256, 0, k_stats_pipe<1>, reads_view(r), t->k, t->canonical, table_view(use), sp,
+                d_out, tickets, grab);
+    else
+      TK_LAUNCH(c, "stats", pgrid, 256, 0, k_stats_pipe<2>, reads_view(r), t->k, t->canonical, table_view(use), sp,
+                d_out, tickets, grab);
   } else if (max_nwin <= 128 && tickets)
     TK_LAUNCH(c, "stats", grid, wpb * 64, lds, k_stats_short<true>, reads_view(r), t->k, t->canonical,
               table_view(use), sp, d_out, slab, tickets, grab);
@@ -3621,9 +3553,9 @@ int tk_r2t_vote_reads_d(tk_ctx* c, const tk_ctable* t, const tk_reads* r, tk_r2t
   const uint32_t grab = read_ticket_grab();
   uint32_t* tickets = grab ? c->d_tickets : nullptr;
   if (tickets) TK_LAUNCH(c, "tickets", 1, 256, 0, k_fill_u32, tickets, kTicketWords, 0u);
-  const size_t lds = (size_t)slab * 4 * wpb + (size_t)wpb * 256;
+  const size_t lds = ((size_t)slab * 4 + 8 * kLookupScratch) * wpb;
   if (tickets && max_nwin <= 128 && vote_pipe()) {
-    const int pgrid = (per_read_grid(c, r->n_reads, 4) + 7) / 8 * 8;
+    const int pgrid = (per_read_grid(c, r->n_reads, 4, 5) + 7) / 8 * 8;
     TK_LAUNCH(c, "vote", pgrid, 256, 0, k_vote_pipe, reads_view(r), t->k, t->canonical, t->d_slots,
               t->nbuckets - 1, d_out, tickets, grab);
   } else if (tickets)
