@@ -84,3 +84,24 @@ def test_vote_run_ends(api, ctx, monkeypatch, longest, k, canonical, pipe):
     assert np.array_equal(got, want.astype(got.dtype))
     for o in (ct, bundles, reads):
         o.free()
+
+
+@pytest.mark.parametrize("resident", ["0", "1"])
+@pytest.mark.parametrize("k,canonical", [(25, True), (25, False), (21, True), (17, True), (16, True), (13, False)])
+def test_count_merge_quarters(api, ctx, monkeypatch, k, canonical, resident):
+    """The block merge on reads whose quarters end anywhere in their words,
+    repeated enough to pass its run limit, and on one-window and empty reads."""
+    print("count_merge_quarters", k, canonical, resident, flush=True)
+    monkeypatch.setenv("TK_ORDER_MIN_READS", "0")
+    monkeypatch.setenv("TK_RESIDENT", resident)
+    monkeypatch.setenv("TK_REGION_KB", "4")
+    seqs = _reads(k, 400, 0.004, 21) + ["A" * 150] * 200 + _reads(k, 128, 0.0, 22) * 3
+    seq, off = concat(seqs)
+    reads = api.Reads(ctx, seq, off)
+    t = api.Table(ctx, k, canonical, 4096, 0.5)
+    t.count(reads)
+    keys, counts = t.dump()
+    ok, oc = O.count(seq, off, k, canonical)
+    assert np.array_equal(keys, ok) and np.array_equal(counts, oc)
+    t.free()
+    reads.free()

@@ -147,13 +147,13 @@ struct BatchGroups {
 
 constexpr int kBatchAggSlots = 4096;
 
-template <bool KHI, int WPR>
-__global__ __launch_bounds__(256, 1) void k_batch_count_agg(ReadsView rv, const BatchGroup* __restrict__ groups,
+template <bool KHI>
+__global__ __launch_bounds__(256, 4) void k_batch_count_agg(ReadsView rv, const BatchGroup* __restrict__ groups,
                                                             uint64_t n_groups, const CompLayout* __restrict__ lay,
                                                             int k, int canonical, TableView base,
                                                             uint32_t* __restrict__ flags) {
-  count_agg<kBatchAggSlots, false, KHI, WPR>(rv, BatchGroups{groups, n_groups, lay, base}, k, canonical, base, flags,
-                                             nullptr, 0, 0, nullptr);
+  count_agg<kBatchAggSlots, false, KHI>(rv, BatchGroups{groups, n_groups, lay, base}, k, canonical, base, flags,
+                                        nullptr, 0, 0, nullptr);
 }
 
 // Locality key of each read within its component: the component in the top
@@ -503,11 +503,11 @@ static int batch_enqueue(tk_ctx* c, tk_batch* b, const tk_stats_opts* o, tk_read
     const unsigned ag = (unsigned)((b->n_groups + 7) / 8 * 8);  // xcd_block maps grids of 8k blocks
     ReadsView ro = rv;
     ro.order = b->d_order;
-    if (b->d_order && b->k >= 16)
-      hipLaunchKernelGGL((k_batch_count_agg<true, 2>), dim3(ag), dim3(256), kBatchAggSlots * 8, c->stream, ro,
+    if (b->d_order && b->k >= 17)
+      hipLaunchKernelGGL(k_batch_count_agg<true>, dim3(ag), dim3(256), kBatchAggSlots * 8, c->stream, ro,
                          b->d_groups, b->n_groups, b->d_lay, b->k, b->canonical, base, c->d_flags);
     else if (b->d_order)
-      hipLaunchKernelGGL((k_batch_count_agg<false, 1>), dim3(ag), dim3(256), kBatchAggSlots * 8, c->stream, ro,
+      hipLaunchKernelGGL(k_batch_count_agg<false>, dim3(ag), dim3(256), kBatchAggSlots * 8, c->stream, ro,
                          b->d_groups, b->n_groups, b->d_lay, b->k, b->canonical, base, c->d_flags);
     else
       hipLaunchKernelGGL(k_batch_count, dim3((rv.n_reads + kBatchReads - 1) / kBatchReads), dim3(256), 0,

@@ -2612,19 +2612,10 @@ static int res_sort_pass(tk_ctx* c, const std::vector<ResSlice>& sl, ResSlice* d
   return TK_OK;
 }
 
-// Windows per thread between the merge's block barriers (TK_MERGE_WPR = 2,
-// the default, or 1; the 3,840-slot merge of k >= 16 only).  Two halve the
-// barriers and shared-counter atomics of a latency-bound loop (36.4 vs
-// 40.2 ms on 5.04 G windows) for 1.4% more merged words (earlier flushes).
-static int merge_wpr() {
-  const char* e = getenv("TK_MERGE_WPR");
-  return e && atoi(e) == 1 ? 1 : 2;
-}
-
-// Words a merge block reserves in the stream at a time, for a pass over
-// `windows` windows with `mgrid` blocks.
+// Words a merge wavefront reserves in the stream at a time, for a pass over
+// `windows` windows with `mgrid` blocks of four.
 static uint64_t res_echunk(uint64_t windows, uint64_t mgrid) {
-  return std::min<uint64_t>(65536, std::max<uint64_t>(16384, next_pow2(windows / (std::max<uint64_t>(mgrid, 1) * 4))));
+  return std::min<uint64_t>(16384, std::max<uint64_t>(4096, next_pow2(windows / (std::max<uint64_t>(mgrid, 1) * 16))));
 }
 
 // Smallest streams a chunked region-resident count uses (2^26 words, 512 MB
@@ -2632,17 +2623,17 @@ static uint64_t res_echunk(uint64_t windows, uint64_t mgrid) {
 constexpr uint64_t kResMinStreamWords = 1ull << 26;
 
 // Stream capacity of a region-resident count of `windows` windows: the
-// words the merge can reserve (merged words <= windows, plus < one flush
-// (at most `slots` words) given up per reserved chunk of `echunk`, plus each
-// block's last chunk), so no merged word ever misses the stream.  False when that does not fit the
+// words the merge can reserve (merged words <= windows, plus < one flush of a
+// wavefront (at most `slots` words) given up per reserved chunk of `echunk`,
+// plus each wavefront's last chunk), so no merged word ever misses the stream.  False when that does not fit the
 // device memory the count may use: the table atomics then count instead
 // (the merge of a very large or error-rich read set leaves too many words).
 static bool resident_plan(tk_ctx* c, uint64_t windows, uint64_t* cap, uint64_t* echunk, uint64_t* mgrid,
                           uint64_t* cap_max, uint64_t* cap_chunked = nullptr) {
-  const uint64_t slots = (uint64_t)kResSlots;
+  const uint64_t slots = (uint64_t)kResSlots / 4;
   static const int pc = [] {  // resident merge blocks per CU (same for every device of the process)
     int nb = 0;
-    const hipError_t e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, (k_count_agg<kResSlots, true, true, 2>),
+    const hipError_t e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, (k_count_agg<kResSlots, true, true>),
                                                                       256, kResSlots * 8);
     if (e != hipSuccess || nb < 1) nb = 1;
     (void)hipGetLastError();
@@ -2650,7 +2641,7 @@ static bool resident_plan(tk_ctx* c, uint64_t windows, uint64_t* cap, uint64_t* 
   }();
   *mgrid = (uint64_t)std::max(c->num_cu, 1) * pc;
   *echunk = res_echunk(windows, *mgrid);
-  *cap = windows + windows / (*echunk / slots - 1) + *mgrid * (*echunk + slots);
+  *cap = windows + windows / (*echunk / slots - 1) + 4 * *mgrid * (*echunk + slots);
   size_t fr = 0, tot = 0;
   if (hipMemGetInfo(&fr, &tot) != hipSuccess) {
     (void)hipGetLastError();
@@ -2740,10 +2731,7 @@ static int count_resident(tk_ctx* c, tk_table* t, const tk_reads* r, const Reads
     // persistent: as many blocks per CU as its registers and LDS allow
     const uint64_t grid = std::max<uint64_t>(8, std::min<uint64_t>((ceil_div(qe - q, kReadsPerBlock) + 7) / 8 * 8, mgrid));
     const int table_ok = t->zero_pending ? 0 : 1;
-    if (t->k >= 16 && merge_wpr() == 2)
-      TK_LAUNCH(c, "count_merge", grid, 256, kResSlots * 8, (k_count_agg<kResSlots, true, true, 2>), rview, q, qe,
-                t->k, t->canonical, v, c->d_flags, A, cap, echunk, cursor, table_ok);
-    else if (t->k >= 16)
+    if (t->k >= 17)
       TK_LAUNCH(c, "count_merge", grid, 256, kResSlots * 8, (k_count_agg<kResSlots, true, true>), rview, q, qe,
                 t->k, t->canonical, v, c->d_flags, A, cap, echunk, cursor, table_ok);
     else
@@ -2931,11 +2919,11 @@ int tk_count(tk_ctx* c, tk_table* t, const tk_reads* r) {
     TK_HIP(hipMemsetAsync(c->d_flags, 0, 16, c->stream));
     const uint64_t grid = (ceil_div(nreads, kReadsPerBlock) + 7) / 8 * 8;
     TableView v = table_view(t);
-    // reads in the locality order: merge each block's windows in LDS first
-    // (two windows per thread per round for k >= 16); else a window per thread
+    // reads in the locality order: merge each block's windows in LDS first;
+    // else a window per thread
     const bool agg = rview.order && 63 - 2 * t->k >= 13;
-    if (agg && t->k >= 16)
-      TK_LAUNCH(c, "count", grid, 256, kAggSlots * 8, (k_count_agg<kAggSlots, false, true, 2>), rview, rb,
+    if (agg && t->k >= 17)
+      TK_LAUNCH(c, "count", grid, 256, kAggSlots * 8, (k_count_agg<kAggSlots, false, true>), rview, rb,
                 rb + nreads, t->k, t->canonical, v, c->d_flags, nullptr, 0, 0, nullptr, 1);
     else if (agg)
       TK_LAUNCH(c, "count", grid, 256, kAggSlots * 8, (k_count_agg<kAggSlots, false, false>), rview, rb,

@@ -138,7 +138,7 @@ __device__ __forceinline__ void summarize_regs(const uint32_t (&x)[NV], const bo
 #pragma unroll
     for (int i = 0; i < NV; i++) {
       s += x[i];
-      q += __umul24(x[i], x[i]);
+      q += (x[i] & 0xFFFFu) * (x[i] & 0xFFFFu);  // full-rate multiply
     }
     sum = wave_sum_u32(s);
     sqlo = wave_sum_u32(q);
