@@ -738,7 +738,7 @@ __global__ __launch_bounds__(256) void k_count(ReadsView rv, uint64_t r_begin,
 // HBM traffic, not by the device's atomic rate.
 // ---------------------------------------------------------------------
 constexpr uint32_t kResRegionBitsMax = 10;  // 1024 buckets = 64 KB of LDS
-constexpr uint64_t kResSlice = 65536;       // words per block of a sort pass
+constexpr uint64_t kResSlice = 65536;       // most words per block of a sort pass
 constexpr uint32_t kResMaxBins = 2048;      // bins per sort pass
 
 // A slice of a sort pass: words [begin, end) of the input, whose bin b
@@ -748,17 +748,31 @@ struct ResSlice {
   uint32_t m, j;
 };
 
+// Slice of this block: from the table, or (sl NULL) the block's share of
+// [0, n) in slices of `slice` words, one group.
+__device__ __forceinline__ ResSlice res_slice(const ResSlice* sl, uint64_t n, uint64_t slice) {
+  if (sl) return sl[blockIdx.x];
+  ResSlice d;
+  d.begin = (uint64_t)blockIdx.x * slice;
+  d.end = std::min<uint64_t>(n, d.begin + slice);
+  d.hbase = 0;
+  d.m = gridDim.x;
+  d.j = blockIdx.x;
+  return d;
+}
+
 __device__ __forceinline__ uint32_t res_region(const TableView& t, uint64_t w) {
   return (uint32_t)((bucket0(t, w & (t.occ - 1)) - t.boff) >> t.rbits);
 }
 
 // Bin of every nonzero word: (region >> shift) & mask, bins < nbins.
 __global__ __launch_bounds__(256) void k_res_hist(const uint64_t* __restrict__ in,
-                                                  const ResSlice* __restrict__ sl, TableView t,
-                                                  uint32_t shift, uint32_t mask, uint32_t nbins,
+                                                  const ResSlice* __restrict__ sl, uint64_t n, uint64_t slice,
+                                                  TableView t, uint32_t shift, uint32_t mask, uint32_t nbins,
                                                   uint64_t* __restrict__ hist) {
   __shared__ uint32_t s_cnt[kResMaxBins];
-  const ResSlice d = sl[blockIdx.x];
+  const ResSlice d = res_slice(sl, n, slice);
+  if (!d.m) return;  // past the last slice
   for (uint32_t i = threadIdx.x; i < nbins; i += blockDim.x) s_cnt[i] = 0;
   __syncthreads();
   for (uint64_t i0 = d.begin; i0 < d.end; i0 += 4 * blockDim.x) {
@@ -821,8 +835,9 @@ __device__ __forceinline__ uint32_t res_bin_scan(const uint32_t* s_cnt, uint32_t
 // bin in the write loop instead of keeping it in LDS.
 template <uint32_t kResTile, uint32_t kThreads>
 __global__ __launch_bounds__(kThreads) void k_res_scatter(const uint64_t* __restrict__ in,
-                                                          const ResSlice* __restrict__ sl, TableView t,
-                                                          uint32_t shift, uint32_t mask, uint32_t nbins,
+                                                          const ResSlice* __restrict__ sl, uint64_t n,
+                                                          uint64_t slice, TableView t, uint32_t shift,
+                                                          uint32_t mask, uint32_t nbins,
                                                           const uint64_t* __restrict__ base,
                                                           uint64_t* __restrict__ out) {
   constexpr bool kKeepBin = kResTile <= 4096;
@@ -835,7 +850,8 @@ __global__ __launch_bounds__(kThreads) void k_res_scatter(const uint64_t* __rest
   __shared__ uint32_t s_w[kThreads / 64];
   constexpr int kPer = kResTile / kThreads;
   const int tid = threadIdx.x;
-  const ResSlice d = sl[blockIdx.x];
+  const ResSlice d = res_slice(sl, n, slice);
+  if (!d.m) return;  // past the last slice
   for (uint32_t i = tid; i < nbins; i += kThreads) s_pos[i] = base[d.hbase + (uint64_t)i * d.m + d.j];
   for (uint64_t t0 = d.begin; t0 < d.end; t0 += kResTile) {
     const uint32_t nt = (uint32_t)std::min<uint64_t>(kResTile, d.end - t0);
@@ -878,23 +894,50 @@ __global__ __launch_bounds__(kThreads) void k_res_scatter(const uint64_t* __rest
   }
 }
 
-// First entry of every coarse bin of the scanned coarse histogram (bin c at
-// c * ns1) and the total, into out[0, C].
-__global__ void k_res_coarse_starts(const uint64_t* __restrict__ hs, uint64_t ns1, uint32_t C,
-                                    uint64_t* __restrict__ out) {
+// First entry of every bin of a scanned histogram of one slice group (bin c
+// at c * m) and the total, into out[0, C].
+__global__ void k_res_starts(const uint64_t* __restrict__ hs, uint64_t m, uint32_t C, uint64_t* __restrict__ out) {
   const uint32_t c = blockIdx.x * blockDim.x + threadIdx.x;
-  if (c <= C) out[c] = hs[(uint64_t)c * ns1];
+  if (c <= C) out[c] = hs[(uint64_t)c * m];
+}
+
+// Slice table of the fine pass (one block): every coarse bin's words in slices
+// of `slice`, at least one per bin, m[c] slices at histogram base hb[c]; the
+// table's entries past the last slice (up to `cap`, the bound the host launches
+// with, so that it need not wait for the counts) are empty.
+__global__ __launch_bounds__(1024) void k_res_plan(const uint64_t* __restrict__ cs, uint32_t C, uint32_t F,
+                                                   uint64_t slice, uint32_t cap, ResSlice* __restrict__ sl,
+                                                   uint64_t* __restrict__ hb, uint32_t* __restrict__ m) {
+  __shared__ uint32_t s_cnt[kResMaxBins], s_loc[kResMaxBins], s_w[1024 / 64];
+  const uint32_t tid = threadIdx.x;
+  for (uint32_t c = tid; c < C; c += 1024) {
+    const uint64_t n = (cs[c + 1] - cs[c] + slice - 1) / slice;
+    s_cnt[c] = n ? (uint32_t)n : 1u;
+  }
+  __syncthreads();
+  const uint32_t total = res_bin_scan<1024>(s_cnt, s_loc, C, s_w);
+  __syncthreads();
+  for (uint32_t c = tid; c < C; c += 1024) {
+    const uint64_t base = (uint64_t)F * s_loc[c], e = cs[c + 1];
+    hb[c] = base;
+    m[c] = s_cnt[c];
+    for (uint32_t j = 0; j < s_cnt[c] && s_loc[c] + j < cap; j++) {
+      const uint64_t at = cs[c] + j * slice;
+      sl[s_loc[c] + j] = ResSlice{at < e ? at : e, at + slice < e ? at + slice : e, base, s_cnt[c], j};
+    }
+  }
+  for (uint32_t i = total + tid; i < cap; i += 1024) sl[i] = ResSlice{0, 0, 0, 0, 0};
 }
 
 // First word of every region (region g = coarse g >> fs, fine g & (2^fs-1))
 // from the scanned fine histogram; rstart[R] = total.
 __global__ void k_res_bounds(const uint64_t* __restrict__ base2, const uint64_t* __restrict__ hb,
-                             const uint32_t* __restrict__ m, uint32_t fs, uint32_t R, uint64_t total,
-                             uint64_t* __restrict__ rstart) {
+                             const uint32_t* __restrict__ m, uint32_t fs, uint32_t R,
+                             const uint64_t* __restrict__ total, uint64_t* __restrict__ rstart) {
   const uint64_t g = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (g > R) return;
   if (g == R) {
-    rstart[R] = total;
+    rstart[R] = *total;
     return;
   }
   const uint32_t c = (uint32_t)(g >> fs), f = (uint32_t)g & ((1u << fs) - 1);
@@ -2515,18 +2558,29 @@ constexpr int kAggSlots = 4096;
 constexpr int kResSlots = 3840;
 
 // Whether a count of `windows` windows takes the region-resident passes
-// (reads in the locality order, k <= 25, tables of 64 KB regions).  By
-// default only counts of >= 2^32 windows do: their word streams are tens of
-// GB held by the context, and on smaller jobs the gain does not pay for the
-// memory (a context that holds them leaves less room for the per-job tables
-// of a sample stream, whose allocations then stall).  TK_RESIDENT=0 never,
-// TK_RESIDENT=1 always (when the streams fit).
+// (reads in the locality order, k <= 25, tables of 64 KB regions): from 2^23
+// windows on.  TK_RESIDENT=0 never, TK_RESIDENT=1 always (when the streams fit).
+// With table atomics / resident, count alone: 4.2 M windows 317 / 392 us, 6.2 M
+// 427 / 426, 10.1 M 647 / 497, 75.6 M 3.33 / 2.23 ms, 756 M 20.5 / 14.3 ms,
+// 2.0 G 46.5 / 33.1 ms.
+constexpr uint64_t kResMinWindows = 1ull << 23;
 static bool resident_enabled(uint64_t windows) {
   const char* e = getenv("TK_RESIDENT");
   if (e && e[0] == '0') return false;
   if (e && e[0] == '1') return true;
-  return windows >= (1ull << 32);
+  return windows >= kResMinWindows;
 }
+
+// Most words in each stream of a count below kResLargeWindows windows: their
+// context keeps at most 34 GB for them, and counts whose windows could merge
+// to more take the read chunks.  Larger counts may use 40% of the memory.
+constexpr uint64_t kResLargeWindows = 1ull << 32;
+constexpr uint64_t kResMidWords = 1ull << 31;
+
+// Regions up to which the words are sorted by region in one pass (runs of at
+// least eight words per tile and bin, and one reading and writing of the stream
+// less).
+constexpr uint32_t kResOnePass = 960;
 
 // The kernel attributes below are set once per process, by whichever thread
 // gets here first (a function-local static is initialised under the
@@ -2583,32 +2637,30 @@ static uint32_t res_tile() {
 enum { kSlotResA = 4, kSlotResB = 5, kSlotResHist = 6, kSlotResMisc = 7 };
 
 // One counting-sort pass of the region-resident count: the nonzero words of
-// `in` (slice table dsl, copied from sl) to `out`, grouped by bin
-// (region >> shift) & mask.  h holds nhist + 1 counts, hs their scan.
-static int res_sort_pass(tk_ctx* c, const std::vector<ResSlice>& sl, ResSlice* dsl, uint64_t nhist,
+// `in` (`blocks` slices from the table dsl, or of [0, n) by `slice` words when
+// it is NULL) to `out`, grouped by bin (region >> shift) & mask.  h holds nhist
+// + 1 counts, hs their scan.
+static int res_sort_pass(tk_ctx* c, const ResSlice* dsl, uint64_t blocks, uint64_t n, uint64_t slice, uint64_t nhist,
                          uint64_t* h, uint64_t* hs, const uint64_t* in, uint64_t* out, const TableView& v,
                          uint32_t shift, uint32_t mask, uint32_t nbins) {
-  TK_HIP(hipMemcpyAsync(dsl, sl.data(), sl.size() * sizeof(ResSlice), hipMemcpyHostToDevice, c->stream));
   TK_HIP(hipMemsetAsync(h + nhist, 0, 8, c->stream));
-  TK_LAUNCH(c, "count_hist", sl.size(), 256, 0, k_res_hist, in, dsl, v, shift, mask, nbins, h);
+  TK_LAUNCH(c, "count_hist", blocks, 256, 0, k_res_hist, in, dsl, n, slice, v, shift, mask, nbins, h);
   int rc = exclusive_scan_u64(c, h, hs, nhist + 1);
   if (rc) return rc;
   uint32_t tile = res_tile();
   if (tile == 16384 && res_scatter_lds(nbins, 16384) + 1024 > 160 * 1024) tile = 8192;  // LDS of one CU
   if (tile == 2048)
-    TK_LAUNCH(c, "count_scatter", sl.size(), 256, res_scatter_lds(nbins, 2048), (k_res_scatter<2048, 256>), in,
-              dsl, v, shift, mask, nbins, hs, out);
+    TK_LAUNCH(c, "count_scatter", blocks, 256, res_scatter_lds(nbins, 2048), (k_res_scatter<2048, 256>), in, dsl, n,
+              slice, v, shift, mask, nbins, hs, out);
   else if (tile == 8192)
-    TK_LAUNCH(c, "count_scatter", sl.size(), 512, res_scatter_lds(nbins, 8192), (k_res_scatter<8192, 512>), in,
-              dsl, v, shift, mask, nbins, hs, out);
+    TK_LAUNCH(c, "count_scatter", blocks, 512, res_scatter_lds(nbins, 8192), (k_res_scatter<8192, 512>), in, dsl, n,
+              slice, v, shift, mask, nbins, hs, out);
   else if (tile == 16384)
-    TK_LAUNCH(c, "count_scatter", sl.size(), 1024, res_scatter_lds(nbins, 16384), (k_res_scatter<16384, 1024>),
-              in, dsl, v, shift, mask, nbins, hs, out);
+    TK_LAUNCH(c, "count_scatter", blocks, 1024, res_scatter_lds(nbins, 16384), (k_res_scatter<16384, 1024>), in, dsl,
+              n, slice, v, shift, mask, nbins, hs, out);
   else
-    TK_LAUNCH(c, "count_scatter", sl.size(), 256, res_scatter_lds(nbins, 4096), (k_res_scatter<4096, 256>), in,
-              dsl, v, shift, mask, nbins, hs, out);
-  // the slice table is host memory read by the copy above
-  TK_HIP(hipStreamSynchronize(c->stream));
+    TK_LAUNCH(c, "count_scatter", blocks, 256, res_scatter_lds(nbins, 4096), (k_res_scatter<4096, 256>), in, dsl, n,
+              slice, v, shift, mask, nbins, hs, out);
   return TK_OK;
 }
 
@@ -2686,7 +2738,11 @@ static int count_resident(tk_ctx* c, tk_table* t, const tk_reads* r, const Reads
                                             (unsigned long long)(1ull << t->rbits));
   }
   uint64_t cap = 0, echunk = 0, mgrid = 0, cap_max = 0, cap_chunked = 0;
-  const bool whole = resident_plan(c, windows, &cap, &echunk, &mgrid, &cap_max, &cap_chunked);
+  bool whole = resident_plan(c, windows, &cap, &echunk, &mgrid, &cap_max, &cap_chunked);
+  if (windows < kResLargeWindows) {
+    whole = whole && cap <= kResMidWords;
+    cap_chunked = std::min(cap_chunked, kResMidWords);
+  }
   // TK_RES_CHUNK_READS=n: read chunks of n reads even when one pass fits
   // (tests), TK_RES_STREAM_WORDS=n: streams of at most n words.
   const char* ecr = getenv("TK_RES_CHUNK_READS");
@@ -2696,7 +2752,8 @@ static int count_resident(tk_ctx* c, tk_table* t, const tk_reads* r, const Reads
   const uint64_t n_all = re - rb;
   const double win_per_read = (double)windows / (double)std::max<uint64_t>(1, n_all);
   uint64_t chunk = n_all;
-  double ratio = 2.5;  // windows per stream word, until a chunk has measured it
+  // windows per stream word, until a chunk has measured it
+  double ratio = windows < kResLargeWindows ? 1.5 : 2.5;
   const bool chunked = !whole || forced_reads || forced_words;
   if (chunked) {
     // The streams of every window do not fit (or a test asks for chunks):
@@ -2767,14 +2824,20 @@ static int count_resident(tk_ctx* c, tk_table* t, const tk_reads* r, const Reads
       if ((rc = table_zero(c, t))) return rc;
       continue;
     }
-    // coarse bins of F = 2^fs regions, then single regions
+    // Words grouped by coarse bins of F = 2^fs regions, then by single regions;
+    // tables of at most kResOnePass regions by region at once.  Slices of a
+    // sort pass shrink with the stream, so that a small one still gives every
+    // CU several blocks.
     const uint32_t R = (uint32_t)(t->nb >> t->rbits);
+    const bool one_pass = R <= kResOnePass;
     uint32_t fs = 0;
-    while ((1ull << (2 * fs)) < R) fs++;
+    while (!one_pass && (1ull << (2 * fs)) < R) fs++;
     const uint32_t F = 1u << fs, C = (uint32_t)ceil_div(R, F);
-    const uint64_t ns1 = ceil_div(n, kResSlice);
+    const uint64_t slice = std::min<uint64_t>(
+        kResSlice, std::max<uint64_t>(8192, ceil_div(n, (uint64_t)std::max(c->num_cu, 1) * 8) / 8192 * 8192));
+    const uint64_t ns1 = ceil_div(n, slice);
     const uint64_t ns2_max = ns1 + C;  // sum over coarse bins of ceil(n_c / slice)
-    const uint64_t nh1 = (uint64_t)C * ns1, nh_max = std::max<uint64_t>(nh1, (uint64_t)F * ns2_max);
+    const uint64_t nh1 = (uint64_t)C * ns1, nh2 = one_pass ? 0 : (uint64_t)F * ns2_max, nh_max = std::max(nh1, nh2);
     void *hp = nullptr, *mp = nullptr;
     const uint64_t sl_bytes = ns2_max * sizeof(ResSlice), hb_off = sl_bytes, m_off = hb_off + (uint64_t)C * 8,
                    rs_off = (m_off + (uint64_t)C * 4 + 7) / 8 * 8, cs_off = rs_off + ((uint64_t)R + 1) * 8,
@@ -2788,50 +2851,33 @@ static int count_resident(tk_ctx* c, tk_table* t, const tk_reads* r, const Reads
     uint32_t* dm = (uint32_t*)((char*)mp + m_off);
     uint64_t* drs = (uint64_t*)((char*)mp + rs_off);
     uint64_t* dcs = (uint64_t*)((char*)mp + cs_off);
-    std::vector<ResSlice> sl;
-    sl.reserve(ns2_max);
-    for (uint64_t j = 0; j < ns1; j++)
-      sl.push_back({j * kResSlice, std::min<uint64_t>(n, (j + 1) * kResSlice), 0, (uint32_t)ns1, (uint32_t)j});
-    if ((rc = res_sort_pass(c, sl, dsl, nh1, h, hs, A, B, v, fs, 0xFFFFFFFFu, C))) return rc;
-    std::vector<uint64_t> cs(C + 1);
-    TK_LAUNCH(c, "count_bounds", ceil_div((uint64_t)C + 1, 256), 256, 0, k_res_coarse_starts, hs, ns1, C, dcs);
-    TK_HIP(hipMemcpyAsync(cs.data(), dcs, ((size_t)C + 1) * 8, hipMemcpyDeviceToHost, c->stream));
-    TK_HIP(hipStreamSynchronize(c->stream));
-    const uint64_t total = cs[C];
-    c->count_words += total;
-    std::vector<uint64_t> hb(C);
-    std::vector<uint32_t> m(C);
-    sl.clear();
-    uint64_t nh2 = 0;
-    for (uint32_t cc = 0; cc < C; cc++) {
-      const uint64_t ncc = cs[cc + 1] - cs[cc];
-      m[cc] = (uint32_t)std::max<uint64_t>(1, ceil_div(ncc, kResSlice));
-      hb[cc] = nh2;
-      for (uint32_t j = 0; j < m[cc]; j++)
-        sl.push_back({cs[cc] + j * kResSlice, std::min<uint64_t>(cs[cc + 1], cs[cc] + (j + 1) * kResSlice), nh2,
-                      m[cc], j});
-      nh2 += (uint64_t)F * m[cc];
+    if ((rc = res_sort_pass(c, nullptr, ns1, n, slice, nh1, h, hs, A, B, v, fs, 0xFFFFFFFFu, C))) return rc;
+    TK_LAUNCH(c, "count_bounds", ceil_div((uint64_t)C + 1, 256), 256, 0, k_res_starts, hs, ns1, C,
+              one_pass ? drs : dcs);
+    uint64_t* W = one_pass ? B : A;  // the words by region
+    if (!one_pass) {
+      TK_LAUNCH(c, "count_bounds", 1, 1024, 0, k_res_plan, dcs, C, F, slice, (uint32_t)ns2_max, dsl, dhb, dm);
+      if ((rc = res_sort_pass(c, dsl, ns2_max, 0, 0, nh2, h, hs, B, A, v, 0, F - 1, F))) return rc;
+      TK_LAUNCH(c, "count_bounds", ceil_div((uint64_t)R + 1, 256), 256, 0, k_res_bounds, hs, dhb, dm, fs, R, dcs + C,
+                drs);
     }
-    if (sl.size() > ns2_max) return fail(TK_ERR_HIP, "count: %zu fine slices (bound %llu)", sl.size(),
-                                         (unsigned long long)ns2_max);
-    TK_HIP(hipMemcpyAsync(dhb, hb.data(), (size_t)C * 8, hipMemcpyHostToDevice, c->stream));
-    TK_HIP(hipMemcpyAsync(dm, m.data(), (size_t)C * 4, hipMemcpyHostToDevice, c->stream));
-    if ((rc = res_sort_pass(c, sl, dsl, nh2, h, hs, B, A, v, 0, F - 1, F))) return rc;
-    TK_LAUNCH(c, "count_bounds", ceil_div((uint64_t)R + 1, 256), 256, 0, k_res_bounds, hs, dhb, dm, fs, R, total,
-              drs);
     TK_HIP(hipMemsetAsync(c->d_flags, 0, 64, c->stream));
     const size_t lds = (size_t)72 << t->rbits;  // slots + tags
     if (keys_before == 0 && nnew == 0)
-      TK_LAUNCH(c, "count_regions", R, 1024, lds, k_res_count<true>, A, drs, v, c->d_flags,
+      TK_LAUNCH(c, "count_regions", R, 1024, lds, k_res_count<true>, W, drs, v, c->d_flags,
                 t->zero_pending ? 1 : 0);
     else
-      TK_LAUNCH(c, "count_regions", R, 1024, lds, k_res_count<false>, A, drs, v, c->d_flags, 0);
+      TK_LAUNCH(c, "count_regions", R, 1024, lds, k_res_count<false>, W, drs, v, c->d_flags, 0);
     t->zero_pending = false;  // every region written (fresh) or the table was clear
     TK_HIP(hipMemcpyAsync(c->h_flags, c->d_flags, 64, hipMemcpyDeviceToHost, c->stream));
+    TK_HIP(hipMemcpyAsync(c->h_flags + 16, drs + R, 8, hipMemcpyDeviceToHost, c->stream));
     TK_HIP(hipStreamSynchronize(c->stream));
     if (c->h_flags[0]) return fail(TK_ERR_FULL, "count: table error (flags=%u)", c->h_flags[0]);
     memcpy(&nnew, &c->h_flags[2], 8);
     t->n_keys += nnew;
+    uint64_t total = 0;
+    memcpy(&total, &c->h_flags[16], 8);
+    c->count_words += total;
     // words of crowded regions: grow, then add them (growing again while any
     // still finds no room)
     for (int round = 0; c->h_flags[6]; round++) {
@@ -2839,7 +2885,7 @@ static int count_resident(tk_ctx* c, tk_table* t, const tk_reads* r, const Reads
       if ((rc = table_grow(c, t, t->n_keys + total))) return rc;
       TK_HIP(hipMemsetAsync(c->d_flags, 0, 64, c->stream));
       TableView v3 = table_view(t);
-      TK_LAUNCH(c, "count_retry", std::min<uint64_t>(ceil_div(total, 256), 65536), 256, 0, k_res_retry, A, total,
+      TK_LAUNCH(c, "count_retry", std::min<uint64_t>(ceil_div(total, 256), 65536), 256, 0, k_res_retry, W, total,
                 v3, c->d_flags);
       TK_HIP(hipMemcpyAsync(c->h_flags, c->d_flags, 64, hipMemcpyDeviceToHost, c->stream));
       TK_HIP(hipStreamSynchronize(c->stream));
