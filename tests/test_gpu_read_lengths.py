@@ -105,3 +105,31 @@ def test_count_merge_quarters(api, ctx, monkeypatch, k, canonical, resident):
     assert np.array_equal(keys, ok) and np.array_equal(counts, oc)
     t.free()
     reads.free()
+
+
+@pytest.mark.parametrize("n", [1, 3, 500])
+@pytest.mark.parametrize("k", [13, 25, 31])
+def test_small_sets_spread(api, ctx, k, n):
+    """Few sequences of very different lengths (windows spread over the whole
+    device in the unordered count, the component table and the sketch)."""
+    print("small_sets_spread", k, n, flush=True)
+    rng = np.random.default_rng(k + n)
+    seqs = ["".join(rng.choice(list("ACGTN"), size=int(L), p=[0.2495] * 4 + [0.002]))
+            for L in rng.choice([0, 5, 24, 25, 31, 33, 64, 300, 4097, 9000], size=n)] + ["ACGT" * 500]
+    seq, off = concat(seqs)
+    comps = rng.integers(0, 4, size=len(seqs)).astype(np.uint32)
+    reads = api.Reads(ctx, seq, off)
+    t = api.Table(ctx, k, True, 64, 0.5)
+    t.count(reads)
+    keys, counts = t.dump()
+    ok, oc = O.count(seq, off, k, True)
+    assert np.array_equal(keys, ok) and np.array_equal(counts, oc)
+    est = api.estimate_distinct(ctx, reads, k, True)
+    assert abs(est - len(ok)) <= 0.1 * len(ok) + 2
+    ct = api.CTable(ctx, reads, comps, k, True)
+    bk, bc = O.r2t_build(seq, off, comps, k, True)
+    assert ct.info()[0] == len(bk)
+    want = O.r2t_vote(seq, off, bk, bc, k, True)
+    assert np.array_equal(ct.vote(reads), want.astype(api.R2T_VOTE_DTYPE))
+    for o in (ct, t, reads):
+        o.free()

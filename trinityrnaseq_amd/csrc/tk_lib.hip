@@ -613,27 +613,39 @@ constexpr int kHllRegs = 1 << kHllBits;
 // end there), so each base is read once instead of once per window;
 // block-private registers in LDS merged with one atomicMax per register.
 // When `keys`/`idx` are given, the same pass writes each read's locality
-// sort key exactly as k_minimizer does.
+// sort key exactly as k_minimizer does (segw = 0).  segw > 0: a thread takes
+// segw windows of a read, `segs` threads per read, for the k - 1 bases before
+// them read again: sets of few or long reads (200 150-base reads: 28 us with a
+// thread each).
 __global__ __launch_bounds__(256) void k_hll(ReadsView rv, uint64_t r_begin, uint64_t r_end, int k,
                                                   int canonical, uint32_t sbits, uint32_t* __restrict__ regs,
-                                                  uint64_t* __restrict__ keys, uint32_t* __restrict__ idx) {
+                                                  uint64_t* __restrict__ keys, uint32_t* __restrict__ idx,
+                                                  uint32_t segw, uint32_t segs) {
   __shared__ uint32_t s_reg[kHllRegs];
   for (int i = threadIdx.x; i < kHllRegs; i += blockDim.x) s_reg[i] = 0;
   __syncthreads();
   const uint64_t kmask = (1ull << (2 * k)) - 1;  // k <= 31
   const int rsh = 2 * k - 2;
-  for (uint64_t r = r_begin + (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; r < r_end;
-       r += (uint64_t)gridDim.x * blockDim.x) {
-    const uint32_t L = rv.len[r];
+  const uint64_t items = (r_end - r_begin) * segs;
+  for (uint64_t it = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; it < items;
+       it += (uint64_t)gridDim.x * blockDim.x) {
+    const uint64_t r = r_begin + (segw ? it / segs : it);
+    // the bases of this thread's windows: [b0, L)
+    uint32_t L = rv.len[r], b0 = 0;
+    if (segw) {
+      const uint64_t first = it % segs * segw;
+      b0 = (uint32_t)std::min<uint64_t>(first, L);
+      L = (uint32_t)std::min<uint64_t>(L, first + segw + k - 1);
+    }
     const uint64_t wb = rv.word_off[r];
     uint64_t fwd = 0, rc = 0;
     uint32_t run = 0;
     MinKey mk;
-    for (uint32_t w = 0; 32 * w < L; w++) {
+    for (uint32_t w = b0 >> 5; 32 * w < L; w++) {
       const uint64_t code = rv.codes[wb + w];
       const uint32_t msk = rv.nmask[wb + w];
       const uint32_t nb = L - 32 * w < 32u ? L - 32 * w : 32u;
-      for (uint32_t j = 0; j < nb; j++) {
+      for (uint32_t j = 32 * w < b0 ? b0 - 32 * w : 0; j < nb; j++) {
         const uint32_t b = (uint32_t)(code >> (62 - 2 * j)) & 3u;
         fwd = ((fwd << 2) | b) & kmask;
         rc = (rc >> 2) | ((uint64_t)(3u - b) << rsh);
@@ -665,18 +677,18 @@ __global__ __launch_bounds__(256) void k_hll(ReadsView rv, uint64_t r_begin, uin
 // Counting
 // =====================================================================
 
-// One thread per k-window of a block of 64 consecutive reads.  flags[0] gets
+// One thread per k-window of a block of rpb (<= 64) consecutive reads.  flags[0] gets
 // error bits, flags[2..3] (u64) the number of newly claimed slots.  Four
 // lanes of 16 bytes probe each key's bucket.
 __global__ __launch_bounds__(256) void k_count(ReadsView rv, uint64_t r_begin,
-                                               uint64_t r_end, int k, int canonical,
+                                               uint64_t r_end, int k, int canonical, uint32_t rpb,
                                                TableView t, uint32_t* __restrict__ flags) {
   __shared__ uint32_t s_off[kReadsPerBlock + 1];
   __shared__ uint64_t s_wb[kReadsPerBlock];
   __shared__ uint32_t s_new;
-  const uint64_t r0 = r_begin + xcd_block(blockIdx.x, gridDim.x) * kReadsPerBlock;
+  const uint64_t r0 = r_begin + xcd_block(blockIdx.x, gridDim.x) * rpb;
   if (r0 >= r_end) return;
-  const int nr = (int)std::min<uint64_t>(kReadsPerBlock, r_end - r0);
+  const int nr = (int)std::min<uint64_t>(rpb, r_end - r0);
   const int tid = threadIdx.x;
   if (tid < kReadsPerBlock) {
     uint32_t nw = 0;
@@ -1822,53 +1834,55 @@ __global__ __launch_bounds__(256) void k_select(const tk_read_stat* __restrict__
 // =====================================================================
 // ReadsToTranscripts
 // =====================================================================
-__global__ __launch_bounds__(256) void k_ctable_build(ReadsView rv, const uint32_t* __restrict__ comp,
-                                                      int k, int canonical, uint64_t* slots,
-                                                      uint64_t bmask, uint32_t* __restrict__ flags) {
-  __shared__ uint32_t s_off[kReadsPerBlock + 1];
-  __shared__ uint64_t s_wb[kReadsPerBlock];
-  __shared__ uint32_t s_comp[kReadsPerBlock];
-  __shared__ uint32_t s_new;
-  const uint64_t r0 = (uint64_t)blockIdx.x * kReadsPerBlock;
-  if (r0 >= rv.n_reads) return;
-  const int nr = (int)std::min<uint64_t>(kReadsPerBlock, rv.n_reads - r0);
-  const int tid = threadIdx.x;
-  if (tid < kReadsPerBlock) {
-    uint32_t nw = 0;
-    if (tid < nr) {
-      const uint32_t L = rv.len[r0 + tid];
-      nw = L >= (uint32_t)k ? L - k + 1 : 0;
-      s_wb[tid] = rv.word_off[r0 + tid];
-      s_comp[tid] = comp[r0 + tid];
-    }
-    uint32_t x = nw;
-#pragma unroll
-    for (int o = 1; o < 64; o <<= 1) {
-      uint32_t y = __shfl_up(x, o);
-      if (tid >= o) x += y;
-    }
-    s_off[tid + 1] = x;
-    if (tid == 0) { s_off[0] = 0; s_new = 0; }
+// Last read whose first word is at or before word w (the read holding w; empty
+// reads before it are passed over), found by the whole wave: 64 pivots a step.
+__device__ __forceinline__ uint64_t read_of_word(const uint64_t* __restrict__ word_off, uint64_t n_reads, uint64_t w,
+                                                 int lane) {
+  uint64_t lo = 0, hi = n_reads;
+  while (hi - lo > 1) {
+    const uint64_t step = (hi - lo + 63) >> 6;
+    const uint64_t p = lo + (uint64_t)lane * step;
+    const uint64_t m = __ballot(p < hi && word_off[p] <= w);
+    lo += (uint64_t)(63 - __clzll((long long)(m | 1ull))) * step;
+    hi = hi < lo + step ? hi : lo + step;
   }
+  return lo;
+}
+
+// Lane per base position: a wave takes `per` packed words (two at a time),
+// whatever reads they belong to, so a few long sequences fill the device as
+// well as many short ones (a block per 64 sequences, looping over their
+// windows, took 105 us for six contigs of 900 bases, 14 us now; large sets are
+// bound by the two memory-side atomics per new key, 6.5 ms for 96 M windows).
+__global__ __launch_bounds__(256) void k_ctable_build(ReadsView rv, uint64_t n_words, uint32_t per,
+                                                      const uint32_t* __restrict__ comp, int k, int canonical,
+                                                      uint64_t* slots, uint64_t bmask, uint32_t* __restrict__ flags) {
+  __shared__ uint32_t s_new;
+  if (threadIdx.x == 0) s_new = 0;
   __syncthreads();
+  const int lane = threadIdx.x & 63;
   const uint64_t occ = 1ull << (2 * k);
-  const uint32_t total = s_off[nr];
   uint32_t mynew = 0;
-  for (uint32_t w = tid; w < total; w += blockDim.x) {
-    int lo = 0, hi = nr;
-    while (hi - lo > 1) {
-      int mid = (lo + hi) >> 1;
-      if (s_off[mid] <= w) lo = mid; else hi = mid;
+  for (uint64_t w0 = ((uint64_t)blockIdx.x * 4 + (threadIdx.x >> 6)) * per; w0 < n_words;
+       w0 += (uint64_t)gridDim.x * 4 * per) {
+    uint64_t r = read_of_word(rv.word_off, rv.n_reads, w0, lane);
+    const uint64_t wend = std::min<uint64_t>(n_words, w0 + per);
+    for (uint64_t w = w0 + (lane >> 5); w < wend; w += 2) {
+      while (rv.word_off[r + 1] <= w) r++;
+      const uint64_t wb = rv.word_off[r];
+      const uint64_t pos = (w - wb) * 32 + (lane & 31);
+      if (pos + k <= rv.len[r]) {
+        uint64_t fwd;
+        bool valid;
+        window_at(rv, wb, (uint32_t)pos, k, fwd, valid);
+        if (valid) ctable_add(slots, 0, bmask, occ, canon_key(fwd, k, canonical), comp[r], mynew, &flags[0]);
+      }
     }
-    uint64_t fwd;
-    bool valid;
-    window_at(rv, s_wb[lo], w - s_off[lo], k, fwd, valid);
-    if (valid) ctable_add(slots, 0, bmask, occ, canon_key(fwd, k, canonical), s_comp[lo], mynew, &flags[0]);
   }
   mynew = wave_sum_u32(mynew);
-  if ((tid & 63) == 0 && mynew) atomicAdd(&s_new, mynew);
+  if (lane == 0 && mynew) atomicAdd(&s_new, mynew);
   __syncthreads();
-  if (tid == 0 && s_new)
+  if (threadIdx.x == 0 && s_new)
     atomicAdd(reinterpret_cast<unsigned long long*>(&flags[2]), (unsigned long long)s_new);
 }
 
@@ -1945,10 +1959,12 @@ static bool vote_pipe() {
 }
 
 // Reads per ticket grab in the per-read table passes (TK_READ_TICKET, default
-// 4; 0 = each wave takes a fixed stride of the XCD's range instead).
-static uint32_t read_ticket_grab() {
+// 4, or 1 for fewer reads than four per wave the device holds, which a few
+// waves would otherwise take all; 0 = each wave takes a fixed stride of the
+// XCD's range instead).
+static uint32_t read_ticket_grab(const tk_ctx* ctx, uint64_t n_reads) {
   const char* e = getenv("TK_READ_TICKET");
-  if (!e) return 4;
+  if (!e) return n_reads < (uint64_t)std::max(ctx->num_cu, 1) * 64 ? 1 : 4;
   const unsigned long v = strtoul(e, nullptr, 10);
   return v > 1024 ? 1024u : (uint32_t)v;
 }
@@ -2360,11 +2376,16 @@ static int hll_estimate(tk_ctx* c, const tk_reads* r, uint64_t rb, uint64_t re, 
     // atomicMax per register into the global registers
     const char* hb = getenv("TK_HLL_BLOCKS_PER_CU");
     const uint64_t per_cu = hb && atoi(hb) > 0 ? (uint64_t)atoi(hb) : 64;
-    const uint64_t grid = std::min<uint64_t>(ceil_div(re - rb, 256), (uint64_t)std::max(c->num_cu, 1) * per_cu);
+    // too few reads to fill the device with a thread each: segments of 64
+    // windows (the keys need whole reads, but only large sets want them)
+    const uint32_t nwin = r->max_len >= (uint32_t)k ? r->max_len - k + 1 : 0;
+    const bool seg = !keys && nwin > 64 && re - rb < (uint64_t)std::max(c->num_cu, 1) * 256;
+    const uint32_t segw = seg ? 64 : 0, segs = seg ? (nwin + 63) / 64 : 1;
+    const uint64_t grid = std::min<uint64_t>(ceil_div((re - rb) * segs, 256), (uint64_t)std::max(c->num_cu, 1) * per_cu);
     hipEvent_t a;
     timing_begin(c, &a);
     hipLaunchKernelGGL(k_hll, dim3(grid), dim3(256), 0, c->stream, reads_view(r), rb, re, k, canonical,
-                       sbits, regs, keys, order);
+                       sbits, regs, keys, order, segw, segs);
     timing_end(c, "hll", a);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) {
@@ -2974,8 +2995,15 @@ int tk_count(tk_ctx* c, tk_table* t, const tk_reads* r) {
     else if (agg)
       TK_LAUNCH(c, "count", grid, 256, kAggSlots * 8, (k_count_agg<kAggSlots, false, false>), rview, rb,
                 rb + nreads, t->k, t->canonical, v, c->d_flags, nullptr, 0, 0, nullptr, 1);
-    else
-      TK_LAUNCH(c, "count", grid, 256, 0, k_count, rview, rb, rb + nreads, t->k, t->canonical, v, c->d_flags);
+    else {
+      // few reads: fewer per block, so that the windows still spread over the
+      // device (a round of 256 windows is a chain of memory round trips: 200
+      // 150-base reads in four blocks took 112 us)
+      const uint32_t rpb = (uint32_t)std::min<uint64_t>(
+          kReadsPerBlock, std::max<uint64_t>(1, nreads / ((uint64_t)std::max(c->num_cu, 1) * 4)));
+      TK_LAUNCH(c, "count", (ceil_div(nreads, rpb) + 7) / 8 * 8, 256, 0, k_count, rview, rb, rb + nreads, t->k,
+                t->canonical, rpb, v, c->d_flags);
+    }
     TK_HIP(hipMemcpyAsync(c->h_flags, c->d_flags, 16, hipMemcpyDeviceToHost, c->stream));
     TK_HIP(hipStreamSynchronize(c->stream));
     if (c->h_flags[0]) return fail(TK_ERR_FULL, "count: table probe limit reached (flags=%u)", c->h_flags[0]);
@@ -3334,7 +3362,7 @@ int tk_read_cov_stats_d(tk_ctx* c, tk_table* t, const tk_reads* r, const tk_stat
     return TK_OK;
   }
   const size_t lds = (size_t)slab * 4 * wpb + (size_t)wpb * 8 * kLookupScratch;
-  const uint32_t grab = read_ticket_grab();
+  const uint32_t grab = read_ticket_grab(c, r->n_reads);
   uint32_t* tickets = grab ? c->d_tickets : nullptr;
   if (tickets) TK_LAUNCH(c, "tickets", 1, 256, 0, k_fill_u32, tickets, kTicketWords, 0u);
   if (max_nwin <= 256 && tickets && stats_pipe()) {
@@ -3546,9 +3574,12 @@ int tk_ctable_build(tk_ctx* c, int k, int canonical, const tk_reads* b, const ui
     if (b->n_reads) {
       hipEvent_t a;
       timing_begin(c, &a);
-      hipLaunchKernelGGL(k_ctable_build, dim3(ceil_div(b->n_reads, kReadsPerBlock)), dim3(256), 0,
-                         c->stream, reads_view(b), dcomp, k, t->canonical, t->d_slots,
-                         t->nbuckets - 1, c->d_flags);
+      // a few waves per slot of the device: each block ends in an atomic on one word
+      const uint64_t cus = (uint64_t)std::max(c->num_cu, 1);
+      const uint32_t per = b->n_words < cus * 128 ? 2 : 32;
+      const uint64_t grid = std::max<uint64_t>(1, std::min<uint64_t>(ceil_div(b->n_words, 4 * per), cus * 32));
+      hipLaunchKernelGGL(k_ctable_build, dim3(grid), dim3(256), 0, c->stream, reads_view(b), b->n_words, per, dcomp,
+                         k, t->canonical, t->d_slots, t->nbuckets - 1, c->d_flags);
       timing_end(c, "ctable_build", a);
       if ((e = hipGetLastError()) != hipSuccess) { rc = hip_fail(e, "k_ctable_build"); break; }
     }
@@ -3584,7 +3615,7 @@ int tk_r2t_vote_reads_d(tk_ctx* c, const tk_ctable* t, const tk_reads* r, tk_r2t
   int rc = reads_order(c, r);
   if (rc) return rc;
   const int grid = (per_read_grid(c, r->n_reads, wpb) + 7) / 8 * 8;
-  const uint32_t grab = read_ticket_grab();
+  const uint32_t grab = read_ticket_grab(c, r->n_reads);
   uint32_t* tickets = grab ? c->d_tickets : nullptr;
   if (tickets) TK_LAUNCH(c, "tickets", 1, 256, 0, k_fill_u32, tickets, kTicketWords, 0u);
   const size_t lds = ((size_t)slab * 4 + 8 * kLookupScratch) * wpb;

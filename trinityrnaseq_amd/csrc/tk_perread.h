@@ -364,7 +364,8 @@ __device__ inline void ctable_add(uint64_t* slots, uint64_t boff, uint64_t bmask
         if (s == 0) { mynew++; s = tagged; }
       }
       if (s == tagged) {
-        atomicMax((unsigned int*)&line[2 * j + 1], ~comp);
+        // a value seen is never above the slot's: it only grows
+        if ((uint32_t)line[2 * j + 1] < ~comp) atomicMax((unsigned int*)&line[2 * j + 1], ~comp);
         return;
       }
     }
