@@ -1115,3 +1115,32 @@ def test_kset_count_tagged_and_errors(api, ctx):
         api.KSet(ctx, np.concatenate([kv[:50], kv[10:11]]))
     empty = api.KSet(ctx, np.zeros((0, 2), np.uint64))
     assert len(empty.count(api.Reads(ctx, seq, off), k, True)) == 0
+
+
+@pytest.mark.parametrize("kk", [31, 32, 33, 48, 63])
+@pytest.mark.parametrize("n", [1, 2048, 2049, (1 << 22), (1 << 22) + 1])
+def test_kset_filter_sizes(api, ctx, n, kk):
+    """Key counts on both sides of a filter size's step and of the largest
+    filtered set, k-mers on both sides of a 64-bit word."""
+    say("kset filter", n, kk)
+    if n > 4096 and kk not in (32, 48):
+        pytest.skip("large sets at one k of each kind")
+    seqs = edge_reads() + random_reads(kk, 300, 0, 400, n_rate=0.01) + random_reads(kk + 1, 2, 5000, 6000)
+    wins = sorted({min(w, brute.rc(w)) for s in seqs for w in (s.upper()[i:i + kk] for i in range(0, len(s) - kk + 1, 7))
+                   if set(w) <= set("ACGT")})
+    kv = _kset_keys(wins[:max(1, n // 2)])
+    rng = np.random.default_rng(n)
+    more = rng.integers(0, 1 << 62, (n - len(kv), 2), dtype=np.uint64)
+    if kk < 63:
+        more[:, 1] &= np.uint64((1 << max(0, 2 * kk - 64)) - 1)
+    if kk < 32:
+        more[:, 0] &= np.uint64((1 << (2 * kk)) - 1)
+    kv = np.unique(np.concatenate([kv, more]), axis=0)
+    seq, off = concat(seqs)
+    ks = api.KSet(ctx, kv)
+    reads = api.Reads(ctx, seq, off)
+    want = O.kset_count(kv, seq, off, kk, True)
+    for _ in range(2):
+        assert np.array_equal(ks.count(reads, kk, True), want)
+    assert int(want.sum()) > 0
+    ks.free()

@@ -31,6 +31,8 @@ struct tk_kset {
   uint64_t* d_slots = nullptr;   // 2 words per slot
   uint32_t* d_idx = nullptr;     // input index per slot
   unsigned long long* d_counts = nullptr;  // per slot
+  uint32_t* d_filter = nullptr;  // 2^fbits bits, one set per key (nullptr: none)
+  uint32_t fbits = 0;
   uint64_t bytes = 0;
 };
 
@@ -52,17 +54,32 @@ constexpr uint64_t kOcc = 1ull << 63;
 inline uint64_t cdiv(uint64_t a, uint64_t b) { return (a + b - 1) / b; }
 
 __device__ __forceinline__ uint64_t ks_hash(uint64_t hi, uint64_t lo) {
-  return mix64(lo ^ mix64(hi + 0x9E3779B97F4A7C15ULL));
+  return mix64(lo ^ (hi * 0x9E3779B97F4A7C15ULL));
 }
+
+// Bit of a hash in the filter: its top bits (the bucket comes from the low ones).
+__device__ __forceinline__ bool ks_maybe(const uint32_t* __restrict__ filter, uint32_t fbits, uint64_t h) {
+  const uint32_t b = (uint32_t)(h >> (64 - fbits));
+  return (filter[b >> 5] >> (b & 31u)) & 1u;
+}
+
+// Most keys of a set that gets a filter: 2^22, whose bits fill one XCD's L2.
+constexpr uint64_t kFilterKeys = 1ull << 22;
 
 // Claim the first empty slot on the key's probe path (keys distinct: no
 // compare needed).  flags[0] |= 1 when the table has no room.
 __global__ void k_ks_build(const uint64_t* __restrict__ keys, uint64_t n, uint64_t* __restrict__ slots,
-                           uint32_t* __restrict__ idx, uint64_t nb, uint32_t* __restrict__ flags) {
+                           uint32_t* __restrict__ idx, uint64_t nb, uint32_t* __restrict__ filter,
+                           uint32_t fbits, uint32_t* __restrict__ flags) {
   for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n;
        i += (uint64_t)gridDim.x * blockDim.x) {
     const uint64_t lo = keys[2 * i], hi = keys[2 * i + 1];
-    uint64_t b = ks_hash(hi, lo) & (nb - 1);
+    const uint64_t h = ks_hash(hi, lo);
+    if (filter) {
+      const uint32_t fb = (uint32_t)(h >> (64 - fbits));
+      atomicOr(&filter[fb >> 5], 1u << (fb & 31u));
+    }
+    uint64_t b = h & (nb - 1);
     bool done = false;
     for (uint64_t p = 0; p < nb && !done; p++) {
       for (int j = 0; j < 4 && !done; j++) {
@@ -80,11 +97,11 @@ __global__ void k_ks_build(const uint64_t* __restrict__ keys, uint64_t n, uint64
   }
 }
 
-// Slot holding (hi, lo), or ~0 when absent.
-__device__ __forceinline__ uint64_t ks_find(const uint64_t* __restrict__ slots, uint64_t nb, uint64_t hi,
+// Slot holding (hi, lo) of hash h, or ~0 when absent.
+__device__ __forceinline__ uint64_t ks_find(const uint64_t* __restrict__ slots, uint64_t nb, uint64_t h, uint64_t hi,
                                             uint64_t lo) {
   const uint64_t w1want = hi | kOcc;
-  uint64_t b = ks_hash(hi, lo) & (nb - 1);
+  uint64_t b = h & (nb - 1);
   for (uint64_t p = 0; p < nb; p++) {
     const ulonglong2* l2 = reinterpret_cast<const ulonglong2*>(slots + b * 8);
 #pragma unroll
@@ -127,18 +144,31 @@ __global__ void k_ks_verify(const uint64_t* __restrict__ keys, uint64_t n, const
 // reverse-complement 2kk-bit values (run of ACGT bases >= kk: valid window),
 // and add one to the slot of each valid window's key.  With tags, the key is
 // (tags[read], k-mer) and kk <= 32.
+//
+// Few of a sample's windows are in a weld set, and each cost a random 64-B
+// line past L2 to find that out (300 k keys, 206 M windows: 3.54 ms, 58 G
+// lines/s).  kFilter: a bit per key, 16 or more bits per key up to 2^21 keys,
+// is asked first; it lies in L2, and only windows whose bit is set go on: the
+// pass with its upload, 4.32 -> 1.94 ms.  What is left runs at the rate of L2
+// hits (180 G windows/s).  Not for tagged sets, whose reads' windows mostly are
+// in the set, nor above 2^22 keys, where a filter of L2's size says little.
+template <bool kFilter>
 __global__ __launch_bounds__(256) void k_ks_count(ReadsView rv, int kk, int canonical,
                                                   const uint32_t* __restrict__ tags,
                                                   const uint64_t* __restrict__ slots, uint64_t nb,
+                                                  const uint32_t* __restrict__ filter, uint32_t fbits,
                                                   unsigned long long* __restrict__ counts) {
-  typedef unsigned __int128 u128;
-  const u128 mask = ((u128)1 << (2 * kk)) - 1;
+  // a base enters the reverse value at bit 2kk-2, in one of its two words
+  const uint64_t mlo = kk >= 32 ? ~0ull : (1ull << (2 * kk)) - 1;
+  const uint64_t mhi = kk > 32 ? (1ull << (2 * kk - 64)) - 1 : 0;
+  const bool top = 2 * kk - 2 >= 64;
+  const int sh = (2 * kk - 2) & 63;
   for (uint64_t r = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; r < rv.n_reads;
        r += (uint64_t)gridDim.x * blockDim.x) {
     const uint32_t len = rv.len[r];
     const uint64_t wbase = rv.word_off[r];
     const uint64_t tag = tags ? (uint64_t)tags[r] : 0;
-    u128 f = 0, rc = 0;
+    uint64_t fl = 0, fh = 0, rl = 0, rh = 0;
     uint32_t run = 0;
     uint64_t code_word = 0;
     uint32_t mask_word = 0;
@@ -147,23 +177,23 @@ __global__ __launch_bounds__(256) void k_ks_count(ReadsView rv, int kk, int cano
         code_word = rv.codes[wbase + (i >> 5)];
         mask_word = rv.nmask[wbase + (i >> 5)];
       }
-      const uint32_t o = i & 31;
-      const uint32_t c = (uint32_t)(code_word >> (62 - 2 * o)) & 3u;
-      const bool bad = (mask_word >> (31 - o)) & 1u;
-      run = bad ? 0 : run + 1;
-      f = ((f << 2) | (u128)c) & mask;
-      rc = (rc >> 2) | ((u128)(3u - c) << (2 * kk - 2));
+      const uint64_t c = code_word >> 62;
+      run = (int32_t)mask_word < 0 ? 0 : run + 1;
+      code_word <<= 2;
+      mask_word <<= 1;
+      fh = ((fh << 2) | (fl >> 62)) & mhi;
+      fl = ((fl << 2) | c) & mlo;
+      rl = (rl >> 2) | (rh << 62);
+      rh >>= 2;
+      const uint64_t in = (c ^ 3u) << sh;
+      if (top) rh |= in;
+      else rl |= in;
       if (run < (uint32_t)kk) continue;
-      const u128 key = (canonical && rc < f) ? rc : f;
-      uint64_t hi, lo;
-      if (tags) {
-        hi = tag;
-        lo = (uint64_t)key;
-      } else {
-        hi = (uint64_t)(key >> 64);
-        lo = (uint64_t)key;
-      }
-      const uint64_t s = ks_find(slots, nb, hi, lo);
+      const bool rev = canonical && (rh < fh || (rh == fh && rl < fl));
+      const uint64_t lo = rev ? rl : fl, hi = tags ? tag : (rev ? rh : fh);
+      const uint64_t h = ks_hash(hi, lo);
+      if (kFilter && !ks_maybe(filter, fbits, h)) continue;
+      const uint64_t s = ks_find(slots, nb, h, hi, lo);
       if (s != ~0ull) atomicAdd(&counts[s], 1ull);
     }
   }
@@ -207,18 +237,25 @@ int tk_kset_create(tk_ctx* c, const uint64_t* keys, uint64_t n, tk_kset** out) {
   int rc = dev_alloc((void**)&s->d_slots, ns * 16);
   if (!rc) rc = dev_alloc((void**)&s->d_idx, ns * 4);
   if (!rc) rc = dev_alloc((void**)&s->d_counts, ns * 8);
+  if (n && n <= kFilterKeys) {
+    s->fbits = 15;
+    while ((1ull << s->fbits) < 16 * n && s->fbits < 25) s->fbits++;
+  }
+  const uint64_t fbytes = s->fbits ? (1ull << s->fbits) / 8 : 0;
+  if (!rc && fbytes) rc = dev_alloc((void**)&s->d_filter, fbytes);
   uint64_t* dk = nullptr;
   if (!rc && n) rc = dev_alloc((void**)&dk, n * 16);
   auto cleanup = [&]() {
     if (dk) dev_free(dk, n * 16);
   };
-  s->bytes = ns * 28;
+  s->bytes = ns * 28 + fbytes;
   if (rc) {
     cleanup();
     tk_kset_free(s);
     return rc;
   }
   hipError_t e = hipMemsetAsync(s->d_slots, 0, ns * 16, c->stream);
+  if (e == hipSuccess && fbytes) e = hipMemsetAsync(s->d_filter, 0, fbytes, c->stream);
   if (e == hipSuccess) e = hipMemsetAsync(c->d_flags, 0, 4, c->stream);
   if (e == hipSuccess && n) e = hipMemcpyAsync(dk, keys, n * 16, hipMemcpyHostToDevice, c->stream);
   if (e != hipSuccess) {
@@ -229,7 +266,8 @@ int tk_kset_create(tk_ctx* c, const uint64_t* keys, uint64_t n, tk_kset** out) {
   auto launch = [&]() -> int {
     if (!n) return TK_OK;
     const uint64_t grid = std::min<uint64_t>(cdiv(n, 256), 65536);
-    KS_LAUNCH(c, "kset_build", grid, 256, k_ks_build, dk, n, s->d_slots, s->d_idx, nb, c->d_flags);
+    KS_LAUNCH(c, "kset_build", grid, 256, k_ks_build, dk, n, s->d_slots, s->d_idx, nb, s->d_filter, s->fbits,
+              c->d_flags);
     KS_LAUNCH(c, "kset_verify", grid, 256, k_ks_verify, dk, n, s->d_slots, nb, c->d_flags);
     return TK_OK;
   };
@@ -281,9 +319,13 @@ int tk_kset_count(tk_ctx* c, tk_kset* s, const tk_reads* reads, int kk, int cano
     rv.word_off = reads->d_word_off;
     rv.len = reads->d_len;
     rv.n_reads = reads->n_reads;
-    if (reads->n_reads)
-      KS_LAUNCH(c, "kset_count", std::min<uint64_t>(cdiv(reads->n_reads, 256), (uint64_t)std::max(c->num_cu, 1) * 32),
-                256, k_ks_count, rv, kk, canonical, dtags, s->d_slots, s->nb, s->d_counts);
+    const uint64_t grid = std::min<uint64_t>(cdiv(reads->n_reads, 256), (uint64_t)std::max(c->num_cu, 1) * 32);
+    if (reads->n_reads && s->d_filter && !dtags)
+      KS_LAUNCH(c, "kset_count", grid, 256, k_ks_count<true>, rv, kk, canonical, dtags, s->d_slots, s->nb,
+                s->d_filter, s->fbits, s->d_counts);
+    else if (reads->n_reads)
+      KS_LAUNCH(c, "kset_count", grid, 256, k_ks_count<false>, rv, kk, canonical, dtags, s->d_slots, s->nb,
+                s->d_filter, s->fbits, s->d_counts);
     if (s->n) {
       KS_LAUNCH(c, "kset_gather", std::min<uint64_t>(cdiv(ns, 256), 65536), 256, k_ks_gather, s->d_slots, s->d_idx,
                 s->d_counts, ns, dout);
@@ -304,6 +346,7 @@ int tk_kset_free(tk_kset* s) {
   tk::dev_free(s->d_slots, ns * 16);
   tk::dev_free(s->d_idx, ns * 4);
   tk::dev_free(s->d_counts, ns * 8);
+  if (s->d_filter) tk::dev_free(s->d_filter, (1ull << s->fbits) / 8);
   delete s;
   return TK_OK;
 }
