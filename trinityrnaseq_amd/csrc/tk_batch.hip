@@ -33,13 +33,27 @@ struct CompLayout {
   uint64_t ct_mask;  // component-table buckets - 1
   uint32_t rbits;
   uint32_t flags;    // kCompCtInLds: the component table is built in LDS (k_batch_ctable_lds)
+  uint32_t piece0;   // first of the regions built in LDS
 };
 
 constexpr uint32_t kCompCtInLds = 1;
-// Component tables of at most kCtLdsBuckets 64-B buckets (64 KB) are built
-// by one workgroup in LDS and written out whole (32 KB when the 64 KB of
-// dynamic LDS cannot be granted).
-constexpr uint64_t kCtLdsBuckets = 1024;
+// Component tables of at most kCtLdsRegions regions (kCtRegion 64-B buckets,
+// 64 KB) are built in LDS, a workgroup per region, and written out whole.  The
+// limit is the LDS counters of k_batch_ctable_split; larger components (1 M
+// windows and more) are few and take the memory-side atomics.
+constexpr uint64_t kCtLdsRegions = 256;
+constexpr int kCtLdsThreads = 1024;
+constexpr uint32_t kCtQueue = 128;  // entries of a wave's queue
+constexpr int kCtSplitSteps = 8;    // two words a step and wave
+constexpr uint32_t kCtSplitWords = 2 * kCtSplitSteps * (kCtLdsThreads / 64);  // words of a workgroup
+
+struct CtPiece {
+  uint32_t comp, region;
+};
+struct CtSplit {
+  uint32_t comp, nwords;
+  uint64_t w0;  // first word, from the component's first
+};
 
 __device__ __forceinline__ TableView comp_view(const TableView& base, const CompLayout& L) {
   TableView v = base;
@@ -266,47 +280,188 @@ __global__ void k_batch_ctable(ReadsView cv, const uint32_t* __restrict__ contig
   }
 }
 
-// The component tables of small components (kCompCtInLds), one workgroup
-// each: the table is built in LDS with the same insert protocol and probe
-// sequence as in global memory (every contig k-mer's word claimed with a
-// CAS, the smallest contig index kept), then written out whole, so each
-// contig window costs an LDS atomic instead of a memory-side one.  Waves
-// take the component's contigs in turn, lanes their windows.
+// A wave's run of a component's packed contig words, lanes at the base
+// positions of two words a step, the next two words in flight.
+struct ContigWalk {
+  uint64_t w, wb, wn, r;
+  words2 x;
+  uint32_t mx, my, len;
+  __device__ __forceinline__ void start(const ReadsView& cv, uint64_t c0, uint64_t c1, uint64_t w0, int lane) {
+    r = c0 + read_of_word(cv.word_off + c0, c1 - c0, w0, lane);
+    w = w0 + ((uint32_t)lane >> 5);
+    wb = cv.word_off[r];
+    wn = cv.word_off[r + 1];
+    len = cv.len[r];
+    x = *reinterpret_cast<const words2*>(cv.codes + w);
+    mx = cv.nmask[w];
+    my = cv.nmask[w + 1];
+  }
+  // Key of the lane's window before word wend and its contig; false: none.
+  __device__ __forceinline__ bool next(const ReadsView& cv, uint64_t wend, int lane, int k, int canonical,
+                                       uint64_t& key, uint64_t& contig) {
+    const words2 nx = *reinterpret_cast<const words2*>(cv.codes + w + 2);  // the arrays end in padding
+    const uint32_t nmx = cv.nmask[w + 2], nmy = cv.nmask[w + 3];
+    if (w < wend && wn <= w) {
+      do r++; while (cv.word_off[r + 1] <= w);
+      wb = cv.word_off[r];
+      wn = cv.word_off[r + 1];
+      len = cv.len[r];
+    }
+    uint64_t f;
+    bool v;
+    const uint32_t o = (uint32_t)lane & 31u;
+    pair_window(x.x, x.y, mx, my, o, k, f, v);
+    v = v && w < wend && (w - wb) * 32 + o + k <= len;
+    key = canon_key(f, k, canonical);
+    contig = r;
+    x = nx;
+    mx = nmx;
+    my = nmy;
+    w += 2;
+    return v;
+  }
+};
+
+// Contig k-mers of the components built in LDS, grouped by table region: each
+// k-mer is computed once, its place among the workgroup's keys of that region
+// counted in LDS, and its slot word written into the region's own memory (as
+// many entries as the region has slots, so half full like the table; a region
+// that gets more is built from the contigs).  cnt: keys of each region.
 template <bool kPacked>
-__global__ __launch_bounds__(256) void k_batch_ctable_lds(ReadsView cv, const uint32_t* __restrict__ comps,
-                                                          const uint64_t* __restrict__ contig_off,
-                                                          const CompLayout* __restrict__ lay, int k, int canonical,
-                                                          uint64_t* __restrict__ ct, uint32_t* __restrict__ flags) {
-  extern __shared__ uint64_t s_ct[];
-  const uint32_t c = comps[blockIdx.x];
-  const CompLayout L = lay[c];
-  const uint64_t words = (L.ct_mask + 1) << 3;
-  for (uint64_t i = threadIdx.x; i < words; i += blockDim.x) s_ct[i] = 0;
+__global__ __launch_bounds__(kCtLdsThreads) void k_batch_ctable_split(ReadsView cv, const CtSplit* __restrict__ splits,
+                                                            const uint64_t* __restrict__ contig_off,
+                                                            const CompLayout* __restrict__ lay, int k, int canonical,
+                                                            uint64_t* __restrict__ ct, uint32_t* __restrict__ cnt) {
+  __shared__ uint32_t s_n[kCtLdsRegions], s_base[kCtLdsRegions];
+  const CtSplit sp = splits[blockIdx.x];
+  const CompLayout L = lay[sp.comp];
+  const uint32_t regions = (uint32_t)((L.ct_mask + 1) >> kCtRegionBits);
+  for (uint32_t i = threadIdx.x; i < regions; i += blockDim.x) s_n[i] = 0;
   __syncthreads();
-  const uint64_t occ = 1ull << (2 * k);
   const int lane = threadIdx.x & 63;
-  const uint64_t wpb = blockDim.x >> 6;
-  uint32_t dummy = 0;
-  const uint64_t c0 = contig_off[c], c1 = contig_off[c + 1];
-  for (uint64_t r = c0 + (threadIdx.x >> 6); r < c1; r += wpb) {
-    const uint32_t local = (uint32_t)(r - c0);
-    const uint32_t len = cv.len[r];
-    const uint32_t nwin = len >= (uint32_t)k ? len - k + 1 : 0;
-    const uint64_t wb = cv.word_off[r];
-    for (uint32_t p = lane; p < nwin; p += 64) {
-      uint64_t fwd;
-      bool valid;
-      window_at(cv, wb, p, k, fwd, valid);
-      if (!valid) continue;
-      if (kPacked)
-        pctable_add(s_ct, 0, L.ct_mask, k, canon_key(fwd, k, canonical), local, &flags[0]);
-      else
-        ctable_add(s_ct, 0, L.ct_mask, occ, canon_key(fwd, k, canonical), local, dummy, &flags[0]);
+  const uint64_t c0 = contig_off[sp.comp], c1 = contig_off[sp.comp + 1];
+  const uint64_t wfirst = cv.word_off[c0] + sp.w0, wlast = wfirst + sp.nwords;
+  const uint64_t w0 = wfirst + (threadIdx.x >> 6) * (2 * kCtSplitSteps);
+  const uint64_t occ = 1ull << (2 * k), vmax = (1ull << (63 - 2 * k)) - 1;
+  uint64_t e[kCtSplitSteps];
+  uint32_t local[kCtSplitSteps], at[kCtSplitSteps];  // at: region << 16 | place, all ones when no window
+#pragma unroll
+  for (int i = 0; i < kCtSplitSteps; i++) at[i] = ~0u;
+  if (w0 < wlast) {
+    ContigWalk cw;
+    cw.start(cv, c0, c1, w0, lane);
+#pragma unroll
+    for (int i = 0; i < kCtSplitSteps; i++) {
+      uint64_t key, r;
+      const bool v = cw.next(cv, wlast, lane, k, canonical, key, r);
+      local[i] = (uint32_t)(r - c0);
+      e[i] = kPacked ? ((vmax - local[i]) << (2 * k + 1)) | occ | key : key;
+      const uint32_t g = (uint32_t)((mix64(key) & L.ct_mask) >> kCtRegionBits);
+      if (v) at[i] = (g << 16) | atomicAdd(&s_n[g], 1u);
+      if (w0 + 2 * (i + 1) >= wlast) break;  // before reads past the arrays' padding
     }
   }
   __syncthreads();
-  uint64_t* g = ct + (L.ct_boff << 3);
-  for (uint64_t i = threadIdx.x; i < words; i += blockDim.x) g[i] = s_ct[i];
+  for (uint32_t i = threadIdx.x; i < regions; i += blockDim.x)
+    if (s_n[i]) s_base[i] = atomicAdd(&cnt[L.piece0 + i], s_n[i]);
+  __syncthreads();
+  constexpr uint32_t kCap = kPacked ? kCtRegion * 8 : kCtRegion * 4;
+#pragma unroll
+  for (int i = 0; i < kCtSplitSteps; i++) {
+    if (at[i] == ~0u) continue;
+    const uint32_t g = at[i] >> 16, p = s_base[g] + (at[i] & 0xFFFFu);
+    if (p >= kCap) continue;
+    uint64_t* to = ct + ((L.ct_boff + ((uint64_t)g << kCtRegionBits)) << 3);
+    if (kPacked) {
+      to[p] = e[i];
+    } else {
+      to[2 * p] = e[i];
+      to[2 * p + 1] = local[i];
+    }
+  }
+}
+
+// One region of a component's table (kCompCtInLds), built in LDS with the
+// same insert protocol and probe sequence as in global memory (every contig
+// k-mer's word claimed with a CAS, the smallest contig index kept), then
+// written out whole: a contig window costs an LDS atomic instead of a
+// memory-side one, which come at 14 G/s (1500 components, 42 M windows: 2.95 ms,
+// 0.23 + 0.60 now, bound by the chains of LDS probes; 2.0 ms with every
+// region's workgroup going over all contigs of its component).
+// The region's keys come from its own memory, where k_batch_ctable_split left
+// them, or, for a table of one region or a region that was sent more than it
+// holds, from the contigs: each wave takes a run of their words, and the
+// region's keys queue up in LDS, so that 64 lanes insert at a time.
+template <bool kPacked>
+__global__ __launch_bounds__(kCtLdsThreads) void k_batch_ctable_lds(ReadsView cv, const CtPiece* __restrict__ pieces,
+                                                          const uint64_t* __restrict__ contig_off,
+                                                          const CompLayout* __restrict__ lay, int k, int canonical,
+                                                          uint64_t* __restrict__ ct, const uint32_t* __restrict__ cnt,
+                                                          uint32_t lds_words, uint32_t* __restrict__ flags) {
+  extern __shared__ uint64_t s_ct[];
+  const CtPiece pc = pieces[blockIdx.x];
+  const CompLayout L = lay[pc.comp];
+  const uint64_t rmask = ct_rmask(L.ct_mask);
+  const uint32_t words = (uint32_t)(rmask + 1) << 3;
+  const uint64_t b0 = (uint64_t)pc.region << kCtRegionBits;
+  uint64_t* g = ct + ((L.ct_boff + b0) << 3);
+  const uint64_t occ = 1ull << (2 * k), vmax = (1ull << (63 - 2 * k)) - 1;
+  const int lane = threadIdx.x & 63;
+  const uint32_t n = cnt[blockIdx.x];
+  uint32_t dummy = 0;
+  for (uint32_t i = threadIdx.x; i < words; i += blockDim.x) s_ct[i] = 0;
+  __syncthreads();
+  // slots of the region's first bucket: the insert adds the bucket's number in the table
+  auto insert = [&](uint64_t e, uint32_t local) {
+    if (kPacked) pctable_put(s_ct, 0 - b0, L.ct_mask, k, e, &flags[0]);
+    else ctable_add(s_ct, 0 - b0, L.ct_mask, occ, e, local, dummy, &flags[0]);
+  };
+  if (L.ct_mask >= kCtRegion && n <= (kPacked ? words : words / 2)) {
+    for (uint32_t i = threadIdx.x; i < n; i += blockDim.x)
+      insert(kPacked ? g[i] : g[2 * i], kPacked ? 0 : (uint32_t)g[2 * i + 1]);
+  } else {
+    const uint32_t wv = threadIdx.x >> 6, nwv = blockDim.x >> 6;
+    uint64_t* q = s_ct + lds_words + wv * kCtQueue;
+    uint32_t* qc = reinterpret_cast<uint32_t*>(s_ct + lds_words + nwv * kCtQueue) + wv * kCtQueue;
+    uint32_t qn = 0;
+    const uint64_t c0 = contig_off[pc.comp], c1 = contig_off[pc.comp + 1];
+    const uint64_t wfirst = cv.word_off[c0], wlast = cv.word_off[c1];
+    const uint64_t per = ((wlast - wfirst + nwv - 1) / nwv + 1) & ~1ull;
+    const uint64_t w0 = wfirst + wv * per, wend = w0 + per < wlast ? w0 + per : wlast;
+    ContigWalk cw;
+    if (w0 < wend) cw.start(cv, c0, c1, w0, lane);
+    for (uint64_t at = w0; at < wend; at += 2) {
+      uint64_t key, r;
+      bool mine = cw.next(cv, wend, lane, k, canonical, key, r);
+      mine = mine && (mix64(key) & L.ct_mask & ~rmask) == b0;
+      const uint64_t m = __ballot(mine);
+      if (mine) {
+        const uint32_t i = qn + __popcll(m & ((1ull << lane) - 1));
+        const uint32_t local = (uint32_t)(r - c0);
+        q[i] = kPacked ? ((vmax - local) << (2 * k + 1)) | occ | key : key;
+        if (!kPacked) qc[i] = local;
+      }
+      qn += (uint32_t)__popcll(m);
+      wave_sync();
+      if (qn >= 64) {
+        insert(q[lane], kPacked ? 0 : qc[lane]);
+        qn -= 64;
+        wave_sync();
+        if ((uint32_t)lane < qn) {
+          q[lane] = q[64 + lane];
+          if (!kPacked) qc[lane] = qc[64 + lane];
+        }
+        wave_sync();
+      }
+    }
+    if ((uint32_t)lane < qn) insert(q[lane], kPacked ? 0 : qc[lane]);
+  }
+  __syncthreads();
+  for (uint32_t i = threadIdx.x; i < words; i += blockDim.x) g[i] = s_ct[i];
+}
+
+static constexpr size_t ct_lds_bytes(bool packed, uint64_t buckets) {
+  return buckets * 64 + (size_t)(kCtLdsThreads / 64) * kCtQueue * (packed ? 8 : 12);
 }
 
 template <bool kPacked>
@@ -357,12 +512,16 @@ struct tk_batch {
   uint64_t n_groups = 0;
   uint32_t* d_order = nullptr;     // reads of each component in locality order (merged count)
   uint64_t* d_contig_off = nullptr;  // contigs of each component (n_comp + 1)
-  uint32_t* d_ct_lds = nullptr;      // components whose table is built in LDS
-  uint64_t n_ct_lds = 0, ct_lds_bytes = 0;
+  CtPiece* d_ct_lds = nullptr;       // the table regions built in LDS
+  uint64_t n_ct_lds = 0, ct_lds_buckets = 0;
+  CtSplit* d_ct_split = nullptr;     // runs of contig words of the tables of several regions
+  uint64_t n_ct_split = 0;
+  uint32_t* d_ct_cnt = nullptr;      // keys sent to each region
   uint64_t* d_slots = nullptr;
   uint64_t* d_ovf = nullptr;
   uint64_t* d_ct = nullptr;
   uint64_t n_slots_words = 0, n_ovf_pairs = 0, n_ct_words = 0;
+  uint64_t n_ct_clear = 0;  // words of the component tables not built in LDS (the first ones)
   uint64_t bytes = 0;
   // captured launch sequence
   hipGraph_t graph = nullptr;
@@ -372,7 +531,7 @@ struct tk_batch {
   tk_stats_opts g_opts{};
   // host copies for re-layout
   std::vector<uint64_t> read_off, contig_off;
-  std::vector<uint64_t> comp_windows, comp_cwindows;
+  std::vector<uint64_t> comp_windows, comp_cwindows, comp_cwords;
 };
 
 static void batch_release_device(tk_batch* b) {
@@ -382,22 +541,28 @@ static void batch_release_device(tk_batch* b) {
   dev_free(b->d_ovf, b->n_ovf_pairs * 16);
   dev_free(b->d_ct, b->n_ct_words * 8);
   dev_free(b->d_lay, b->n_comp * sizeof(CompLayout));
-  dev_free(b->d_ct_lds, std::max<uint64_t>(b->n_ct_lds, 1) * 4);
+  dev_free(b->d_ct_lds, std::max<uint64_t>(b->n_ct_lds, 1) * sizeof(CtPiece));
+  dev_free(b->d_ct_cnt, std::max<uint64_t>(b->n_ct_lds, 1) * 4);
+  dev_free(b->d_ct_split, std::max<uint64_t>(b->n_ct_split, 1) * sizeof(CtSplit));
   b->d_slots = b->d_ovf = b->d_ct = nullptr;
   b->d_lay = nullptr;
   b->d_ct_lds = nullptr;
-  b->n_ct_lds = b->ct_lds_bytes = 0;
+  b->d_ct_cnt = nullptr;
+  b->d_ct_split = nullptr;
+  b->n_ct_lds = b->ct_lds_buckets = b->n_ct_split = 0;
 }
 
-// Whether k_batch_ctable_lds may take 64 KB of dynamic LDS (the attribute is
+// Whether k_batch_ctable_lds may take a whole region's LDS (the attribute is
 // set once per process; a function-local static is initialised once even
 // when several threads get here together).
-static bool ct_lds_64k() {
+static bool ct_lds_ok() {
   static const bool ok = [] {
     const bool r = hipFuncSetAttribute(reinterpret_cast<const void*>(&k_batch_ctable_lds<true>),
-                                       hipFuncAttributeMaxDynamicSharedMemorySize, 65536) == hipSuccess &&
+                                       hipFuncAttributeMaxDynamicSharedMemorySize,
+                                       (int)ct_lds_bytes(true, kCtRegion)) == hipSuccess &&
                    hipFuncSetAttribute(reinterpret_cast<const void*>(&k_batch_ctable_lds<false>),
-                                       hipFuncAttributeMaxDynamicSharedMemorySize, 65536) == hipSuccess;
+                                       hipFuncAttributeMaxDynamicSharedMemorySize,
+                                       (int)ct_lds_bytes(false, kCtRegion)) == hipSuccess;
     (void)hipGetLastError();
     return r;
   }();
@@ -410,6 +575,8 @@ static int batch_layout(tk_ctx* c, tk_batch* b) {
   std::vector<CompLayout> lay(b->n_comp);
   uint64_t boff = 0, ooff = 0, coff = 0;
   const uint32_t cbits = 63 - 2 * b->k;
+  const char* ev = getenv("TK_BATCH_CT_LDS");  // 0: no component table is built in LDS
+  const bool ct_lds = !(ev && ev[0] == '0') && ct_lds_ok() && b->n_comp <= 0xFFFFFFFFull;
   for (uint64_t i = 0; i < b->n_comp; i++) {
     CompLayout& L = lay[i];
     const uint64_t w = b->comp_windows[i];
@@ -426,40 +593,49 @@ static int batch_layout(tk_ctx* c, tk_batch* b) {
     // buckets of eight packed or four two-word slots, at most half full
     const uint64_t cb = p2(std::max<uint64_t>(b->ct_packed ? (2 * b->comp_cwindows[i] + 7) / 8
                                                             : (2 * b->comp_cwindows[i] + 3) / 4, 4));
-    L.ct_boff = coff;
     L.ct_mask = cb - 1;
-    coff += cb;
-    L.flags = cb <= kCtLdsBuckets ? kCompCtInLds : 0u;
+    L.flags = ct_lds && cb <= kCtLdsRegions * kCtRegion && b->contig_off[i + 1] > b->contig_off[i] ? kCompCtInLds : 0u;
+  }
+  // the tables that are cleared and filled in place first, then the ones built
+  // in LDS, whose regions are written whole
+  std::vector<CtPiece> pieces;
+  std::vector<CtSplit> splits;
+  for (uint32_t in_lds : {0u, kCompCtInLds}) {
+    for (uint64_t i = 0; i < b->n_comp; i++) {
+      CompLayout& L = lay[i];
+      if (L.flags != in_lds) continue;
+      const uint64_t cb = L.ct_mask + 1;
+      L.ct_boff = coff;
+      coff += cb;
+      if (!in_lds) continue;
+      L.piece0 = (uint32_t)pieces.size();
+      for (uint64_t x = 0; cb > kCtRegion && x < b->comp_cwords[i]; x += kCtSplitWords)
+        splits.push_back({(uint32_t)i, (uint32_t)std::min<uint64_t>(kCtSplitWords, b->comp_cwords[i] - x), x});
+      for (uint64_t g = 0; g < cb; g += kCtRegion) pieces.push_back({(uint32_t)i, (uint32_t)(g >> kCtRegionBits)});
+      b->ct_lds_buckets = std::max(b->ct_lds_buckets, std::min(cb, kCtRegion));
+    }
+    if (!in_lds) b->n_ct_clear = coff * 8;
   }
   b->n_slots_words = boff * 8;
   b->n_ovf_pairs = ooff;
   b->n_ct_words = coff * 8;
-  // components whose table is built in LDS (TK_BATCH_CT_LDS=0: none); one
-  // launch takes them all, with the LDS of the largest
-  std::vector<uint32_t> small;
-  {
-    const char* ev = getenv("TK_BATCH_CT_LDS");
-    const bool on = !(ev && ev[0] == '0');
-    const uint64_t max_buckets = ct_lds_64k() ? kCtLdsBuckets : kCtLdsBuckets / 2;
-    for (uint64_t i = 0; i < b->n_comp; i++) {
-      if (!on || lay[i].ct_mask + 1 > max_buckets) lay[i].flags &= ~kCompCtInLds;
-      if ((lay[i].flags & kCompCtInLds) && b->contig_off[i + 1] > b->contig_off[i]) {
-        small.push_back((uint32_t)i);
-        b->ct_lds_bytes = std::max<uint64_t>(b->ct_lds_bytes, (lay[i].ct_mask + 1) * 64);
-      }
-    }
-  }
-  b->n_ct_lds = small.size();
+  b->n_ct_lds = pieces.size();
+  b->n_ct_split = splits.size();
   int rc = dev_alloc((void**)&b->d_slots, b->n_slots_words * 8);
   if (!rc) rc = dev_alloc((void**)&b->d_ovf, b->n_ovf_pairs * 16);
   if (!rc) rc = dev_alloc((void**)&b->d_ct, b->n_ct_words * 8);
   if (!rc) rc = dev_alloc((void**)&b->d_lay, b->n_comp * sizeof(CompLayout));
-  if (!rc) rc = dev_alloc((void**)&b->d_ct_lds, std::max<uint64_t>(b->n_ct_lds, 1) * 4);
+  if (!rc) rc = dev_alloc((void**)&b->d_ct_lds, std::max<uint64_t>(b->n_ct_lds, 1) * sizeof(CtPiece));
+  if (!rc) rc = dev_alloc((void**)&b->d_ct_cnt, std::max<uint64_t>(b->n_ct_lds, 1) * 4);
+  if (!rc) rc = dev_alloc((void**)&b->d_ct_split, std::max<uint64_t>(b->n_ct_split, 1) * sizeof(CtSplit));
   if (rc) return rc;
   TK_HIP(hipMemcpyAsync(b->d_lay, lay.data(), b->n_comp * sizeof(CompLayout), hipMemcpyHostToDevice,
                         c->stream));
   if (b->n_ct_lds)
-    TK_HIP(hipMemcpyAsync(b->d_ct_lds, small.data(), b->n_ct_lds * 4, hipMemcpyHostToDevice, c->stream));
+    TK_HIP(hipMemcpyAsync(b->d_ct_lds, pieces.data(), b->n_ct_lds * sizeof(CtPiece), hipMemcpyHostToDevice, c->stream));
+  if (b->n_ct_split)
+    TK_HIP(hipMemcpyAsync(b->d_ct_split, splits.data(), b->n_ct_split * sizeof(CtSplit), hipMemcpyHostToDevice,
+                          c->stream));
   TK_HIP(hipStreamSynchronize(c->stream));
   b->bytes = b->n_slots_words * 8 + b->n_ovf_pairs * 16 + b->n_ct_words * 8;
   return TK_OK;
@@ -530,15 +706,31 @@ static int batch_enqueue(tk_ctx* c, tk_batch* b, const tk_stats_opts* o, tk_read
                          b->d_lay, b->k, b->canonical, base, sp, d_stats, slab);
   }
   if (d_votes && rv.n_reads) {
-    hipLaunchKernelGGL(k_fill_zero, dim3(grid(b->n_ct_words, 256)), dim3(256), 0, c->stream, b->d_ct, b->n_ct_words);
+    if (b->n_ct_clear)
+      hipLaunchKernelGGL(k_fill_zero, dim3(grid(b->n_ct_clear, 256)), dim3(256), 0, c->stream, b->d_ct, b->n_ct_clear);
     const ReadsView cv = rview(b->contigs);
     const size_t vlds = ((size_t)slab * 4 + 8 * kLookupScratch) * wpb;
+    const size_t clds = ct_lds_bytes(b->ct_packed, b->ct_lds_buckets);
+    const uint32_t cwords = (uint32_t)(b->ct_lds_buckets * 8);
+    if (b->n_ct_split) {
+      hipLaunchKernelGGL(k_fill_zero32, dim3(grid(b->n_ct_lds, 256)), dim3(256), 0, c->stream, b->d_ct_cnt,
+                         (uint32_t)b->n_ct_lds);
+      if (b->ct_packed)
+        hipLaunchKernelGGL(k_batch_ctable_split<true>, dim3((unsigned)b->n_ct_split), dim3(kCtLdsThreads), 0,
+                           c->stream, cv, b->d_ct_split, b->d_contig_off, b->d_lay, b->k, b->canonical, b->d_ct,
+                           b->d_ct_cnt);
+      else
+        hipLaunchKernelGGL(k_batch_ctable_split<false>, dim3((unsigned)b->n_ct_split), dim3(kCtLdsThreads), 0,
+                           c->stream, cv, b->d_ct_split, b->d_contig_off, b->d_lay, b->k, b->canonical, b->d_ct,
+                           b->d_ct_cnt);
+    }
     if (b->n_ct_lds && b->ct_packed)
-      hipLaunchKernelGGL(k_batch_ctable_lds<true>, dim3((unsigned)b->n_ct_lds), dim3(256), b->ct_lds_bytes, c->stream,
-                         cv, b->d_ct_lds, b->d_contig_off, b->d_lay, b->k, b->canonical, b->d_ct, c->d_flags);
+      hipLaunchKernelGGL(k_batch_ctable_lds<true>, dim3((unsigned)b->n_ct_lds), dim3(kCtLdsThreads), clds, c->stream,
+                         cv, b->d_ct_lds, b->d_contig_off, b->d_lay, b->k, b->canonical, b->d_ct, b->d_ct_cnt, cwords,
+                         c->d_flags);
     else if (b->n_ct_lds)
-      hipLaunchKernelGGL(k_batch_ctable_lds<false>, dim3((unsigned)b->n_ct_lds), dim3(256), b->ct_lds_bytes,
-                         c->stream, cv, b->d_ct_lds, b->d_contig_off, b->d_lay, b->k, b->canonical, b->d_ct,
+      hipLaunchKernelGGL(k_batch_ctable_lds<false>, dim3((unsigned)b->n_ct_lds), dim3(kCtLdsThreads), clds, c->stream,
+                         cv, b->d_ct_lds, b->d_contig_off, b->d_lay, b->k, b->canonical, b->d_ct, b->d_ct_cnt, cwords,
                          c->d_flags);
     if (b->ct_packed) {
       if (cv.n_reads)
@@ -647,6 +839,7 @@ int tk_batch_create(tk_ctx* c, int k, int canonical, const tk_reads* reads, cons
   if (e != hipSuccess) { delete b; return hip_fail(e, "batch lengths"); }
   b->comp_windows.assign(n_comp, 0);
   b->comp_cwindows.assign(n_comp, 0);
+  b->comp_cwords.assign(n_comp, 0);
   std::vector<uint32_t> rcomp(reads->n_reads), ccomp(contigs->n_reads), clocal(contigs->n_reads);
   for (uint64_t i = 0; i < n_comp; i++) {
     for (uint64_t r = read_comp_off[i]; r < read_comp_off[i + 1]; r++) {
@@ -658,6 +851,7 @@ int tk_batch_create(tk_ctx* c, int k, int canonical, const tk_reads* reads, cons
       ccomp[r] = (uint32_t)i;
       clocal[r] = (uint32_t)(r - contig_comp_off[i]);
       b->comp_cwindows[i] += cl[r] >= (uint32_t)k ? cl[r] - k + 1 : 0;
+      b->comp_cwords[i] += ((uint64_t)cl[r] + 31) / 32;
     }
   }
   if ((uint64_t)(std::max<uint32_t>(64, (b->max_nwin + 63) / 64 * 64)) * 4 + 8 * kLookupScratch > 65536) {

@@ -193,6 +193,21 @@ __device__ __forceinline__ LaneWords lane_words(const ReadsView& rv, uint64_t wb
   return w;
 }
 
+// Last read whose first word is at or before word w (the read holding w; empty
+// reads before it are passed over), found by the whole wave: 64 pivots a step.
+__device__ __forceinline__ uint64_t read_of_word(const uint64_t* __restrict__ word_off, uint64_t n_reads, uint64_t w,
+                                                 int lane) {
+  uint64_t lo = 0, hi = n_reads;
+  while (hi - lo > 1) {
+    const uint64_t step = (hi - lo + 63) >> 6;
+    const uint64_t p = lo + (uint64_t)lane * step;
+    const uint64_t m = __ballot(p < hi && word_off[p] <= w);
+    lo += (uint64_t)(63 - __clzll((long long)(m | 1ull))) * step;
+    hi = hi < lo + step ? hi : lo + step;
+  }
+  return lo;
+}
+
 // Forward k-mer at base o (< 32) of the word pair (hi, lo) with masks (mhi, mlo).
 __device__ __forceinline__ void pair_window(uint64_t hi, uint64_t lo, uint32_t mhi, uint32_t mlo, uint32_t o, int k,
                                             uint64_t& fwd, bool& valid) {

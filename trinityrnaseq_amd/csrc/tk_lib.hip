@@ -1834,21 +1834,6 @@ __global__ __launch_bounds__(256) void k_select(const tk_read_stat* __restrict__
 // =====================================================================
 // ReadsToTranscripts
 // =====================================================================
-// Last read whose first word is at or before word w (the read holding w; empty
-// reads before it are passed over), found by the whole wave: 64 pivots a step.
-__device__ __forceinline__ uint64_t read_of_word(const uint64_t* __restrict__ word_off, uint64_t n_reads, uint64_t w,
-                                                 int lane) {
-  uint64_t lo = 0, hi = n_reads;
-  while (hi - lo > 1) {
-    const uint64_t step = (hi - lo + 63) >> 6;
-    const uint64_t p = lo + (uint64_t)lane * step;
-    const uint64_t m = __ballot(p < hi && word_off[p] <= w);
-    lo += (uint64_t)(63 - __clzll((long long)(m | 1ull))) * step;
-    hi = hi < lo + step ? hi : lo + step;
-  }
-  return lo;
-}
-
 // Lane per base position: a wave takes `per` packed words (two at a time),
 // whatever reads they belong to, so a few long sequences fill the device as
 // well as many short ones (a block per 64 sequences, looping over their

@@ -350,12 +350,21 @@ __device__ inline void stats_read_cached(const ReadsView& rv, uint64_t r, int k,
 }
 
 // Component table: 64-byte buckets of four 16-byte slots (tagged key, ~comp);
-// buckets [boff, boff + bmask] belong to one table.
+// buckets [boff, boff + bmask] belong to one table.  A key's probe sequence
+// wraps within its region of 1024 buckets (half full over its 4096 or 8192
+// slots), so a region can be built apart from the others (k_batch_ctable_lds).
+constexpr uint32_t kCtRegionBits = 10;
+constexpr uint64_t kCtRegion = 1ull << kCtRegionBits;
+
+__device__ __forceinline__ uint64_t ct_rmask(uint64_t bmask) { return bmask < kCtRegion ? bmask : kCtRegion - 1; }
+__device__ __forceinline__ uint64_t ct_next(uint64_t b, uint64_t rmask) { return (b & ~rmask) | ((b + 1) & rmask); }
+
 __device__ inline void ctable_add(uint64_t* slots, uint64_t boff, uint64_t bmask, uint64_t occ,
                                   uint64_t key, uint32_t comp, uint32_t& mynew, uint32_t* err) {
   const uint64_t tagged = key | occ;
+  const uint64_t rmask = ct_rmask(bmask);
   uint64_t b = mix64(key) & bmask;
-  for (uint64_t p = 0; p <= bmask && p < 4096; p++) {
+  for (uint64_t p = 0; p <= rmask; p++) {
     uint64_t* line = slots + ((boff + b) << 3);
     for (int j = 0; j < 4; j++) {
       uint64_t s = line[2 * j];
@@ -369,7 +378,7 @@ __device__ inline void ctable_add(uint64_t* slots, uint64_t boff, uint64_t bmask
         return;
       }
     }
-    b = (b + 1) & bmask;
+    b = ct_next(b, rmask);
   }
   atomicOr(err, 1u);
 }
@@ -378,13 +387,12 @@ __device__ inline void ctable_add(uint64_t* slots, uint64_t boff, uint64_t bmask
 // [vmax - comp : 63-2k | occupied : 1 | key : 2k], vmax = 2^(63-2k) - 1, so
 // a new key costs one CAS and the largest word of one key holds its
 // smallest comp; comp <= vmax.
-__device__ inline void pctable_add(uint64_t* slots, uint64_t boff, uint64_t bmask, int k, uint64_t key,
-                                   uint32_t comp, uint32_t* err) {
-  const uint64_t occ = 1ull << (2 * k), km = (occ << 1) - 1, tagged = key | occ;
-  const uint64_t vmax = (1ull << (63 - 2 * k)) - 1;
-  const uint64_t word = ((vmax - comp) << (2 * k + 1)) | tagged;
-  uint64_t b = mix64(key) & bmask;
-  for (uint64_t p = 0; p <= bmask && p < 4096; p++) {
+__device__ inline void pctable_put(uint64_t* slots, uint64_t boff, uint64_t bmask, int k, uint64_t word,
+                                   uint32_t* err) {
+  const uint64_t occ = 1ull << (2 * k), km = (occ << 1) - 1, tagged = word & km;
+  const uint64_t rmask = ct_rmask(bmask);
+  uint64_t b = mix64(word & (occ - 1)) & bmask;
+  for (uint64_t p = 0; p <= rmask; p++) {
     uint64_t* line = slots + ((boff + b) << 3);
     for (int j = 0; j < 8; j++) {
       uint64_t s = line[j];
@@ -397,9 +405,15 @@ __device__ inline void pctable_add(uint64_t* slots, uint64_t boff, uint64_t bmas
         return;
       }
     }
-    b = (b + 1) & bmask;
+    b = ct_next(b, rmask);
   }
   atomicOr(err, 1u);
+}
+
+__device__ inline void pctable_add(uint64_t* slots, uint64_t boff, uint64_t bmask, int k, uint64_t key,
+                                   uint32_t comp, uint32_t* err) {
+  const uint64_t vmax = (1ull << (63 - 2 * k)) - 1;
+  pctable_put(slots, boff, bmask, k, ((vmax - comp) << (2 * k + 1)) | (1ull << (2 * k)) | key, err);
 }
 
 __device__ __forceinline__ uint32_t pctable_comp(uint64_t s, int k) {
@@ -433,9 +447,10 @@ struct PtLayout {  // eight one-word slots, two per lane
 template <class L>
 __device__ __forceinline__ uint64_t comp_after(const uint64_t* slots, uint64_t boff, uint64_t bmask, const L& lay,
                                                uint64_t key, uint64_t tag) {
+  const uint64_t rmask = ct_rmask(bmask);
   uint64_t b = mix64(key) & bmask;
-  for (uint64_t p = 1; p <= bmask && p < 4096; p++) {
-    b = (b + 1) & bmask;
+  for (uint64_t p = 1; p <= rmask; p++) {
+    b = ct_next(b, rmask);
     const ulonglong2* l2 = reinterpret_cast<const ulonglong2*>(slots + ((boff + b) << 3));
     const ulonglong2 v[4] = {l2[0], l2[1], l2[2], l2[3]};
     uint64_t res = L::kNone, x;
