@@ -1023,6 +1023,21 @@ def test_inchworm_parity_forced_rounds(api, ctx, monkeypatch, walks, lmax):
     say("  ", info)
 
 
+@pytest.mark.parametrize("walks", [2, 7, 300, 16384])
+@pytest.mark.parametrize("genome_len,err", [(300, 0.06), (6000, 0.02)])
+def test_inchworm_parity_conflicting_walks(api, ctx, monkeypatch, genome_len, err, walks):
+    """Walks that take each other's k-mers: a short, error-rich genome (many
+    branches off the same contigs) and a longer one, in epochs of few and of
+    all seeds, path buffers that some walks outgrow."""
+    say("inchworm_parity_conflicting_walks", genome_len, err, walks)
+    monkeypatch.setenv("TK_IWORM_WALKS", str(walks))
+    monkeypatch.setenv("TK_IWORM_LMAX", "64")
+    seqs = repetitive_reads(91 + genome_len, 2000, genome_len=genome_len, read_len=80, err=err)
+    for k in (13, 25):
+        r, t, _, _ = _count(api, ctx, seqs, k, True)
+        say("  ", _iworm_check(api, ctx, t, k, True, 1))
+
+
 @pytest.mark.parametrize("k", [13, 25, 31])
 def test_inchworm_parity_pruned_with_seed_entropy(api, ctx, k):
     """After Inchworm's prune (min count 2, entropy 1.0), seeds filtered by a

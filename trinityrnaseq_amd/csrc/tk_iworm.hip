@@ -9,22 +9,24 @@
 //
 //  * seeds: the table's keys with count >= min_seed_cov (and a seed-entropy
 //    composition table) sorted by key, then stably by inverted count;
-//  * rounds: the next B seeds still unused are walked at once, one four-lane
+//  * epochs: the next B seeds still unused are walked at once, one four-lane
 //    group per walk (lane b looks up the candidate ending, or starting, with
-//    base b).  Walk w of round base S has rank S+1+w; a walk claims each
+//    base b).  Walk w of epoch base S has rank S+1+w; a walk claims each
 //    k-mer it takes with atomicMin(claim[slot], rank), so a k-mer goes to the
 //    earliest walk that wants it and a later walk that held it is marked lost.
-//    A walk treats k-mers claimed by earlier ranks (committed rounds, or
-//    earlier walks of this round) as used;
-//  * commit: in rank order, walks that finished without losing a k-mer, and
-//    seeds an earlier walk had already taken (skipped), form the committed
-//    prefix; the first lost or overflowing walk ends it.  By induction every
-//    committed walk equals the serial greedy walk: the earlier walks it saw
-//    as claimers are committed with exactly those k-mers, and any k-mer an
-//    earlier serial walk takes was taken from it in this round (it would be
-//    lost).  Walks past the prefix release their claims and are walked again
-//    in a later round; the first walk of a round always commits, so every
-//    round progresses.
+//    A walk treats k-mers claimed by earlier ranks (committed epochs, or
+//    earlier walks of this one) as used and records the latter;
+//  * rounds: a walk holds if it lost no k-mer and every earlier walk whose
+//    k-mers it treated as used holds and gives a contig, or if its seed was
+//    taken by such a walk (skipped).  The others give their claims back and
+//    are walked again with their ranks, the rest keep theirs, until all hold:
+//    a round lasts as long as its longest walk, and few walks are ever in
+//    conflict (3 to 16 of 16,384 beyond the seeds taken).  The earliest walk
+//    of a round sees only walks that stay and so holds afterwards;
+//  * commit: when every walk of the epoch holds, each equals the serial greedy
+//    walk: the earlier walks it saw as claimers have exactly those k-mers, and
+//    any k-mer an earlier serial walk takes was taken from it (it would be
+//    lost).
 //
 // Claims are one u32 per table slot (tables of < 2^32 slots).
 #include <stdlib.h>
@@ -263,14 +265,14 @@ __global__ __launch_bounds__(1024) void k_iw_pick(const uint32_t* __restrict__ s
 struct WalkParams {
   TableView t;
   uint64_t kmask;
-  uint32_t S;       // ranks of this round: S+1 ... S+n
-  uint32_t n;       // walks
+  uint32_t S;       // ranks of this epoch: S+1 ... S+walks
+  uint32_t n;       // walks of this round
   uint32_t lmax;    // path entries per walk and side
   int k;
   int canonical;
 };
 
-constexpr uint32_t kDeps = 8;  // recorded dependencies per walk (more: the walk is redone)
+constexpr uint32_t kDeps = 8;  // recorded dependencies per walk (more: walked again as a round's first)
 
 // Record that walk w treated a k-mer claimed by earlier walk `dep` of this
 // round as used (the decision holds only if that walk commits a contig).
@@ -340,14 +342,16 @@ __device__ __forceinline__ uint64_t iw_resolve(const TableView& t, const uint32_
 // rank is seen to hold is dropped without an atomic (claims only fall within a
 // round, so what an out-of-date word says is held, is).  Each group changes
 // side on its own.  120 k reads' dictionary: 3.98 -> 2.94 ms a round.
-__global__ __launch_bounds__(256) void k_iw_walk(WalkParams p, const uint32_t* __restrict__ picked_slot,
+__global__ __launch_bounds__(256) void k_iw_walk(WalkParams p, const uint32_t* __restrict__ list,
+                                                 const uint32_t* __restrict__ picked_slot,
                                                  uint32_t* claim, uint32_t* __restrict__ lost,
                                                  uint32_t* __restrict__ status, uint32_t* __restrict__ lens,
                                                  uint64_t* __restrict__ sums, uint32_t* __restrict__ path_slot,
                                                  uint8_t* __restrict__ path_base, uint32_t* __restrict__ deps,
                                                  uint32_t* __restrict__ dep_n) {
-  const uint32_t w = (blockIdx.x * blockDim.x + threadIdx.x) >> 2;
-  if (w >= p.n) return;  // whole groups leave together
+  const uint32_t g = (blockIdx.x * blockDim.x + threadIdx.x) >> 2;
+  if (g >= p.n) return;  // whole groups leave together
+  const uint32_t w = list ? list[g] : g;
   const int b = threadIdx.x & 3;
   const TableView& t = p.t;
   const uint32_t r = p.S + 1 + w;
@@ -449,7 +453,16 @@ __global__ __launch_bounds__(256) void k_iw_walk(WalkParams p, const uint32_t* _
   }
 }
 
-// The seed slot's final claim of every walk (its own rank unless an earlier
+// Walks about to be walked again.
+__global__ void k_iw_reset(const uint32_t* __restrict__ list, uint32_t n, uint32_t* __restrict__ lost,
+                           uint32_t* __restrict__ dep_n) {
+  for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) {
+    lost[list[i]] = 0;
+    dep_n[list[i]] = 0;
+  }
+}
+
+// The seed slot's claim of every walk (its own rank unless an earlier
 // walk took the seed).
 __global__ void k_iw_owner(const uint32_t* __restrict__ picked_slot, uint32_t n, const uint32_t* __restrict__ claim,
                            uint32_t* __restrict__ owner) {
@@ -557,7 +570,7 @@ int inchworm_run(tk_ctx* c, tk_table* t, uint32_t min_seed_cov, const uint8_t* s
   IW_LAUNCH(c, "iworm_fill", std::min<uint64_t>(cdiv(n_slots, 256), 65536), 256, k_iw_fill,
             dclaim.as<uint32_t>(), n_slots, kFree);
   // ---- rounds
-  // TK_IWORM_WALKS caps the walks per round (default 16,384, starting at
+  // TK_IWORM_WALKS caps the walks per epoch (default 16,384, starting at
   // 1,024) and TK_IWORM_LMAX sets the first path capacity per walk side
   // (default 4,096 k-mers): small values force the conflict and regrowth
   // paths on small inputs.
@@ -609,7 +622,9 @@ int inchworm_run(tk_ctx* c, tk_table* t, uint32_t min_seed_cov, const uint8_t* s
   uint32_t* h_rel = h_owner + Bmax;
   uint32_t* h_walks = h_rel + Bmax;
   uint32_t* h_deps = h_walks + Bmax;  // Bmax * kDeps
-  std::vector<uint8_t> late(Bmax);
+  enum : uint8_t { kBad, kContig, kSkipped };
+  std::vector<uint8_t> state(Bmax), late(Bmax);  // late: its seed was taken by walk late_by while it ran
+  std::vector<uint32_t> late_by(Bmax);
   uint64_t cursor = 0;
   uint32_t S = 0;
   std::string chunk;
@@ -626,94 +641,104 @@ int inchworm_run(tk_ctx* c, tk_table* t, uint32_t min_seed_cov, const uint8_t* s
     TK_HIP(hipStreamSynchronize(c->stream));
     const uint32_t n = (uint32_t)h_out[0];
     if (n == 0) break;
-    res->rounds++;
-    res->walks += n;
     IW_LAUNCH(c, "iworm_fill", cdiv(n, 256), 256, k_iw_fill, dlost.as<uint32_t>(), (uint64_t)n, 0u);
     IW_LAUNCH(c, "iworm_fill", cdiv(n, 256), 256, k_iw_fill, ddepn.as<uint32_t>(), (uint64_t)n, 0u);
+    TK_HIP(hipMemcpyAsync(h_pos, dpos.p, (size_t)n * 8, hipMemcpyDeviceToHost, c->stream));
     WalkParams wp;
     wp.t = v;
     wp.kmask = k >= 32 ? ~0ull : ((1ull << (2 * k)) - 1);
     wp.S = S;
-    wp.n = n;
     wp.lmax = lmax;
     wp.k = k;
     wp.canonical = t->canonical;
-    IW_LAUNCH(c, "iworm_walk", cdiv((uint64_t)n * 4, 256), 256, k_iw_walk, wp, dpick.as<uint32_t>(),
-              dclaim.as<uint32_t>(), dlost.as<uint32_t>(), dstat.as<uint32_t>(), dlens.as<uint32_t>(),
-              dsums.as<uint64_t>(), dpslot.as<uint32_t>(), dpbase.as<uint8_t>(), ddeps.as<uint32_t>(),
-              ddepn.as<uint32_t>());
-    IW_LAUNCH(c, "iworm_owner", cdiv(n, 256), 256, k_iw_owner, dpick.as<uint32_t>(), n, dclaim.as<uint32_t>(),
-              downer.as<uint32_t>());
-    TK_HIP(hipMemcpyAsync(h_depn, ddepn.p, n * 4, hipMemcpyDeviceToHost, c->stream));
-    TK_HIP(hipMemcpyAsync(h_deps, ddeps.p, (size_t)n * kDeps * 4, hipMemcpyDeviceToHost, c->stream));
-    TK_HIP(hipMemcpyAsync(h_owner, downer.p, n * 4, hipMemcpyDeviceToHost, c->stream));
-    TK_HIP(hipMemcpyAsync(h_stat, dstat.p, n * 4, hipMemcpyDeviceToHost, c->stream));
-    TK_HIP(hipMemcpyAsync(h_lost, dlost.p, n * 4, hipMemcpyDeviceToHost, c->stream));
-    TK_HIP(hipMemcpyAsync(h_lens, dlens.p, (size_t)n * 8, hipMemcpyDeviceToHost, c->stream));
-    TK_HIP(hipMemcpyAsync(h_sums, dsums.p, (size_t)n * 8, hipMemcpyDeviceToHost, c->stream));
-    TK_HIP(hipMemcpyAsync(h_pos, dpos.p, (size_t)n * 8, hipMemcpyDeviceToHost, c->stream));
-    TK_HIP(hipStreamSynchronize(c->stream));
-    // Committed prefix, in rank order.  A walk whose seed an earlier walk of
-    // the round took ("late skip") is the serial skip of that seed when the
-    // taker commits a contig; its own claims are void.  Any decision that
-    // treated a k-mer as used because an earlier walk of the round held it
-    // (the dependencies) holds only if that walk commits a contig, i.e. is
-    // not a late skip.  Seeds claimed at the start by an earlier walk are
-    // skips under the same condition.  The first walk that lost a k-mer
-    // without losing its seed, outgrew its buffers or recorded too many
-    // dependencies ends the prefix.
-    uint32_t P = n;
-    for (uint32_t i = 0; i < n; i++) {
-      late[i] = 0;
-      bool deps_ok = h_depn[i] <= kDeps;
-      for (uint32_t j = 0; deps_ok && j < h_depn[i]; j++) {
-        const uint32_t d = h_deps[(size_t)i * kDeps + j];
-        deps_ok = d < i && !late[d];
-      }
-      const uint32_t r = S + 1 + i;
-      if (h_stat[i] == kSkip) {
-        if (!deps_ok) { P = i; break; }
-        continue;
-      }
-      if (h_owner[i] != r) {  // seed taken during the round by walk h_owner[i] - S - 1 < i
-        const uint32_t o = h_owner[i] - S - 1;
-        if (h_owner[i] <= S || o >= i || late[o]) { P = i; break; }
-        late[i] = 1;
-        continue;
-      }
-      if (h_stat[i] == kDone && !h_lost[i] && deps_ok) continue;
-      P = i;
-      break;
-    }
-    // release: late skips of the prefix and every walk past it
-    bool any_rel = false;
-    for (uint32_t i = 0; i < n; i++) {
-      h_rel[i] = (i >= P && h_stat[i] != kSkip) || (i < P && late[i]) ? 1u : 0u;
-      any_rel = any_rel || h_rel[i];
-    }
-    if (any_rel) {
-      TK_HIP(hipMemcpyAsync(drel.p, h_rel, n * 4, hipMemcpyHostToDevice, c->stream));
-      IW_LAUNCH(c, "iworm_release", cdiv((uint64_t)n * 64, 256), 256, k_iw_release, n, S,
-                lmax, dpick.as<uint32_t>(), drel.as<uint32_t>(), dlens.as<uint32_t>(), dpslot.as<uint32_t>(),
-                dclaim.as<uint32_t>());
-    }
-    if (P == 0) {
-      // the first walk outgrew its path buffers: larger buffers, fewer walks
-      if (h_stat[0] != kOverflow) return fail(TK_ERR_STATE, "inchworm: first walk of a round did not commit");
-      if (lmax >= (1u << 28)) return fail(TK_ERR_STATE, "inchworm: walk longer than 2^28 k-mers");
+    std::fill(late.begin(), late.begin() + n, 0);
+    uint32_t m = n;         // walks of this round: all of the epoch, then h_walks[0 ... m)
+    uint32_t first = 0;     // the earliest of them: it saw only walks that hold
+    uint32_t P = n;         // committed walks
+    bool outgrown = false;  // walk P outgrew its path buffers
+    for (;;) {
+      res->rounds++;
+      res->walks += m;
+      wp.n = m;
+      IW_LAUNCH(c, "iworm_walk", cdiv((uint64_t)m * 4, 256), 256, k_iw_walk, wp,
+                m == n ? nullptr : dwalks.as<uint32_t>(), dpick.as<uint32_t>(), dclaim.as<uint32_t>(),
+                dlost.as<uint32_t>(), dstat.as<uint32_t>(), dlens.as<uint32_t>(), dsums.as<uint64_t>(),
+                dpslot.as<uint32_t>(), dpbase.as<uint8_t>(), ddeps.as<uint32_t>(), ddepn.as<uint32_t>());
+      IW_LAUNCH(c, "iworm_owner", cdiv(n, 256), 256, k_iw_owner, dpick.as<uint32_t>(), n, dclaim.as<uint32_t>(),
+                downer.as<uint32_t>());
+      TK_HIP(hipMemcpyAsync(h_depn, ddepn.p, n * 4, hipMemcpyDeviceToHost, c->stream));
+      TK_HIP(hipMemcpyAsync(h_deps, ddeps.p, (size_t)n * kDeps * 4, hipMemcpyDeviceToHost, c->stream));
+      TK_HIP(hipMemcpyAsync(h_owner, downer.p, n * 4, hipMemcpyDeviceToHost, c->stream));
+      TK_HIP(hipMemcpyAsync(h_stat, dstat.p, n * 4, hipMemcpyDeviceToHost, c->stream));
+      TK_HIP(hipMemcpyAsync(h_lost, dlost.p, n * 4, hipMemcpyDeviceToHost, c->stream));
+      TK_HIP(hipMemcpyAsync(h_lens, dlens.p, (size_t)n * 8, hipMemcpyDeviceToHost, c->stream));
+      TK_HIP(hipMemcpyAsync(h_sums, dsums.p, (size_t)n * 8, hipMemcpyDeviceToHost, c->stream));
       TK_HIP(hipStreamSynchronize(c->stream));
-      lmax *= 2;
-      Bcap = cap_for(lmax);
-      B = std::min(B, Bcap);
-      if ((rc = alloc_paths())) return rc;
-      S += n;
-      continue;
+      // Which walks hold, in rank order.  A walk whose seed an earlier walk
+      // took while it ran ("late") is the serial skip of that seed when the
+      // taker gives a contig; its own claims are void.  Any decision that
+      // treated a k-mer as used because an earlier walk held it (the
+      // dependencies), and a seed found claimed at the start, holds only if
+      // that walk gives a contig, i.e. is neither late nor skipped.  A walk
+      // with more dependencies than are recorded holds if no earlier walk
+      // changed since it started.
+      uint32_t n_bad = 0;
+      bool any_rel = false, full = false;  // full: the earliest walk that does not hold only lacked room
+      for (uint32_t i = 0; i < n; i++) {
+        const uint32_t r = S + 1 + i;
+        auto contig = [&](uint32_t d) { return d < i && state[d] == kContig; };
+        bool deps_ok = h_depn[i] <= kDeps || i <= first;  // those up to `first` have seen their last change
+        for (uint32_t j = 0; deps_ok && j < std::min(h_depn[i], kDeps); j++)
+          deps_ok = contig(h_deps[(size_t)i * kDeps + j]);
+        h_rel[i] = 0;
+        if (late[i]) {
+          late[i] = contig(late_by[i]);
+          state[i] = late[i] ? kSkipped : kBad;
+        } else if (h_stat[i] == kSkip) {
+          state[i] = deps_ok ? kSkipped : kBad;
+        } else if (h_owner[i] != r) {  // seed taken by walk h_owner[i] - S - 1 < i
+          late[i] = h_owner[i] > S && contig(h_owner[i] - S - 1);
+          late_by[i] = h_owner[i] - S - 1;
+          state[i] = late[i] ? kSkipped : kBad;
+          h_rel[i] = late[i];
+        } else {
+          state[i] = h_stat[i] == kDone && !h_lost[i] && deps_ok ? kContig : kBad;
+        }
+        if (state[i] == kBad) {
+          full = n_bad ? full : h_stat[i] == kOverflow && h_owner[i] == r && !h_lost[i] && deps_ok;
+          h_rel[i] = 1;
+          h_walks[n_bad++] = i;
+        }
+        any_rel = any_rel || h_rel[i];
+      }
+      if (n_bad && full) {
+        // the earliest walk still open outgrew its path buffers: those before
+        // it are committed, the rest is walked again with larger ones
+        P = h_walks[0];
+        outgrown = true;
+        for (uint32_t i = P; i < n; i++) h_rel[i] = 1;
+        any_rel = true;
+      } else if (n_bad && h_walks[0] <= first) {
+        return fail(TK_ERR_STATE, "inchworm: first walk of a round did not hold");
+      }
+      if (any_rel) {
+        TK_HIP(hipMemcpyAsync(drel.p, h_rel, n * 4, hipMemcpyHostToDevice, c->stream));
+        IW_LAUNCH(c, "iworm_release", cdiv((uint64_t)n * 64, 256), 256, k_iw_release, n, S,
+                  lmax, dpick.as<uint32_t>(), drel.as<uint32_t>(), dlens.as<uint32_t>(), dpslot.as<uint32_t>(),
+                  dclaim.as<uint32_t>());
+      }
+      if (!n_bad || outgrown) break;
+      m = n_bad;
+      first = h_walks[0];
+      TK_HIP(hipMemcpyAsync(dwalks.p, h_walks, (size_t)m * 4, hipMemcpyHostToDevice, c->stream));
+      IW_LAUNCH(c, "iworm_fill", cdiv(m, 256), 256, k_iw_reset, dwalks.as<uint32_t>(), m, dlost.as<uint32_t>(),
+                ddepn.as<uint32_t>());
     }
     // contigs of the committed walks, in rank order
     uint32_t nw = 0;
     uint64_t total = 0;
     for (uint32_t i = 0; i < P; i++) {
-      if (h_stat[i] != kDone || late[i]) continue;
+      if (state[i] != kContig) continue;
       h_walks[nw] = i;
       h_woff[nw] = total;
       const uint64_t L = (uint64_t)h_lens[2 * i] + h_lens[2 * i + 1] + k;
@@ -747,8 +772,16 @@ int inchworm_run(tk_ctx* c, tk_table* t, uint32_t min_seed_cov, const uint8_t* s
     }
     cursor = P < n ? h_pos[P] : h_out[1];
     S += n;
-    if (P == n) B = std::min(Bcap, B * 2);
-    else if (P < n / 8) B = std::max(Bmin, B / 2);
+    if (!outgrown) {
+      B = std::min(Bcap, B * 2);
+      continue;
+    }
+    if (lmax >= (1u << 28)) return fail(TK_ERR_STATE, "inchworm: walk longer than 2^28 k-mers");
+    TK_HIP(hipStreamSynchronize(c->stream));
+    lmax *= 2;
+    Bcap = cap_for(lmax);
+    B = std::min(B, Bcap);
+    if ((rc = alloc_paths())) return rc;
   }
   return TK_OK;
 }
