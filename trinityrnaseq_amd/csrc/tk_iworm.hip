@@ -9,9 +9,9 @@
 //
 //  * seeds: the table's keys with count >= min_seed_cov (and a seed-entropy
 //    composition table) sorted by key, then stably by inverted count;
-//  * epochs: the next B seeds still unused are walked at once, one four-lane
-//    group per walk (lane b looks up the candidate ending, or starting, with
-//    base b).  Walk w of epoch base S has rank S+1+w; a walk claims each
+//  * epochs: the next B seeds still unused are walked at once, sixteen
+//    lanes per walk (four look up the candidate ending, or starting, with a
+//    base).  Walk w of epoch base S has rank S+1+w; a walk claims each
 //    k-mer it takes with atomicMin(claim[slot], rank), so a k-mer goes to the
 //    earliest walk that wants it and a later walk that held it is marked lost.
 //    A walk treats k-mers claimed by earlier ranks (committed epochs, or
@@ -94,25 +94,33 @@ __device__ __forceinline__ uint64_t table_find(const TableView& t, uint64_t key,
   return 0;
 }
 
-// Exchanges among a walk's four lanes on DPP quad permutes (one VALU
-// instruction; a shuffle goes through LDS, about a tenth of a step's time).
+// Exchanges among a walk's sixteen lanes (a DPP row), by rotations of the row
+// (one VALU instruction each; a shuffle goes through LDS).
+template <int kRot>
+__device__ __forceinline__ uint32_t row_u32(uint32_t v) {
+  return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x120 + kRot, 0xF, 0xF, true);  // row_ror:kRot
+}
+constexpr int kQuadXor1 = 0xB1, kQuadXor2 = 0x4E;  // lanes 1032 and 2301 of four
 template <int kPerm>
 __device__ __forceinline__ uint32_t quad_u32(uint32_t v) {
   return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, kPerm, 0xF, 0xF, true);
 }
-template <int kPerm>
-__device__ __forceinline__ uint64_t quad_u64(uint64_t v) {
-  return ((uint64_t)quad_u32<kPerm>((uint32_t)(v >> 32)) << 32) | quad_u32<kPerm>((uint32_t)v);
+template <int kRot>
+__device__ __forceinline__ uint64_t row_u64(uint64_t v) {
+  return ((uint64_t)row_u32<kRot>((uint32_t)(v >> 32)) << 32) | row_u32<kRot>((uint32_t)v);
 }
-constexpr int kQuadXor1 = 0xB1, kQuadXor2 = 0x4E, kQuadLane0 = 0x00;  // lanes 1032, 2301, 0000
-__device__ __forceinline__ uint64_t quad_max_u64(uint64_t v) {
-  v = std::max(v, quad_u64<kQuadXor1>(v));
-  return std::max(v, quad_u64<kQuadXor2>(v));
+__device__ __forceinline__ uint64_t row_max_u64(uint64_t v) {
+  v = std::max(v, row_u64<8>(v));
+  v = std::max(v, row_u64<4>(v));
+  v = std::max(v, row_u64<2>(v));
+  return std::max(v, row_u64<1>(v));
 }
-// OR over the quad: a value that one lane holds and the others pass 0 for.
-__device__ __forceinline__ uint32_t quad_or_u32(uint32_t v) {
-  v |= quad_u32<kQuadXor1>(v);
-  return v | quad_u32<kQuadXor2>(v);
+// OR over the row: a value that one lane holds and the others pass 0 for.
+__device__ __forceinline__ uint32_t row_or_u32(uint32_t v) {
+  v |= row_u32<8>(v);
+  v |= row_u32<4>(v);
+  v |= row_u32<2>(v);
+  return v | row_u32<1>(v);
 }
 
 // Seed candidates: (key, slot) of every slot with count >= min_cov whose
@@ -274,74 +282,77 @@ struct WalkParams {
 
 constexpr uint32_t kDeps = 8;  // recorded dependencies per walk (more: walked again as a round's first)
 
-// Record that walk w treated a k-mer claimed by earlier walk `dep` of this
-// round as used (the decision holds only if that walk commits a contig).
+// Record that walk w treated a k-mer claimed by an earlier walk of this epoch
+// (claim cl, the same on all lanes of the walk) as used: the decision holds
+// only if that walk commits a contig.
 __device__ __forceinline__ void iw_dep(uint32_t* __restrict__ deps, uint32_t* __restrict__ dep_n, uint32_t w,
-                                       uint32_t dep, uint32_t& last) {
-  if (dep == last) return;
-  last = dep;
-  const uint32_t j = atomicAdd(&dep_n[w], 1u);
-  if (j < kDeps) deps[w * kDeps + j] = dep;
+                                       uint32_t S, uint32_t cl, uint32_t l16, uint32_t& last) {
+  if (cl <= S || cl >= S + 1 + w || cl == last) return;
+  last = cl;
+  if (l16) return;
+  const uint32_t j = dep_n[w];  // this lane alone counts them
+  dep_n[w] = j + 1;
+  if (j < kDeps) deps[w * kDeps + j] = cl - S - 1;
 }
 
-// A candidate's home bucket and the claims of its eight slots, loaded but not
-// yet looked at.
+// Two slots of a candidate's home bucket and their claims, loaded but not yet
+// looked at.
 struct CandLoad {
   uint64_t tagged, b;
-  ulonglong2 v[4];
-  uint4 q[2];
+  ulonglong2 v;
+  uint2 q;
 };
 
-__device__ __forceinline__ CandLoad iw_load(const WalkParams& p, const uint32_t* claim, uint64_t x,
-                                            int side, int b) {
-  const uint64_t y = side == 0 ? (((x << 2) | (uint64_t)b) & p.kmask)
-                               : (((uint64_t)b << (2 * (p.k - 1))) | (x >> 2));
+// The k-mer after x on a side (0 right, all ones left) by base b, without a
+// branch: a wait at its join would put the claim in flight before the loads.
+__device__ __forceinline__ uint64_t iw_extend(const WalkParams& p, uint64_t x, uint64_t side, uint32_t b) {
+  const uint64_t right = ((x << 2) | b) & p.kmask, left = ((uint64_t)b << (2 * (p.k - 1))) | (x >> 2);
+  return right ^ ((right ^ left) & side);
+}
+
+__device__ __forceinline__ CandLoad iw_load(const WalkParams& p, const uint32_t* claim, uint64_t y, uint32_t part) {
   const uint64_t key = canon_key(y, p.k, p.canonical);
   CandLoad d;
   d.tagged = key | p.t.occ;
   d.b = bucket0(p.t, key);
-  const ulonglong2* l2 = reinterpret_cast<const ulonglong2*>(p.t.slots + (d.b << 3));
-  const uint4* q4 = reinterpret_cast<const uint4*>(claim + (d.b << 3));
-#pragma unroll
-  for (int j = 0; j < 4; j++) d.v[j] = l2[j];
-  d.q[0] = q4[0];
-  d.q[1] = q4[1];
+  d.v = reinterpret_cast<const ulonglong2*>(p.t.slots + (d.b << 3))[part];
+  d.q = reinterpret_cast<const uint2*>(claim + (d.b << 3))[part];
   return d;
 }
 
-// Count (0 = absent or pruned), slot and claim (possibly out of date) of a loaded candidate.
-__device__ __forceinline__ uint64_t iw_resolve(const TableView& t, const uint32_t* claim,
-                                               const CandLoad& d, uint32_t& slot, uint32_t& cl) {
-  const uint64_t sv[8] = {d.v[0].x, d.v[0].y, d.v[1].x, d.v[1].y, d.v[2].x, d.v[2].y, d.v[3].x, d.v[3].y};
-  const uint32_t cv[8] = {d.q[0].x, d.q[0].y, d.q[0].z, d.q[0].w, d.q[1].x, d.q[1].y, d.q[1].z, d.q[1].w};
-  uint64_t hit = 0;
-  uint32_t at = 0;
-  cl = 0;
-#pragma unroll
-  for (int j = 0; j < 8; j++) {
-    const bool m = (sv[j] & t.kmo) == d.tagged;
-    hit = m ? sv[j] : hit;
-    at = m ? (uint32_t)j : at;
-    cl = m ? cv[j] : cl;
+// Count (0 = absent or pruned), slot and claim (possibly out of date) of a
+// loaded candidate, on the lane of its four that holds it; 0 on the others.
+__device__ __forceinline__ uint64_t iw_resolve(const TableView& t, const uint32_t* claim, const CandLoad& d,
+                                               uint32_t part, uint32_t& slot, uint32_t& cl) {
+  const bool m0 = (d.v.x & t.kmo) == d.tagged, m1 = (d.v.y & t.kmo) == d.tagged;
+  slot = (uint32_t)(d.b << 3) + 2 * part + (m0 ? 0u : 1u);
+  cl = m0 ? d.q.x : d.q.y;
+  // full home bucket without it: the probe goes on, on the lane of its last slots
+  const bool hit = m0 || m1;
+  uint32_t any = hit ? 1u : 0u;
+  any |= quad_u32<kQuadXor1>(any);
+  any |= quad_u32<kQuadXor2>(any);
+  uint64_t c = hit ? slot_count(t, m0 ? d.v.x : d.v.y) : 0;
+  if (!any && part == 3 && d.v.y != 0) {
+    c = table_find(t, d.tagged & (t.occ - 1), &slot);
+    if (c) cl = claim[slot];
   }
-  slot = (uint32_t)(d.b << 3) + at;
-  if (hit) return slot_count(t, hit);
-  if (sv[7] == 0) return 0;
-  const uint64_t c = table_find(t, d.tagged & (t.occ - 1), &slot);  // full home bucket: the probe goes on
-  if (c) cl = claim[slot];
   return c;
 }
 
-// One four-lane group per walk: claim the seed, extend right, then left, lane b
-// looking up the candidate with base b.  A walk is a chain of dependent steps
-// and a round lasts as long as its longest walk, so the step's latency is what
-// counts: a claim (a memory-side atomic) and a lookup.  The two run at once:
-// the lookups of the step after are issued with the claim of the best
-// candidate, as if it went through, and thrown away when it does not.  A
-// candidate's claim word is loaded with its bucket, and one that an earlier
-// rank is seen to hold is dropped without an atomic (claims only fall within a
-// round, so what an out-of-date word says is held, is).  Each group changes
-// side on its own.  120 k reads' dictionary: 3.98 -> 2.94 ms a round.
+// Sixteen lanes per walk, four to a candidate base, two slots of its bucket to
+// a lane: claim the seed, extend right, then left.  A walk is a chain of
+// dependent steps and a round lasts as long as its longest walk, so the step's
+// latency is what counts: a claim (a memory-side atomic), a lookup and the
+// instructions between.  Claim and lookup run at once: the lookups of the step
+// after are issued with the claim of the best candidate, as if it went
+// through, and thrown away when it does not.  A candidate's claim word is
+// loaded with its bucket, and one that an earlier rank is seen to hold is
+// dropped without an atomic (claims only fall within a round, so what an
+// out-of-date word says is held, is).  Each walk changes side on its own.
+// 120 k reads' dictionary, 27 k steps: 3.98 -> 2.94 ms a round with the two at
+// once, and 49.1 -> 43.8 ms in all from four lanes, each comparing the eight
+// slots of a candidate, to sixteen.
 __global__ __launch_bounds__(256) void k_iw_walk(WalkParams p, const uint32_t* __restrict__ list,
                                                  const uint32_t* __restrict__ picked_slot,
                                                  uint32_t* claim, uint32_t* __restrict__ lost,
@@ -349,10 +360,10 @@ __global__ __launch_bounds__(256) void k_iw_walk(WalkParams p, const uint32_t* _
                                                  uint64_t* __restrict__ sums, uint32_t* __restrict__ path_slot,
                                                  uint8_t* __restrict__ path_base, uint32_t* __restrict__ deps,
                                                  uint32_t* __restrict__ dep_n) {
-  const uint32_t g = (blockIdx.x * blockDim.x + threadIdx.x) >> 2;
-  if (g >= p.n) return;  // whole groups leave together
+  const uint32_t g = (blockIdx.x * blockDim.x + threadIdx.x) >> 4;
+  if (g >= p.n) return;  // whole rows leave together
   const uint32_t w = list ? list[g] : g;
-  const int b = threadIdx.x & 3;
+  const uint32_t l16 = threadIdx.x & 15, base = l16 >> 2, part = l16 & 3;
   const TableView& t = p.t;
   const uint32_t r = p.S + 1 + w;
   const uint32_t seed_slot = picked_slot[w];
@@ -360,51 +371,50 @@ __global__ __launch_bounds__(256) void k_iw_walk(WalkParams p, const uint32_t* _
   const uint64_t seed_key = seed_word & (t.occ - 1);
   uint64_t sum = slot_count(t, seed_word);
   uint32_t st = kRunning;
-  uint32_t last_dep = 0xFFFFFFFFu;
-  if (b == 0) {
-    const uint32_t old = atomicMin(&claim[seed_slot], r);
+  uint32_t last_dep = 0;
+  {
+    uint32_t old = 0;
+    if (l16 == 0) {
+      old = atomicMin(&claim[seed_slot], r);
+      if (old > r && old != kFree) atomicOr(&lost[old - p.S - 1], 1u);
+    }
+    old = row_or_u32(old);
     if (old < r) {
       st = kSkip;
-      if (old > p.S) iw_dep(deps, dep_n, w, old - p.S - 1, last_dep);
-    } else if (old != kFree && old != r) {
-      atomicOr(&lost[old - p.S - 1], 1u);
+      iw_dep(deps, dep_n, w, p.S, old, l16, last_dep);
     }
   }
-  st = quad_u32<kQuadLane0>(st);
   uint32_t nright = 0, len = 0;
-  int side = 0;
+  uint64_t side = 0;
   uint64_t x = seed_key;
   uint32_t* pslot = path_slot + (uint64_t)w * 2 * p.lmax;
   uint8_t* pbase = path_base + (uint64_t)w * 2 * p.lmax;
   if (st == kRunning) {
     uint32_t slot, cl;
-    uint64_t c = iw_resolve(t, claim, iw_load(p, claim, x, 0, b), slot, cl);
-    bool avail = c > 0;
+    uint64_t c = iw_resolve(t, claim, iw_load(p, claim, iw_extend(p, x, side, base), part), part, slot, cl);
     for (;;) {
-      // best remaining candidate of the group: count, then smallest base;
-      // candidates seen held by an earlier rank (or this walk) are dropped
+      // best remaining candidate: count, then smallest base; those seen held
+      // by an earlier rank (or this walk) are dropped (c = 0)
       uint64_t best = 0;
+      bool mine = false;
       for (;;) {
-        best = avail ? (((c < (1ull << 61) ? c : (1ull << 61)) << 2) | (uint64_t)(3 - b)) : 0;
-        best = quad_max_u64(best);
-        const bool mine = avail && (uint32_t)b == 3 - (uint32_t)(best & 3);
-        const bool held = mine && cl <= r;
-        if (held) {
-          avail = false;
-          if (cl > p.S && cl < r) iw_dep(deps, dep_n, w, cl - p.S - 1, last_dep);
-        }
-        if (!quad_or_u32(held ? 1u : 0u)) break;
+        const uint64_t my = c ? (((c < (1ull << 61) ? c : (1ull << 61)) << 2) | (3 - base)) : 0;
+        best = row_max_u64(my);
+        mine = my && my == best;
+        const uint32_t held = row_or_u32(mine && cl <= r ? cl : 0u);
+        if (!held) break;
+        if (mine) c = 0;
+        iw_dep(deps, dep_n, w, p.S, held, l16, last_dep);
       }
       if (best == 0) {  // this side ends here
-        if (side == 1) break;
+        if (side) break;
         nright = len;
-        side = 1;
+        side = ~0ull;
         len = 0;
         x = seed_key;
         pslot += p.lmax;
         pbase += p.lmax;
-        c = iw_resolve(t, claim, iw_load(p, claim, x, 1, b), slot, cl);
-        avail = c > 0;
+        c = iw_resolve(t, claim, iw_load(p, claim, iw_extend(p, x, side, base), part), part, slot, cl);
         continue;
       }
       if (len == p.lmax) {  // no room to record the claim: stop unclaimed
@@ -413,39 +423,37 @@ __global__ __launch_bounds__(256) void k_iw_walk(WalkParams p, const uint32_t* _
       }
       const uint32_t best_b = 3 - (uint32_t)(best & 3);
       uint32_t old = 0;
-      if ((uint32_t)b == best_b) old = atomicMin(&claim[slot], r);
-      // this walk's lost flag and the next step's lookups travel with the claim
+      if (mine) old = atomicMin(&claim[slot], r);
+      // this walk's lost flag, the record (which does not count unless the
+      // claim goes through) and the next step's lookups travel with the claim
       uint32_t l = 0;
-      if (b == 0) l = __hip_atomic_load(&lost[w], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      const uint64_t xn = side == 0 ? (((x << 2) | (uint64_t)best_b) & p.kmask)
-                                    : (((uint64_t)best_b << (2 * (p.k - 1))) | (x >> 2));
-      const CandLoad next = iw_load(p, claim, xn, side, b);
-      old = quad_or_u32(old);
-      if (old > r) {
-        if ((uint32_t)b == best_b) {
-          if (old != kFree) atomicOr(&lost[old - p.S - 1], 1u);
-          pslot[len] = slot;
-          pbase[len] = (uint8_t)best_b;
-        }
-        len++;
-        // the count field of a taken slot is exact up to 2^61 (clamped above)
-        sum += best >> 2;
-        x = xn;
-        l = quad_u32<kQuadLane0>(l);
-        if (l) {
-          st = kLost;
-          break;
-        }
-        c = iw_resolve(t, claim, next, slot, cl);
-        avail = c > 0;
-      } else if ((uint32_t)b == best_b) {  // held by an earlier rank (or this walk)
-        avail = false;
-        if (old > p.S && old < r) iw_dep(deps, dep_n, w, old - p.S - 1, last_dep);
+      if (l16 == 0) l = __hip_atomic_load(&lost[w], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      if (mine) {
+        pslot[len] = slot;
+        pbase[len] = (uint8_t)best_b;
       }
+      const uint64_t xn = iw_extend(p, x, side, best_b);
+      const CandLoad next = iw_load(p, claim, iw_extend(p, xn, side, base), part);
+      old = row_or_u32(old);
+      if (old <= r) {  // held by an earlier rank (or this walk)
+        if (mine) c = 0;
+        iw_dep(deps, dep_n, w, p.S, old, l16, last_dep);
+        continue;
+      }
+      if (mine && old != kFree) atomicOr(&lost[old - p.S - 1], 1u);
+      len++;
+      // the count field of a taken slot is exact up to 2^61 (clamped above)
+      sum += best >> 2;
+      x = xn;
+      if (row_or_u32(l)) {
+        st = kLost;
+        break;
+      }
+      c = iw_resolve(t, claim, next, part, slot, cl);
     }
     if (side == 0) nright = len, len = 0;
   }
-  if (b == 0) {
+  if (l16 == 0) {
     status[w] = st == kRunning ? kDone : st;
     lens[2 * w] = nright;
     lens[2 * w + 1] = len;
@@ -572,9 +580,10 @@ int inchworm_run(tk_ctx* c, tk_table* t, uint32_t min_seed_cov, const uint8_t* s
   // ---- rounds
   // TK_IWORM_WALKS caps the walks per epoch (default 16,384, starting at
   // 1,024) and TK_IWORM_LMAX sets the first path capacity per walk side
-  // (default 4,096 k-mers): small values force the conflict and regrowth
+  // (default 8,192 k-mers, 1.3 GB for a full epoch; 4,096 had 120 k reads' longest
+  // contigs walked twice, 4 of 57 ms): small values force the conflict and regrowth
   // paths on small inputs.
-  uint32_t Bmax = 16384, lmax = 4096;
+  uint32_t Bmax = 16384, lmax = 8192;
   if (const char* e = getenv("TK_IWORM_WALKS")) Bmax = (uint32_t)std::min<unsigned long>(std::max(1ul, strtoul(e, nullptr, 10)), 16384ul);
   if (const char* e = getenv("TK_IWORM_LMAX")) lmax = (uint32_t)std::min<unsigned long>(std::max(4ul, strtoul(e, nullptr, 10)), 1ul << 20);
   const uint32_t Bmin = std::min<uint32_t>(64, Bmax);
@@ -597,7 +606,10 @@ int inchworm_run(tk_ctx* c, tk_table* t, uint32_t min_seed_cov, const uint8_t* s
     if (!r2) r2 = dpbase.alloc((size_t)Bcap * 2 * lmax);
     return r2;
   };
-  if ((rc = alloc_paths())) return rc;
+  if (alloc_paths()) {  // no room for those: the smaller ones
+    lmax = std::min(lmax, 4096u);
+    if ((rc = alloc_paths())) return rc;
+  }
   // the per-round host copies live in page-locked memory, so each is one DMA
   // (copies to pageable memory are staged and wait on the host)
   struct Pinned {
@@ -660,7 +672,7 @@ int inchworm_run(tk_ctx* c, tk_table* t, uint32_t min_seed_cov, const uint8_t* s
       res->rounds++;
       res->walks += m;
       wp.n = m;
-      IW_LAUNCH(c, "iworm_walk", cdiv((uint64_t)m * 4, 256), 256, k_iw_walk, wp,
+      IW_LAUNCH(c, "iworm_walk", cdiv((uint64_t)m * 16, 256), 256, k_iw_walk, wp,
                 m == n ? nullptr : dwalks.as<uint32_t>(), dpick.as<uint32_t>(), dclaim.as<uint32_t>(),
                 dlost.as<uint32_t>(), dstat.as<uint32_t>(), dlens.as<uint32_t>(), dsums.as<uint64_t>(),
                 dpslot.as<uint32_t>(), dpbase.as<uint8_t>(), ddeps.as<uint32_t>(), ddepn.as<uint32_t>());
