@@ -43,7 +43,6 @@ constexpr uint32_t kCompCtInLds = 1;
 // windows and more) are few and take the memory-side atomics.
 constexpr uint64_t kCtLdsRegions = 256;
 constexpr int kCtLdsThreads = 1024;
-constexpr uint32_t kCtQueue = 128;  // entries of a wave's queue
 constexpr int kCtSplitSteps = 8;    // two words a step and wave
 constexpr uint32_t kCtSplitWords = 2 * kCtSplitSteps * (kCtLdsThreads / 64);  // words of a workgroup
 
@@ -390,14 +389,13 @@ __global__ __launch_bounds__(kCtLdsThreads) void k_batch_ctable_split(ReadsView 
 // region's workgroup going over all contigs of its component).
 // The region's keys come from its own memory, where k_batch_ctable_split left
 // them, or, for a table of one region or a region that was sent more than it
-// holds, from the contigs: each wave takes a run of their words, and the
-// region's keys queue up in LDS, so that 64 lanes insert at a time.
+// holds, from the contigs, each wave taking a run of their words.
 template <bool kPacked>
 __global__ __launch_bounds__(kCtLdsThreads) void k_batch_ctable_lds(ReadsView cv, const CtPiece* __restrict__ pieces,
                                                           const uint64_t* __restrict__ contig_off,
                                                           const CompLayout* __restrict__ lay, int k, int canonical,
                                                           uint64_t* __restrict__ ct, const uint32_t* __restrict__ cnt,
-                                                          uint32_t lds_words, uint32_t* __restrict__ flags) {
+                                                          uint32_t* __restrict__ flags) {
   extern __shared__ uint64_t s_ct[];
   const CtPiece pc = pieces[blockIdx.x];
   const CompLayout L = lay[pc.comp];
@@ -409,7 +407,8 @@ __global__ __launch_bounds__(kCtLdsThreads) void k_batch_ctable_lds(ReadsView cv
   const int lane = threadIdx.x & 63;
   const uint32_t n = cnt[blockIdx.x];
   uint32_t dummy = 0;
-  for (uint32_t i = threadIdx.x; i < words; i += blockDim.x) s_ct[i] = 0;
+  ulonglong2* s2 = reinterpret_cast<ulonglong2*>(s_ct);
+  for (uint32_t i = threadIdx.x; i < words / 2; i += blockDim.x) s2[i] = make_ulonglong2(0, 0);
   __syncthreads();
   // slots of the region's first bucket: the insert adds the bucket's number in the table
   auto insert = [&](uint64_t e, uint32_t local) {
@@ -421,9 +420,6 @@ __global__ __launch_bounds__(kCtLdsThreads) void k_batch_ctable_lds(ReadsView cv
       insert(kPacked ? g[i] : g[2 * i], kPacked ? 0 : (uint32_t)g[2 * i + 1]);
   } else {
     const uint32_t wv = threadIdx.x >> 6, nwv = blockDim.x >> 6;
-    uint64_t* q = s_ct + lds_words + wv * kCtQueue;
-    uint32_t* qc = reinterpret_cast<uint32_t*>(s_ct + lds_words + nwv * kCtQueue) + wv * kCtQueue;
-    uint32_t qn = 0;
     const uint64_t c0 = contig_off[pc.comp], c1 = contig_off[pc.comp + 1];
     const uint64_t wfirst = cv.word_off[c0], wlast = cv.word_off[c1];
     const uint64_t per = ((wlast - wfirst + nwv - 1) / nwv + 1) & ~1ull;
@@ -432,36 +428,13 @@ __global__ __launch_bounds__(kCtLdsThreads) void k_batch_ctable_lds(ReadsView cv
     if (w0 < wend) cw.start(cv, c0, c1, w0, lane);
     for (uint64_t at = w0; at < wend; at += 2) {
       uint64_t key, r;
-      bool mine = cw.next(cv, wend, lane, k, canonical, key, r);
-      mine = mine && (mix64(key) & L.ct_mask & ~rmask) == b0;
-      const uint64_t m = __ballot(mine);
-      if (mine) {
-        const uint32_t i = qn + __popcll(m & ((1ull << lane) - 1));
-        const uint32_t local = (uint32_t)(r - c0);
-        q[i] = kPacked ? ((vmax - local) << (2 * k + 1)) | occ | key : key;
-        if (!kPacked) qc[i] = local;
-      }
-      qn += (uint32_t)__popcll(m);
-      wave_sync();
-      if (qn >= 64) {
-        insert(q[lane], kPacked ? 0 : qc[lane]);
-        qn -= 64;
-        wave_sync();
-        if ((uint32_t)lane < qn) {
-          q[lane] = q[64 + lane];
-          if (!kPacked) qc[lane] = qc[64 + lane];
-        }
-        wave_sync();
-      }
+      if (!cw.next(cv, wend, lane, k, canonical, key, r) || (mix64(key) & L.ct_mask & ~rmask) != b0) continue;
+      const uint32_t local = (uint32_t)(r - c0);
+      insert(kPacked ? ((vmax - local) << (2 * k + 1)) | occ | key : key, local);
     }
-    if ((uint32_t)lane < qn) insert(q[lane], kPacked ? 0 : qc[lane]);
   }
   __syncthreads();
-  for (uint32_t i = threadIdx.x; i < words; i += blockDim.x) g[i] = s_ct[i];
-}
-
-static constexpr size_t ct_lds_bytes(bool packed, uint64_t buckets) {
-  return buckets * 64 + (size_t)(kCtLdsThreads / 64) * kCtQueue * (packed ? 8 : 12);
+  for (uint32_t i = threadIdx.x; i < words / 2; i += blockDim.x) reinterpret_cast<ulonglong2*>(g)[i] = s2[i];
 }
 
 template <bool kPacked>
@@ -559,10 +532,10 @@ static bool ct_lds_ok() {
   static const bool ok = [] {
     const bool r = hipFuncSetAttribute(reinterpret_cast<const void*>(&k_batch_ctable_lds<true>),
                                        hipFuncAttributeMaxDynamicSharedMemorySize,
-                                       (int)ct_lds_bytes(true, kCtRegion)) == hipSuccess &&
+                                       (int)kCtRegion * 64) == hipSuccess &&
                    hipFuncSetAttribute(reinterpret_cast<const void*>(&k_batch_ctable_lds<false>),
                                        hipFuncAttributeMaxDynamicSharedMemorySize,
-                                       (int)ct_lds_bytes(false, kCtRegion)) == hipSuccess;
+                                       (int)kCtRegion * 64) == hipSuccess;
     (void)hipGetLastError();
     return r;
   }();
@@ -710,8 +683,7 @@ static int batch_enqueue(tk_ctx* c, tk_batch* b, const tk_stats_opts* o, tk_read
       hipLaunchKernelGGL(k_fill_zero, dim3(grid(b->n_ct_clear, 256)), dim3(256), 0, c->stream, b->d_ct, b->n_ct_clear);
     const ReadsView cv = rview(b->contigs);
     const size_t vlds = ((size_t)slab * 4 + 8 * kLookupScratch) * wpb;
-    const size_t clds = ct_lds_bytes(b->ct_packed, b->ct_lds_buckets);
-    const uint32_t cwords = (uint32_t)(b->ct_lds_buckets * 8);
+    const size_t clds = b->ct_lds_buckets * 64;
     if (b->n_ct_split) {
       hipLaunchKernelGGL(k_fill_zero32, dim3(grid(b->n_ct_lds, 256)), dim3(256), 0, c->stream, b->d_ct_cnt,
                          (uint32_t)b->n_ct_lds);
@@ -726,12 +698,10 @@ static int batch_enqueue(tk_ctx* c, tk_batch* b, const tk_stats_opts* o, tk_read
     }
     if (b->n_ct_lds && b->ct_packed)
       hipLaunchKernelGGL(k_batch_ctable_lds<true>, dim3((unsigned)b->n_ct_lds), dim3(kCtLdsThreads), clds, c->stream,
-                         cv, b->d_ct_lds, b->d_contig_off, b->d_lay, b->k, b->canonical, b->d_ct, b->d_ct_cnt, cwords,
-                         c->d_flags);
+                         cv, b->d_ct_lds, b->d_contig_off, b->d_lay, b->k, b->canonical, b->d_ct, b->d_ct_cnt, c->d_flags);
     else if (b->n_ct_lds)
       hipLaunchKernelGGL(k_batch_ctable_lds<false>, dim3((unsigned)b->n_ct_lds), dim3(kCtLdsThreads), clds, c->stream,
-                         cv, b->d_ct_lds, b->d_contig_off, b->d_lay, b->k, b->canonical, b->d_ct, b->d_ct_cnt, cwords,
-                         c->d_flags);
+                         cv, b->d_ct_lds, b->d_contig_off, b->d_lay, b->k, b->canonical, b->d_ct, b->d_ct_cnt, c->d_flags);
     if (b->ct_packed) {
       if (cv.n_reads)
         hipLaunchKernelGGL(k_batch_ctable<true>, dim3(grid(cv.n_reads, 4)), dim3(256), 0, c->stream, cv,
