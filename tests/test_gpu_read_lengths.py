@@ -133,3 +133,31 @@ def test_small_sets_spread(api, ctx, k, n):
     assert np.array_equal(ct.vote(reads), want.astype(api.R2T_VOTE_DTYPE))
     for o in (ct, t, reads):
         o.free()
+
+
+@pytest.mark.parametrize("n", [0, 1, 2, 16384, 16385])
+def test_uploaded_and_device_reads_agree(api, ctx, n):
+    """Sizes and windows of a read set, taken on the host up to 16,384 reads of
+    an upload and on the device otherwise, with empty reads and reads below k."""
+    print("uploaded_and_device_reads", n, flush=True)
+    rng = np.random.default_rng(n)
+    lens = rng.choice([0, 1, 24, 25, 26, 31, 32, 33, 64, 90], size=n)
+    off = np.concatenate([[0], np.cumsum(lens)]).astype(np.uint64)
+    seq = rng.choice(np.frombuffer(b"ACGTN", np.uint8), p=[.24, .24, .24, .24, .04], size=int(off[-1])).tobytes()
+    up = api.Reads(ctx, seq, off)
+    d_seq, d_off = api.DeviceBuffer(ctx, max(1, len(seq))), api.DeviceBuffer(ctx, off.nbytes)
+    if seq:
+        d_seq.upload(np.frombuffer(seq, np.uint8))
+    d_off.upload(off)
+    dev = api.Reads.from_device(ctx, d_seq.ptr, d_off.ptr, n)
+    keys, counts = O.count(seq, off, 25, True)
+    for r in (up, dev):
+        assert tuple(r.info()) == (n, int(off[-1]), int(lens.max()) if n else 0)
+        for k in (1, 25, 31):
+            assert r.windows(k) == int(np.maximum(lens - k + 1, 0).sum())
+        t = api.Table(ctx, 25, True, 1 << 12)
+        t.count(r)
+        gk, gc = t.dump()
+        assert np.array_equal(gk, keys) and np.array_equal(gc, counts)
+        t.free()
+        r.free()

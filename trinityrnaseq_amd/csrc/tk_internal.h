@@ -77,6 +77,7 @@ struct tk_reads {
   uint64_t* d_codes = nullptr;     // n_words + kWordPad
   uint32_t* d_nmask = nullptr;     // n_words + kWordPad
   std::map<int, uint64_t> windows; // k -> total windows
+  std::vector<uint32_t> h_len;     // lengths of a small set uploaded from the host (kHostLens reads at most)
   std::map<int, double> est;       // 2k + canonical -> distinct estimate of all reads
   uint32_t* d_order = nullptr;     // locality order of the table passes (n_reads)
   bool order_done = false;         // d_order built, or found not worth building

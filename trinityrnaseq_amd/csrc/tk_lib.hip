@@ -303,7 +303,7 @@ __global__ __launch_bounds__(256) void k_read_words(const uint64_t* __restrict__
   __syncthreads();
   if (threadIdx.x == 0) {
     for (int i = 1; i < (int)(blockDim.x >> 6); i++) m = s_max[i] > m ? s_max[i] : m;
-    if (m) atomicMax(maxlen, m);
+    if (m && maxlen) atomicMax(maxlen, m);
   }
 }
 
@@ -369,6 +369,10 @@ __global__ __launch_bounds__(256) void k_pack(const char* __restrict__ seq,
                                               uint64_t* __restrict__ codes,
                                               uint32_t* __restrict__ nmask) {
   __shared__ uint64_t s_woff[kPackReadsLds + 1];
+  if (blockIdx.x == 0 && threadIdx.x < kWordPad) {
+    codes[n_words + threadIdx.x] = 0;
+    nmask[n_words + threadIdx.x] = ~0u;
+  }
   const uint64_t w0 = (uint64_t)blockIdx.x * blockDim.x;
   if (w0 >= n_words) return;
   const uint64_t wl = std::min<uint64_t>(w0 + blockDim.x, n_words) - 1;
@@ -430,8 +434,21 @@ __global__ void k_windows(const uint32_t* __restrict__ len, uint64_t n, int k,
   block_sum_add(s, total);
 }
 
+// What a caller that has the offsets on the host knows of a read set: then the
+// upload waits for the device once, at its end (200 reads and their contigs,
+// counted, scored and assigned: 422 -> 327 us with the lengths below).
+struct HostSizes {
+  uint64_t words = 0;
+  uint32_t max_len = 0;
+};
+
+// Reads up to this many keep their lengths on the host too: their windows are
+// then counted there (16,384: 10 us) instead of in a pass with a round trip (25).
+constexpr uint64_t kHostLens = 16384;
+
+// known: the sizes (nullptr: computed here, with a wait).
 static int reads_build(tk_ctx* ctx, const char* d_seq, const uint64_t* d_off, uint64_t n,
-                       uint64_t n_bases, tk_reads** out) {
+                       uint64_t n_bases, const HostSizes* known, tk_reads** out) {
   tk_reads* r = new tk_reads();
   r->device = ctx->device;
   r->n_reads = n;
@@ -443,31 +460,34 @@ static int reads_build(tk_ctx* ctx, const char* d_seq, const uint64_t* d_off, ui
     if ((rc = dev_alloc((void**)&r->d_len, std::max<uint64_t>(n, 1) * 4))) break;
     if ((rc = dev_alloc((void**)&r->d_word_off, nwb))) break;
     if ((rc = dev_alloc((void**)&d_nw, nwb))) break;
-    hipError_t e = hipMemsetAsync(ctx->d_flags, 0, 64 * 4, ctx->stream);
+    hipError_t e = known ? hipSuccess : hipMemsetAsync(ctx->d_flags, 0, 64 * 4, ctx->stream);
     if (e != hipSuccess) { rc = hip_fail(e, "memset flags"); break; }
     {
       uint64_t grid = std::min<uint64_t>(ceil_div(n + 1, 256), (uint64_t)std::max(ctx->num_cu, 1) * 4);
       hipEvent_t a;
       timing_begin(ctx, &a);
       hipLaunchKernelGGL(k_read_words, dim3(grid), dim3(256), 0, ctx->stream, d_off, n,
-                         r->d_len, d_nw, ctx->d_flags);
+                         r->d_len, d_nw, known ? nullptr : ctx->d_flags);
       timing_end(ctx, "read_words", a);
       if ((e = hipGetLastError()) != hipSuccess) { rc = hip_fail(e, "k_read_words"); break; }
     }
     if ((rc = exclusive_scan_u64(ctx, d_nw, r->d_word_off, n + 1))) break;
-    uint64_t nwords = 0;
-    e = hipMemcpyAsync(&nwords, r->d_word_off + n, 8, hipMemcpyDeviceToHost, ctx->stream);
-    if (e == hipSuccess) e = hipMemcpyAsync(ctx->h_flags, ctx->d_flags, 64 * 4, hipMemcpyDeviceToHost, ctx->stream);
-    if (e == hipSuccess) e = hipStreamSynchronize(ctx->stream);
-    if (e != hipSuccess) { rc = hip_fail(e, "read words"); break; }
-    r->max_len = ctx->h_flags[0];
+    uint64_t nwords = known ? known->words : 0;
+    if (!known) {
+      e = hipMemcpyAsync(&nwords, r->d_word_off + n, 8, hipMemcpyDeviceToHost, ctx->stream);
+      if (e == hipSuccess) e = hipMemcpyAsync(ctx->h_flags, ctx->d_flags, 64 * 4, hipMemcpyDeviceToHost, ctx->stream);
+      if (e == hipSuccess) e = hipStreamSynchronize(ctx->stream);
+      if (e != hipSuccess) { rc = hip_fail(e, "read words"); break; }
+    }
+    r->max_len = known ? known->max_len : ctx->h_flags[0];
     r->n_words = nwords;
     if ((rc = dev_alloc((void**)&r->d_codes, (nwords + kWordPad) * 8))) break;
     if ((rc = dev_alloc((void**)&r->d_nmask, (nwords + kWordPad) * 4))) break;
-    e = hipMemsetAsync(r->d_codes + nwords, 0, kWordPad * 8, ctx->stream);
-    if (e == hipSuccess) e = hipMemsetAsync(r->d_nmask + nwords, 0xFF, kWordPad * 4, ctx->stream);
-    if (e != hipSuccess) { rc = hip_fail(e, "pad"); break; }
-    if (nwords) {
+    if (!nwords) {  // k_pack writes the padding otherwise
+      e = hipMemsetAsync(r->d_codes, 0, kWordPad * 8, ctx->stream);
+      if (e == hipSuccess) e = hipMemsetAsync(r->d_nmask, 0xFF, kWordPad * 4, ctx->stream);
+      if (e != hipSuccess) { rc = hip_fail(e, "pad"); break; }
+    } else {
       const uint64_t nblk = ceil_div(nwords, 256);
       void* bp = nullptr;
       if ((rc = ensure_scratch(ctx, 1, nblk * 8, &bp))) break;
@@ -485,6 +505,7 @@ static int reads_build(tk_ctx* ctx, const char* d_seq, const uint64_t* d_off, ui
     e = hipStreamSynchronize(ctx->stream);
     if (e != hipSuccess) { rc = hip_fail(e, "pack sync"); break; }
   } while (0);
+  if (rc) (void)hipStreamSynchronize(ctx->stream);
   dev_free(d_nw, nwb);
   r->bytes = std::max<uint64_t>(n, 1) * 4 + nwb + (r->n_words + kWordPad) * 12;
   if (rc) {
@@ -582,6 +603,12 @@ static int reads_windows(tk_ctx* ctx, const tk_reads* rc_, int k, uint64_t* tota
   tk_reads* r = const_cast<tk_reads*>(rc_);
   auto it = r->windows.find(k);
   if (it != r->windows.end()) { *total = it->second; return TK_OK; }
+  if (!r->h_len.empty() || !r->n_reads) {
+    uint64_t h = 0;
+    for (uint32_t l : r->h_len) h += l >= (uint32_t)k ? l - k + 1 : 0;
+    *total = r->windows[k] = h;
+    return TK_OK;
+  }
   unsigned long long* d = reinterpret_cast<unsigned long long*>(ctx->d_flags + 8);
   TK_HIP(hipMemsetAsync(d, 0, 8, ctx->stream));
   if (r->n_reads) {
@@ -2224,8 +2251,17 @@ int tk_reads_from_host(tk_ctx* c, const char* seq, const uint64_t* offsets, uint
     return fail(TK_ERR_ARG, "NULL argument");
   *out = nullptr;
   if (offsets[0] != 0) return fail(TK_ERR_ARG, "offsets[0] must be 0");
-  for (uint64_t i = 0; i < n; i++)
+  HostSizes hs;
+  std::vector<uint32_t> lens;
+  if (n <= kHostLens) lens.resize(n);
+  for (uint64_t i = 0; i < n; i++) {
     if (offsets[i + 1] < offsets[i]) return fail(TK_ERR_ARG, "offsets not monotone at %llu", (unsigned long long)i);
+    const uint64_t l = offsets[i + 1] - offsets[i];
+    const uint32_t l32 = (uint32_t)std::min<uint64_t>(l, 0xFFFFFFFFull);  // as k_read_words
+    hs.words += (l + 31) / 32;
+    hs.max_len = std::max(hs.max_len, l32);
+    if (!lens.empty()) lens[i] = l32;
+  }
   if (set_device(c->device)) return TK_ERR_HIP;
   const uint64_t nb = offsets[n];
   char* d_seq = nullptr;
@@ -2236,8 +2272,9 @@ int tk_reads_from_host(tk_ctx* c, const char* seq, const uint64_t* offsets, uint
   if (rc) { dev_free(d_seq, nb + 64); return rc; }
   rc = upload_h2d(c, d_seq, seq, nb);
   if (!rc) rc = upload_h2d(c, d_off, offsets, (n + 1) * 8);
-  if (!rc) rc = reads_build(c, d_seq, d_off, n, nb, out);
-  (void)hipStreamSynchronize(c->stream);
+  if (!rc) rc = reads_build(c, d_seq, d_off, n, nb, &hs, out);
+  if (rc) (void)hipStreamSynchronize(c->stream);
+  else (*out)->h_len = std::move(lens);
   dev_free(d_seq, nb + 64);
   dev_free(d_off, (n + 1) * 8);
   return rc;
@@ -2251,7 +2288,7 @@ int tk_reads_from_device_d(tk_ctx* c, const char* d_seq, const uint64_t* d_offse
   uint64_t nb = 0;
   TK_HIP(hipMemcpyAsync(&nb, d_offsets + n, 8, hipMemcpyDeviceToHost, c->stream));
   TK_HIP(hipStreamSynchronize(c->stream));
-  return reads_build(c, d_seq, d_offsets, n, nb, out);
+  return reads_build(c, d_seq, d_offsets, n, nb, nullptr, out);
 }
 
 int tk_reads_info(const tk_reads* r, uint64_t* n_reads, uint64_t* n_bases, uint32_t* max_len) {
