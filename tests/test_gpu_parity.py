@@ -231,6 +231,72 @@ def test_count_resident_merge_windows_per_round(api, ctx, wpr, monkeypatch):
     assert np.array_equal(gk, ok) and np.array_equal(gc, oc)
 
 
+@pytest.mark.parametrize("n_reads,expected,prefill,resident", [
+    (66576, 1 << 22, False, False),   # one read short of 2^23 windows
+    (66577, 1 << 22, False, True),
+    (66577, 1 << 22, True, True),     # onto keys, one slot per window
+    (66577, 12_000_000, True, True),  # 2.9 slots per window
+    (66577, 13_000_000, True, False),  # 3.1
+    (66577, 13_000_000, False, True),  # the same size, empty: written once either way
+])
+def test_count_chooses_regions_by_cost(api, ctx, n_reads, expected, prefill, resident, monkeypatch):
+    """The default choice of the region-resident passes: from 2^23 windows on,
+    and, for a table that holds keys already, up to three slots per window (the
+    passes read and write such a table again wherever a word falls).  Either
+    way the counts are the oracle's."""
+    say("count_choice", n_reads, expected, prefill)
+    from trinityrnaseq_amd import synth
+    monkeypatch.delenv("TK_RESIDENT", raising=False)
+    tx = synth.large_transcriptome(1003, 2000)
+    seq, off = synth.se_reads(tx, n_reads, 150, seed=21)
+    seq = seq.tobytes()
+    r = api.Reads(ctx, seq, off)
+    assert (r.windows(25) >= 1 << 23) == (n_reads == 66577)
+    t = api.Table(ctx, 25, True, expected, 0.5)
+    if prefill:
+        small = api.Reads(ctx, seq[:int(off[500])], off[:501])
+        t.count(small)
+        assert ctx.count_words() == 0
+        small.free()
+    t.count(r)
+    assert (ctx.count_words() > 0) == resident
+    ok, oc = O.count(seq, off, 25, True)
+    if prefill:
+        sk, sc = O.count(seq[:int(off[500])], off[:501], 25, True)
+        oc[np.searchsorted(ok, sk)] += sc
+    gk, gc = t.dump()
+    assert np.array_equal(gk, ok) and np.array_equal(gc, oc)
+    t.free()
+    r.free()
+
+
+def test_count_in_chunks_goes_on_with_atomics(api, ctx, monkeypatch):
+    """A chunked count whose later chunks have fewer windows than a third of
+    the table's slots: the first chunk writes the new table's regions, the
+    rest is added with table atomics from the first read not yet counted."""
+    say("count_chunks_then_atomics")
+    from trinityrnaseq_amd import synth
+    monkeypatch.delenv("TK_RESIDENT", raising=False)
+    monkeypatch.setenv("TK_RES_CHUNK_READS", "20000")
+    tx = synth.large_transcriptome(1003, 2000)
+    seq, off = synth.se_reads(tx, 70000, 150, seed=22)
+    seq = seq.tobytes()
+    r = api.Reads(ctx, seq, off)
+    t = api.Table(ctx, 25, True, 1 << 23, 0.5)  # 16.8 M slots, 2.5 M windows a chunk
+    ctx.timing(True)
+    ctx.timing_reset()
+    t.count(r)
+    ctx.sync()
+    launches = {n: ctx.kernel_time(n)[1] for n in ("count_regions", "count")}
+    ctx.timing(False)
+    assert launches == {"count_regions": 1, "count": 1}
+    ok, oc = O.count(seq, off, 25, True)
+    gk, gc = t.dump()
+    assert np.array_equal(gk, ok) and np.array_equal(gc, oc)
+    t.free()
+    r.free()
+
+
 @pytest.mark.parametrize("resident", ["1", "0"])
 def test_count_reused_blocks(api, ctx, resident, monkeypatch):
     """With the thread's block reuse on, each table takes the block of the

@@ -2603,15 +2603,40 @@ constexpr int kResSlots = 3840;
 // Whether a count of `windows` windows takes the region-resident passes
 // (reads in the locality order, k <= 25, tables of 64 KB regions): from 2^23
 // windows on.  TK_RESIDENT=0 never, TK_RESIDENT=1 always (when the streams fit).
-// With table atomics / resident, count alone: 4.2 M windows 317 / 392 us, 6.2 M
-// 427 / 426, 10.1 M 647 / 497, 75.6 M 3.33 / 2.23 ms, 756 M 20.5 / 14.3 ms,
-// 2.0 G 46.5 / 33.1 ms.
+// With table atomics / resident, count alone into a table made for it: 4.2 M
+// windows 317 / 392 us, 6.2 M 427 / 426, 10.1 M 647 / 497, 75.6 M 3.33 / 2.23 ms,
+// 756 M 20.5 / 14.3 ms, 2.0 G 46.5 / 33.1 ms.  Fewer distinct keys favour the
+// regions however few they are (the atomics then queue on hot addresses): 75 M
+// windows of a 30 kb sequence, 18 regions, 28.5 / 0.50 ms; all 5-mers, two
+// regions, 310 / 3.6 ms.
 constexpr uint64_t kResMinWindows = 1ull << 23;
+static bool resident_forced() {
+  const char* e = getenv("TK_RESIDENT");
+  return e && e[0] == '1';
+}
 static bool resident_enabled(uint64_t windows) {
   const char* e = getenv("TK_RESIDENT");
   if (e && e[0] == '0') return false;
-  if (e && e[0] == '1') return true;
-  return windows >= kResMinWindows;
+  return resident_forced() || windows >= kResMinWindows;
+}
+
+// Whether region passes over `windows` windows of r (a whole count, or one of
+// its read chunks) cost less than table atomics on the table as it is.  A table
+// that holds keys is read and written again where words fall, 0.57 ms per GB of
+// regions, while the atomics do not care for its size: 10.1 M windows added to
+// 0.25 / 1 / 16 GB take 0.60 / 0.57 / 0.61 ms with atomics and 0.53 / 0.95 /
+// 9.59 with regions, 756 M windows added to 8 / 16 / 64 GB 19.9 / 20.0 / 20.1 and
+// 16.0 / 20.2 / 50.3.  The two cost the same at 4.4 slots per window for 10 M
+// windows, 4.1 for 30 M, 4.0 for 76 M, 3.1 for 252 M and 2.8 for 756 M.
+constexpr uint64_t kResSlotsPerWindow = 3;
+static bool resident_pays(const tk_table* t, const tk_reads* r, uint64_t windows) {
+  if (!t->n_keys) return true;  // an empty table is written once either way
+  // regions that can get a word: no more than the reads have distinct keys
+  double keys = (double)windows;
+  const auto it = r->est.find(2 * t->k + t->canonical);
+  if (it != r->est.end()) keys = std::min(keys, 1.05 * it->second);
+  const double regions = std::min((double)(t->nb >> t->rbits), keys);
+  return regions * (double)(8ull << t->rbits) <= (double)kResSlotsPerWindow * (double)windows;
 }
 
 // Most words in each stream of a count below kResLargeWindows windows: their
@@ -2759,10 +2784,13 @@ constexpr int kNotResident = -1000;
 
 // Count reads [rb, re) of the locality order through the region-resident
 // passes: merge + emit, coarse sort, fine sort, per-region LDS count, in one
-// pass whose streams hold every word the merge can emit (resident_plan);
-// kNotResident, with the table unchanged, when they do not fit.
+// pass whose streams hold every word the merge can emit (resident_plan), or in
+// read chunks.  kNotResident: the table holds reads [rb, *done) and table
+// atomics are to count the rest (the streams do not fit, or the table is too
+// large for a chunk's region passes to pay).
 static int count_resident(tk_ctx* c, tk_table* t, const tk_reads* r, const ReadsView& rview, uint64_t rb,
-                          uint64_t re, uint64_t windows, uint32_t max_nwin) {
+                          uint64_t re, uint64_t windows, uint64_t* done) {
+  *done = rb;
   int rc = TK_OK;
   // the table's final regions must be known before words are grouped by them
   if ((double)(t->n_keys + windows) > 0.9 * (double)(t->nb * 8)) {
@@ -2817,6 +2845,11 @@ static int count_resident(tk_ctx* c, tk_table* t, const tk_reads* r, const Reads
     // chunk's region pass writes every region, so a chunk that fits its
     // stream costs no clearing pass.
   }
+  const bool forced = resident_forced();
+  auto pays = [&](uint64_t n_reads) {
+    return forced || resident_pays(t, r, (uint64_t)((double)n_reads * win_per_read));
+  };
+  if (!pays(chunk)) return kNotResident;
   void *pa = nullptr, *pb = nullptr;
   if ((rc = ensure_scratch(c, kSlotResA, cap * 8, &pa))) return rc;
   if ((rc = ensure_scratch(c, kSlotResB, cap * 8, &pb))) return rc;
@@ -2825,6 +2858,8 @@ static int count_resident(tk_ctx* c, tk_table* t, const tk_reads* r, const Reads
   unsigned long long* cursor = reinterpret_cast<unsigned long long*>(c->d_flags + 8);
   for (uint64_t q = rb, qe = rb; q < re; q = qe) {
     qe = std::min<uint64_t>(re, q + chunk);
+    *done = q;
+    if (q > rb && !pays(qe - q)) return kNotResident;
     const uint64_t keys_before = t->n_keys;
     TableView v = table_view(t);
     TK_HIP(hipMemsetAsync(c->d_flags, 0, 64, c->stream));
@@ -2971,14 +3006,13 @@ int tk_count(tk_ctx* c, tk_table* t, const tk_reads* r) {
   } else {
     rview.order = nullptr;
   }
+  uint64_t rb = 0;
   if (rview.order && 63 - 2 * t->k >= 13 && resident_enabled(total) && max_nwin &&
-      !partition_enabled() && resident_usable(c, t))
-  {
-    rc = count_resident(c, t, r, rview, 0, r->n_reads, total, max_nwin);
+      !partition_enabled() && resident_usable(c, t) && (resident_forced() || resident_pays(t, r, total))) {
+    rc = count_resident(c, t, r, rview, 0, r->n_reads, total, &rb);
     if (rc != kNotResident) return rc;
   }
   if ((rc = table_zero(c, t))) return rc;
-  uint64_t rb = 0;
   while (rb < r->n_reads) {
     const uint32_t nparts = (uint32_t)(t->nb >> t->rbits);
     if (partition_enabled() && nparts >= 2 && nparts <= kMaxRegions && max_nwin) {
