@@ -297,6 +297,46 @@ def test_count_in_chunks_goes_on_with_atomics(api, ctx, monkeypatch):
     r.free()
 
 
+@pytest.mark.parametrize("case", ["nothing", "one stream", "all but the last buffer", "everything"])
+def test_count_without_room_for_the_streams(api, case, monkeypatch):
+    """Device memory runs out under the region passes' buffers (forced from
+    the host with TK_DEVICE_ALLOC_LIMIT): the count goes on with table atomics,
+    gives back what it had got, and is the oracle's; with room for everything
+    the region passes count."""
+    say("count_no_room", case)
+    monkeypatch.setenv("TK_ORDER_MIN_READS", "0")
+    monkeypatch.setenv("TK_RESIDENT", "1")
+    seqs = random_reads(17, 8000, 100, 150, n_rate=0.001) + repetitive_reads(25, 1000)
+    seq, off = concat(seqs)
+    ok, oc = O.count(seq, off, 25, True)
+
+    def count(limit):
+        """Counts and the device bytes that the count itself left in use."""
+        with api.Context(0) as c:
+            r = api.Reads(c, seq, off)
+            t = api.Table(c, 25, True, len(seq), 0.5)
+            api.estimate_distinct(c, r, 25, True)  # builds the reads' order
+            before = api.device_bytes_in_use()
+            if limit is not None:
+                monkeypatch.setenv("TK_DEVICE_ALLOC_LIMIT", str(before + limit))
+            t.count(r)
+            monkeypatch.delenv("TK_DEVICE_ALLOC_LIMIT", raising=False)
+            words, held = c.count_words(), api.device_bytes_in_use() - before
+            gk, gc = t.dump()
+            assert np.array_equal(gk, ok) and np.array_equal(gc, oc)
+            t.free()
+            r.free()
+        return words, held
+
+    words, held = count(None)
+    assert words > 0 and held > 2 * (64 << 20)  # two streams, histograms, tables
+    room = {"nothing": 1 << 20, "one stream": held // 2 + (1 << 20), "all but the last buffer": held - 1,
+            "everything": held}[case]
+    words, left = count(room)
+    assert (words > 0) == (case == "everything")
+    assert left <= (held if case == "everything" else 1 << 20)
+
+
 @pytest.mark.parametrize("resident", ["1", "0"])
 def test_count_reused_blocks(api, ctx, resident, monkeypatch):
     """With the thread's block reuse on, each table takes the block of the

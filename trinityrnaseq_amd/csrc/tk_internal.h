@@ -120,6 +120,7 @@ int table_finalize(tk_ctx* ctx, tk_table* t);
 int sort_pairs_u64_u32(tk_ctx* ctx, uint64_t* d_keys, uint32_t* d_vals, uint64_t n,
                        int key_bits);
 int exclusive_scan_u64(tk_ctx* ctx, const uint64_t* d_in, uint64_t* d_out, uint64_t n);
+int scan_reserve_u64(tk_ctx* ctx, uint64_t n);
 int exclusive_scan_u32(tk_ctx* ctx, const uint32_t* d_in, uint32_t* d_out, uint64_t n);
 int exclusive_scan_u32_in(tk_ctx* ctx, const uint32_t* d_in, uint32_t* d_out, uint64_t n, void* temp,
                           size_t temp_bytes);

@@ -2782,16 +2782,80 @@ static bool resident_plan(tk_ctx* c, uint64_t windows, uint64_t* cap, uint64_t* 
 }
 constexpr int kNotResident = -1000;
 
+// Layout of the sort passes of a region-resident count whose first pass has
+// ns1 slices: words grouped by coarse bins of F = 2^fs regions, then by single
+// regions; tables of at most kResOnePass regions by region at once.
+struct ResSort {
+  uint32_t R, F, C, fs = 0;
+  bool one_pass;
+  uint64_t ns2_max, nh1, nh2, nh_max;                           // slices of the second pass, histogram words
+  uint64_t hb_off, m_off, rs_off, cs_off, misc_bytes;           // tables of kSlotResMisc, after the slices
+  ResSort(const tk_table* t, uint64_t ns1) {
+    R = (uint32_t)(t->nb >> t->rbits);
+    one_pass = R <= kResOnePass;
+    while (!one_pass && (1ull << (2 * fs)) < R) fs++;
+    F = 1u << fs;
+    C = (uint32_t)ceil_div(R, F);
+    ns2_max = ns1 + C;  // sum over coarse bins of ceil(n_c / slice)
+    nh1 = (uint64_t)C * ns1;
+    nh2 = one_pass ? 0 : (uint64_t)F * ns2_max;
+    nh_max = std::max(nh1, nh2);
+    hb_off = ns2_max * sizeof(ResSlice);
+    m_off = hb_off + (uint64_t)C * 8;
+    rs_off = (m_off + (uint64_t)C * 4 + 7) / 8 * 8;
+    cs_off = rs_off + ((uint64_t)R + 1) * 8;
+    misc_bytes = cs_off + ((uint64_t)C + 1) * 8;
+  }
+};
+
+// Words per slice of a sort pass over n words: slices shrink with the stream,
+// so that a small one still gives every CU several blocks.
+static uint64_t res_slice_words(const tk_ctx* c, uint64_t n) {
+  const uint64_t blocks = (uint64_t)std::max(c->num_cu, 1) * 8;
+  return std::min<uint64_t>(kResSlice, std::max<uint64_t>(8192, ceil_div(n, blocks) / 8192 * 8192));
+}
+// Most slices of any n <= cap words: at most two per block of a CU's eight
+// until the slices have grown to kResSlice.
+static uint64_t res_slices_max(const tk_ctx* c, uint64_t cap) {
+  const uint64_t blocks = (uint64_t)std::max(c->num_cu, 1) * 8;
+  return std::max(std::min(ceil_div(cap, 8192), 2 * blocks), ceil_div(cap, kResSlice));
+}
+
+// Every buffer of a region pass with streams of cap words, before the merge
+// that needs it: a pass that has begun allocates nothing.
+static int res_reserve(tk_ctx* c, const tk_table* t, uint64_t cap) {
+  const ResSort m(t, res_slices_max(c, cap));
+  void* p = nullptr;
+  int rc = ensure_scratch(c, kSlotResA, cap * 8, &p);
+  if (!rc) rc = ensure_scratch(c, kSlotResB, cap * 8, &p);
+  if (!rc) rc = ensure_scratch(c, kSlotResHist, (m.nh_max + 1) * 16, &p);
+  if (!rc) rc = ensure_scratch(c, kSlotResMisc, m.misc_bytes, &p);
+  if (!rc) rc = scan_reserve_u64(c, m.nh_max + 1);
+  return rc;
+}
+
+// The buffers of the region passes go back to the device.
+static void res_release(tk_ctx* c) {
+  (void)hipStreamSynchronize(c->stream);
+  for (int i = kSlotResA; i <= kSlotResMisc; i++) {
+    dev_free(c->scratch[i].p, c->scratch[i].bytes);
+    c->scratch[i] = Scratch();
+  }
+}
+
 // Count reads [rb, re) of the locality order through the region-resident
 // passes: merge + emit, coarse sort, fine sort, per-region LDS count, in one
 // pass whose streams hold every word the merge can emit (resident_plan), or in
 // read chunks.  kNotResident: the table holds reads [rb, *done) and table
-// atomics are to count the rest (the streams do not fit, or the table is too
-// large for a chunk's region passes to pay).
+// atomics are to count the rest (there is no room for the streams, or the table
+// is too large for a chunk's region passes to pay).
 static int count_resident(tk_ctx* c, tk_table* t, const tk_reads* r, const ReadsView& rview, uint64_t rb,
                           uint64_t re, uint64_t windows, uint64_t* done) {
   *done = rb;
   int rc = TK_OK;
+  uint64_t cap = 0, echunk = 0, mgrid = 0, cap_max = 0, cap_chunked = 0;
+  bool whole = resident_plan(c, windows, &cap, &echunk, &mgrid, &cap_max, &cap_chunked);
+  if (!whole && cap_chunked < kResMinStreamWords) return kNotResident;  // before the table grows for it
   // the table's final regions must be known before words are grouped by them
   if ((double)(t->n_keys + windows) > 0.9 * (double)(t->nb * 8)) {
     double est = 0;
@@ -2799,17 +2863,15 @@ static int count_resident(tk_ctx* c, tk_table* t, const tk_reads* r, const Reads
     if (rb == 0 && re == r->n_reads && it != r->est.end())
       est = it->second;
     else if ((rc = hll_estimate(c, r, rb, re, t->k, t->canonical, windows, &est)))
-      return rc;
+      return rc == TK_ERR_OOM ? kNotResident : rc;
     const double want = (double)t->n_keys + 1.05 * est + 4096;
     if (want > t->max_load * (double)(t->nb * 8)) {
       if ((rc = table_zero(c, t))) return rc;  // the rehash reads the old slots
-      if ((rc = table_grow(c, t, (uint64_t)want))) return rc;
+      if ((rc = table_grow(c, t, (uint64_t)want))) return rc == TK_ERR_OOM ? kNotResident : rc;
+      if (!resident_usable(c, t)) return kNotResident;
+      whole = resident_plan(c, windows, &cap, &echunk, &mgrid, &cap_max, &cap_chunked);
     }
-    if (!resident_usable(c, t)) return fail(TK_ERR_ARG, "count: grown table has %llu-bucket regions",
-                                            (unsigned long long)(1ull << t->rbits));
   }
-  uint64_t cap = 0, echunk = 0, mgrid = 0, cap_max = 0, cap_chunked = 0;
-  bool whole = resident_plan(c, windows, &cap, &echunk, &mgrid, &cap_max, &cap_chunked);
   if (windows < kResLargeWindows) {
     whole = whole && cap <= kResMidWords;
     cap_chunked = std::min(cap_chunked, kResMidWords);
@@ -2850,16 +2912,19 @@ static int count_resident(tk_ctx* c, tk_table* t, const tk_reads* r, const Reads
     return forced || resident_pays(t, r, (uint64_t)((double)n_reads * win_per_read));
   };
   if (!pays(chunk)) return kNotResident;
-  void *pa = nullptr, *pb = nullptr;
-  if ((rc = ensure_scratch(c, kSlotResA, cap * 8, &pa))) return rc;
-  if ((rc = ensure_scratch(c, kSlotResB, cap * 8, &pb))) return rc;
-  uint64_t* A = (uint64_t*)pa;
-  uint64_t* B = (uint64_t*)pb;
   unsigned long long* cursor = reinterpret_cast<unsigned long long*>(c->d_flags + 8);
   for (uint64_t q = rb, qe = rb; q < re; q = qe) {
     qe = std::min<uint64_t>(re, q + chunk);
     *done = q;
     if (q > rb && !pays(qe - q)) return kNotResident;
+    // no room for the streams or the tables (another context, process or
+    // library took it since the plan): what there is goes back, the atomics count
+    if ((rc = res_reserve(c, t, cap))) {
+      res_release(c);
+      return rc == TK_ERR_OOM ? kNotResident : rc;
+    }
+    uint64_t* A = (uint64_t*)c->scratch[kSlotResA].p;
+    uint64_t* B = (uint64_t*)c->scratch[kSlotResB].p;
     const uint64_t keys_before = t->n_keys;
     TableView v = table_view(t);
     TK_HIP(hipMemsetAsync(c->d_flags, 0, 64, c->stream));
@@ -2902,41 +2967,26 @@ static int count_resident(tk_ctx* c, tk_table* t, const tk_reads* r, const Reads
       if ((rc = table_zero(c, t))) return rc;
       continue;
     }
-    // Words grouped by coarse bins of F = 2^fs regions, then by single regions;
-    // tables of at most kResOnePass regions by region at once.  Slices of a
-    // sort pass shrink with the stream, so that a small one still gives every
-    // CU several blocks.
-    const uint32_t R = (uint32_t)(t->nb >> t->rbits);
-    const bool one_pass = R <= kResOnePass;
-    uint32_t fs = 0;
-    while (!one_pass && (1ull << (2 * fs)) < R) fs++;
-    const uint32_t F = 1u << fs, C = (uint32_t)ceil_div(R, F);
-    const uint64_t slice = std::min<uint64_t>(
-        kResSlice, std::max<uint64_t>(8192, ceil_div(n, (uint64_t)std::max(c->num_cu, 1) * 8) / 8192 * 8192));
-    const uint64_t ns1 = ceil_div(n, slice);
-    const uint64_t ns2_max = ns1 + C;  // sum over coarse bins of ceil(n_c / slice)
-    const uint64_t nh1 = (uint64_t)C * ns1, nh2 = one_pass ? 0 : (uint64_t)F * ns2_max, nh_max = std::max(nh1, nh2);
-    void *hp = nullptr, *mp = nullptr;
-    const uint64_t sl_bytes = ns2_max * sizeof(ResSlice), hb_off = sl_bytes, m_off = hb_off + (uint64_t)C * 8,
-                   rs_off = (m_off + (uint64_t)C * 4 + 7) / 8 * 8, cs_off = rs_off + ((uint64_t)R + 1) * 8,
-                   misc_bytes = cs_off + ((uint64_t)C + 1) * 8;
-    if ((rc = ensure_scratch(c, kSlotResHist, (nh_max + 1) * 16, &hp))) return rc;
-    if ((rc = ensure_scratch(c, kSlotResMisc, misc_bytes, &mp))) return rc;
-    uint64_t* h = (uint64_t*)hp;
-    uint64_t* hs = h + nh_max + 1;
+    const uint64_t slice = res_slice_words(c, n), ns1 = ceil_div(n, slice);
+    const ResSort m(t, ns1);
+    const uint32_t R = m.R, F = m.F, C = m.C;
+    const bool one_pass = m.one_pass;
+    uint64_t* h = (uint64_t*)c->scratch[kSlotResHist].p;
+    uint64_t* hs = h + m.nh_max + 1;
+    char* mp = (char*)c->scratch[kSlotResMisc].p;
     ResSlice* dsl = (ResSlice*)mp;
-    uint64_t* dhb = (uint64_t*)((char*)mp + hb_off);
-    uint32_t* dm = (uint32_t*)((char*)mp + m_off);
-    uint64_t* drs = (uint64_t*)((char*)mp + rs_off);
-    uint64_t* dcs = (uint64_t*)((char*)mp + cs_off);
-    if ((rc = res_sort_pass(c, nullptr, ns1, n, slice, nh1, h, hs, A, B, v, fs, 0xFFFFFFFFu, C))) return rc;
+    uint64_t* dhb = (uint64_t*)(mp + m.hb_off);
+    uint32_t* dm = (uint32_t*)(mp + m.m_off);
+    uint64_t* drs = (uint64_t*)(mp + m.rs_off);
+    uint64_t* dcs = (uint64_t*)(mp + m.cs_off);
+    if ((rc = res_sort_pass(c, nullptr, ns1, n, slice, m.nh1, h, hs, A, B, v, m.fs, 0xFFFFFFFFu, C))) return rc;
     TK_LAUNCH(c, "count_bounds", ceil_div((uint64_t)C + 1, 256), 256, 0, k_res_starts, hs, ns1, C,
               one_pass ? drs : dcs);
     uint64_t* W = one_pass ? B : A;  // the words by region
     if (!one_pass) {
-      TK_LAUNCH(c, "count_bounds", 1, 1024, 0, k_res_plan, dcs, C, F, slice, (uint32_t)ns2_max, dsl, dhb, dm);
-      if ((rc = res_sort_pass(c, dsl, ns2_max, 0, 0, nh2, h, hs, B, A, v, 0, F - 1, F))) return rc;
-      TK_LAUNCH(c, "count_bounds", ceil_div((uint64_t)R + 1, 256), 256, 0, k_res_bounds, hs, dhb, dm, fs, R, dcs + C,
+      TK_LAUNCH(c, "count_bounds", 1, 1024, 0, k_res_plan, dcs, C, F, slice, (uint32_t)m.ns2_max, dsl, dhb, dm);
+      if ((rc = res_sort_pass(c, dsl, m.ns2_max, 0, 0, m.nh2, h, hs, B, A, v, 0, F - 1, F))) return rc;
+      TK_LAUNCH(c, "count_bounds", ceil_div((uint64_t)R + 1, 256), 256, 0, k_res_bounds, hs, dhb, dm, m.fs, R, dcs + C,
                 drs);
     }
     TK_HIP(hipMemsetAsync(c->d_flags, 0, 64, c->stream));
@@ -2973,8 +3023,10 @@ static int count_resident(tk_ctx* c, tk_table* t, const tk_reads* r, const Reads
     }
     if ((double)t->n_keys > t->max_load * (double)(t->nb * 8)) {
       if ((rc = table_grow(c, t, t->n_keys))) return rc;
-      if (qe < re && !resident_usable(c, t))
-        return fail(TK_ERR_ARG, "count: grown table has %llu-bucket regions", (unsigned long long)(1ull << t->rbits));
+      if (qe < re && !resident_usable(c, t)) {
+        *done = qe;
+        return kNotResident;
+      }
     }
   }
   return TK_OK;

@@ -4,6 +4,8 @@
 // selection.
 #include <hipcub/hipcub.hpp>
 
+#include <algorithm>
+
 #include "tk_internal.h"
 
 namespace tk {
@@ -87,6 +89,18 @@ int exclusive_scan_u32_in(tk_ctx* ctx, const uint32_t* d_in, uint32_t* d_out, ui
   timing_end(ctx, "scan_u32", a);
   if (e != hipSuccess) return hip_fail(e, "ExclusiveSum");
   return TK_OK;
+}
+
+// Temporary storage of an exclusive_scan_u64 over up to n items.
+int scan_reserve_u64(tk_ctx* ctx, uint64_t n) {
+  size_t temp = 0;
+  const uint64_t* in = nullptr;
+  uint64_t* out = nullptr;
+  hipError_t e = hipcub::DeviceScan::ExclusiveSum(nullptr, temp, in, out, (int)std::min<uint64_t>(n, 0x7FFFFFFF),
+                                                  ctx->stream);
+  if (e != hipSuccess) return hip_fail(e, "ExclusiveSum(size)");
+  void* tp = nullptr;
+  return ensure_scratch(ctx, 2, temp, &tp);
 }
 
 int exclusive_scan_u64(tk_ctx* ctx, const uint64_t* d_in, uint64_t* d_out, uint64_t n) {
