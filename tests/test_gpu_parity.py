@@ -313,6 +313,10 @@ def test_count_without_room_for_the_streams(api, case, monkeypatch):
     def count(limit):
         """Counts and the device bytes that the count itself left in use."""
         with api.Context(0) as c:
+            monkeypatch.setenv("TK_DEVICE_ALLOC_LIMIT", "1")  # other contexts' idle buffers go back
+            with pytest.raises(api.TkError):
+                api.DeviceBuffer(c, 1 << 20)
+            monkeypatch.delenv("TK_DEVICE_ALLOC_LIMIT")
             r = api.Reads(c, seq, off)
             t = api.Table(c, 25, True, len(seq), 0.5)
             api.estimate_distinct(c, r, 25, True)  # builds the reads' order
@@ -335,6 +339,74 @@ def test_count_without_room_for_the_streams(api, case, monkeypatch):
     words, left = count(room)
     assert (words > 0) == (case == "everything")
     assert left <= (held if case == "everything" else 1 << 20)
+
+
+@pytest.mark.parametrize("reuse", [False, True])
+def test_idle_streams_make_room(api, reuse, monkeypatch):
+    """The region passes' buffers that a context keeps between counts are given
+    back when another allocation of the thread would not fit beside them
+    (forced with TK_DEVICE_ALLOC_LIMIT, with and without the thread's block
+    reuse); the context's next count has them again."""
+    say("idle_streams", reuse)
+    monkeypatch.setenv("TK_ORDER_MIN_READS", "0")
+    monkeypatch.setenv("TK_RESIDENT", "1")
+    seqs = random_reads(19, 8000, 100, 150, n_rate=0.001)
+    seq, off = concat(seqs)
+    ok, oc = O.count(seq, off, 25, True)
+    if reuse:
+        api.thread_cache(1 << 20)
+    a, b = api.Context(0), api.Context(0)
+    try:
+        r = api.Reads(a, seq, off)
+        t = api.Table(a, 25, True, len(seq), 0.5)
+        empty = api.device_bytes_in_use()
+        t.count(r)
+        assert a.count_words() > 0
+        in_use = api.device_bytes_in_use()
+        assert in_use - empty > 128 << 20
+        monkeypatch.setenv("TK_DEVICE_ALLOC_LIMIT", str(in_use + (1 << 20)))
+        api.DeviceBuffer(b, 64 << 20).free()
+        assert api.device_bytes_in_use() < empty + (2 << 20)
+        monkeypatch.delenv("TK_DEVICE_ALLOC_LIMIT")
+        t.count(r)
+        assert a.count_words() > 0
+        gk, gc = t.dump()
+        assert np.array_equal(gk, ok) and np.array_equal(gc, 2 * oc)
+        t.free()
+        r.free()
+    finally:
+        a.close()
+        b.close()
+        if reuse:
+            api.thread_cache(0)
+
+
+def test_table_grows_in_place_of_the_streams(api, monkeypatch):
+    """A region-resident count after which the table has to grow (its slots
+    hold every window at load 0.8, its load allows 0.3), where the larger table
+    fits only without the passes' buffers: they go back for it."""
+    say("grow_beside_streams")
+    monkeypatch.setenv("TK_ORDER_MIN_READS", "0")
+    monkeypatch.setenv("TK_RESIDENT", "1")
+    seqs = random_reads(23, 60000, 100, 150, n_rate=0.0)
+    seq, off = concat(seqs)
+    ok, oc = O.count(seq, off, 25, True)
+    with api.Context(0) as c:
+        r = api.Reads(c, seq, off)
+        expected = int(0.3 * r.windows(25) / 0.8)
+        first = api.Table(c, 25, True, expected, 0.3)
+        first.count(r)  # the context has its buffers now
+        first.free()
+        t = api.Table(c, 25, True, expected, 0.3)
+        cap0 = t.info()["capacity"]
+        monkeypatch.setenv("TK_DEVICE_ALLOC_LIMIT", str(api.device_bytes_in_use() + (4 << 20)))
+        t.count(r)
+        monkeypatch.delenv("TK_DEVICE_ALLOC_LIMIT")
+        assert t.info()["capacity"] >= 2 * cap0 and c.count_words() > 0
+        gk, gc = t.dump()
+        assert np.array_equal(gk, ok) and np.array_equal(gc, oc)
+        t.free()
+        r.free()
 
 
 @pytest.mark.parametrize("resident", ["1", "0"])

@@ -16,6 +16,7 @@
 #include <cmath>
 #include <map>
 #include <mutex>
+#include <thread>
 #include <unordered_map>
 
 #include "tk_count_agg.h"
@@ -69,18 +70,83 @@ void cache_begin(size_t limit_bytes) {
 static thread_local uint64_t t_resident_limit = 0;
 void resident_limit(size_t bytes) { t_resident_limit = bytes; }
 
+// Scratch slots of the region-resident count (kept by the context, so the
+// multi-GB word streams are allocated once, not per count call).
+enum { kSlotResA = 4, kSlotResB = 5, kSlotResHist = 6, kSlotResMisc = 7 };
+
+// Contexts whose region-pass buffers are not in use: they may hold up to tens
+// of GB that matter to nothing but the speed of the next large count, so an
+// allocation that finds no memory, on any thread, takes them back before it
+// fails.  A count takes its context off the list while it runs.
+struct IdleBuffers {
+  tk_ctx* ctx;
+  std::thread::id thread;  // that counted
+  BlockCache* cache;       // that thread's: its blocks are for that thread to free
+};
+static std::mutex g_idle_mu;
+static std::vector<IdleBuffers> g_idle;
+
+static void idle_remove(const tk_ctx* c) {
+  std::lock_guard<std::mutex> lk(g_idle_mu);
+  g_idle.erase(std::remove_if(g_idle.begin(), g_idle.end(), [&](const IdleBuffers& b) { return b.ctx == c; }),
+               g_idle.end());
+}
+
+// Frees the idle buffers on the current device, of every thread or of this
+// one; false when there are none.
+static bool idle_release(bool any_thread) {
+  int dev = 0;
+  if (hipGetDevice(&dev) != hipSuccess) return false;
+  std::lock_guard<std::mutex> lk(g_idle_mu);
+  bool any = false;
+  for (auto it = g_idle.begin(); it != g_idle.end();) {
+    const bool mine = it->thread == std::this_thread::get_id();
+    if (it->ctx->device != dev || !(mine || (any_thread && !it->cache))) {
+      ++it;
+      continue;
+    }
+    for (int i = kSlotResA; i <= kSlotResMisc; i++) {
+      Scratch& s = it->ctx->scratch[i];
+      dev_free(s.p, s.bytes);
+      s = Scratch();
+    }
+    any = true;
+    it = g_idle.erase(it);
+  }
+  return any;
+}
+
+// A count's hold on its context's buffers.
+struct BuffersInUse {
+  tk_ctx* c;
+  explicit BuffersInUse(tk_ctx* ctx) : c(ctx) { idle_remove(c); }
+  ~BuffersInUse() {
+    bool any = false;
+    for (int i = kSlotResA; i <= kSlotResMisc; i++) any = any || c->scratch[i].p;
+    if (!any) return;
+    std::lock_guard<std::mutex> lk(g_idle_mu);
+    g_idle.push_back({c, std::this_thread::get_id(), t_cache});
+  }
+};
+
 void cache_end() {
   BlockCache* c = t_cache;
   if (!c) return;
   t_cache = nullptr;
+  {
+    std::lock_guard<std::mutex> lk(g_idle_mu);
+    for (auto& b : g_idle)
+      if (b.cache == c) b.cache = nullptr;
+  }
   for (auto& kv : c->free_blocks) (void)hipFree(kv.second);
   // blocks still handed out are released by their own dev_free (plain hipFree)
   delete c;
 }
 
 // TK_DEVICE_ALLOC_LIMIT=n: an allocation that would take the library's
-// device bytes in use past n fails with TK_ERR_OOM, as an exhausted device
-// would (the out-of-memory paths are tested with it).
+// device bytes in use past n, the calling thread's idle buffers taken back,
+// fails with TK_ERR_OOM, as an exhausted device would (the out-of-memory paths
+// are tested with it).
 static uint64_t alloc_limit() {
   const char* e = getenv("TK_DEVICE_ALLOC_LIMIT");
   return e ? strtoull(e, nullptr, 10) : 0;
@@ -90,6 +156,7 @@ int dev_alloc(void** p, size_t bytes) {
   *p = nullptr;
   if (bytes == 0) bytes = 256;
   if (const uint64_t lim = alloc_limit()) {
+    if (g_dev_bytes.load() + bytes > lim) (void)idle_release(false);
     if (g_dev_bytes.load() + bytes > lim)
       return fail(TK_ERR_OOM, "device allocation of %zu bytes past the limit of %llu bytes (TK_DEVICE_ALLOC_LIMIT)",
                   bytes, (unsigned long long)lim);
@@ -107,15 +174,21 @@ int dev_alloc(void** p, size_t bytes) {
     cap = cache_round(bytes);
   }
   hipError_t e = hipMalloc(p, cap);
-  if (e != hipSuccess && t_cache && !t_cache->free_blocks.empty()) {
-    // give the cached blocks back and try once more
+  // give the cached blocks back and try once more, then the idle buffers of
+  // the region passes
+  for (int step = 0; step < 2 && e != hipSuccess; step++) {
     (void)hipGetLastError();
-    for (auto& kv : t_cache->free_blocks) {
-      (void)hipFree(kv.second);
-      t_cache->owned.erase(kv.second);
+    if (step == 1 && !idle_release(true)) break;
+    if (t_cache) {
+      for (auto& kv : t_cache->free_blocks) {
+        (void)hipFree(kv.second);
+        t_cache->owned.erase(kv.second);
+      }
+      t_cache->free_blocks.clear();
+      t_cache->cached = 0;
+    } else if (step == 0) {
+      continue;
     }
-    t_cache->free_blocks.clear();
-    t_cache->cached = 0;
     e = hipMalloc(p, cap);
   }
   if (e != hipSuccess) {
@@ -2072,6 +2145,7 @@ int tk_ctx_free(tk_ctx* c) {
   if (!c) return TK_OK;
   (void)hipSetDevice(c->device);
   (void)hipStreamSynchronize(c->stream);
+  idle_remove(c);
   for (auto& p : c->pending) { (void)hipEventDestroy(p.a); (void)hipEventDestroy(p.b); }
   for (auto e : c->event_pool) (void)hipEventDestroy(e);
   for (auto& s : c->scratch) dev_free(s.p, s.bytes);
@@ -2700,10 +2774,6 @@ static uint32_t res_tile() {
   return v == 2048 || v == 4096 ? (uint32_t)v : 8192;
 }
 
-// Scratch slots of the region-resident count (kept by the context, so the
-// multi-GB word streams are allocated once, not per count call).
-enum { kSlotResA = 4, kSlotResB = 5, kSlotResHist = 6, kSlotResMisc = 7 };
-
 // One counting-sort pass of the region-resident count: the nonzero words of
 // `in` (`blocks` slices from the table dsl, or of [0, n) by `slice` words when
 // it is NULL) to `out`, grouped by bin (region >> shift) & mask.  h holds nhist
@@ -2834,13 +2904,24 @@ static int res_reserve(tk_ctx* c, const tk_table* t, uint64_t cap) {
   return rc;
 }
 
-// The buffers of the region passes go back to the device.
-static void res_release(tk_ctx* c) {
+// The buffers of the region passes (all but the one at keep) go back to the
+// device.
+static void res_release(tk_ctx* c, const void* keep = nullptr) {
   (void)hipStreamSynchronize(c->stream);
   for (int i = kSlotResA; i <= kSlotResMisc; i++) {
+    if (keep && c->scratch[i].p == keep) continue;
     dev_free(c->scratch[i].p, c->scratch[i].bytes);
     c->scratch[i] = Scratch();
   }
+}
+
+// table_grow beside the region passes' buffers: when it finds no room, all but
+// `keep` of them (the words still to be added) go back and it tries again.
+static int res_grow(tk_ctx* c, tk_table* t, uint64_t min_keys, const void* keep) {
+  int rc = table_grow(c, t, min_keys);
+  if (rc != TK_ERR_OOM) return rc;
+  res_release(c, keep);
+  return table_grow(c, t, min_keys);
 }
 
 // Count reads [rb, re) of the locality order through the region-resident
@@ -2853,6 +2934,7 @@ static int count_resident(tk_ctx* c, tk_table* t, const tk_reads* r, const Reads
                           uint64_t re, uint64_t windows, uint64_t* done) {
   *done = rb;
   int rc = TK_OK;
+  const BuffersInUse hold(c);
   uint64_t cap = 0, echunk = 0, mgrid = 0, cap_max = 0, cap_chunked = 0;
   bool whole = resident_plan(c, windows, &cap, &echunk, &mgrid, &cap_max, &cap_chunked);
   if (!whole && cap_chunked < kResMinStreamWords) return kNotResident;  // before the table grows for it
@@ -3010,7 +3092,7 @@ static int count_resident(tk_ctx* c, tk_table* t, const tk_reads* r, const Reads
     // still finds no room)
     for (int round = 0; c->h_flags[6]; round++) {
       if (round > 8) return fail(TK_ERR_FULL, "count: keys still find no room after growing");
-      if ((rc = table_grow(c, t, t->n_keys + total))) return rc;
+      if ((rc = res_grow(c, t, t->n_keys + total, W))) return rc;
       TK_HIP(hipMemsetAsync(c->d_flags, 0, 64, c->stream));
       TableView v3 = table_view(t);
       TK_LAUNCH(c, "count_retry", std::min<uint64_t>(ceil_div(total, 256), 65536), 256, 0, k_res_retry, W, total,
@@ -3022,7 +3104,7 @@ static int count_resident(tk_ctx* c, tk_table* t, const tk_reads* r, const Reads
       t->n_keys += nnew;
     }
     if ((double)t->n_keys > t->max_load * (double)(t->nb * 8)) {
-      if ((rc = table_grow(c, t, t->n_keys))) return rc;
+      if ((rc = res_grow(c, t, t->n_keys, nullptr))) return rc;
       if (qe < re && !resident_usable(c, t)) {
         *done = qe;
         return kNotResident;
