@@ -270,6 +270,35 @@ def test_count_chooses_regions_by_cost(api, ctx, n_reads, expected, prefill, res
     r.free()
 
 
+@pytest.mark.parametrize("estimated", [True, False])
+def test_count_again_keeps_the_table(api, ctx, estimated, monkeypatch):
+    """A table made for a sample's keys does not grow when the region passes
+    add the same sample, or another of the same transcripts, to it; it does
+    for reads of other transcripts."""
+    say("count_again", estimated)
+    from trinityrnaseq_amd import synth
+    monkeypatch.delenv("TK_RESIDENT", raising=False)
+    tx = synth.large_transcriptome(1003, 2000)
+    sets = [synth.se_reads(t, 70000, 150, seed=s, sub_rate=0.0)
+            for t, s in ((tx, 31), (tx, 32), (synth.large_transcriptome(1004, 8000), 33))]
+    reads = [api.Reads(ctx, s.tobytes(), o) for s, o in sets]
+    est = [api.estimate_distinct(ctx, r, 25, True) if estimated or i == 0 else 0 for i, r in enumerate(reads)]
+    t = api.Table(ctx, 25, True, int(1.35 * est[0]) + 4096, 0.5)
+    caps = []
+    for i in (0, 0, 1, 2):
+        t.count(reads[i])
+        assert ctx.count_words() > 0
+        caps.append(t.info()["capacity"])
+    assert caps[0] == caps[1] == caps[2] < caps[3]
+    seq = b"".join(sets[i][0].tobytes() for i in (0, 0, 1, 2))
+    ok, oc = O.count(seq, np.arange(4 * 70000 + 1, dtype=np.uint64) * np.uint64(150), 25, True)
+    gk, gc = t.dump()
+    assert np.array_equal(gk, ok) and np.array_equal(gc, oc)
+    t.free()
+    for r in reads:
+        r.free()
+
+
 def test_count_in_chunks_goes_on_with_atomics(api, ctx, monkeypatch):
     """A chunked count whose later chunks have fewer windows than a third of
     the table's slots: the first chunk writes the new table's regions, the

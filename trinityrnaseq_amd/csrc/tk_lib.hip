@@ -704,6 +704,16 @@ static int reads_windows(tk_ctx* ctx, const tk_reads* rc_, int k, uint64_t* tota
 constexpr int kHllBits = 12;
 constexpr int kHllRegs = 1 << kHllBits;
 
+// Key into the registers, if it is in the sample (below).
+__device__ __forceinline__ void hll_add(uint32_t* s_reg, uint64_t key, uint32_t sbits) {
+  const uint64_t h0 = mix64(key ^ 0x5bd1e9955bd1e995ULL);
+  if (sbits && (h0 >> (64 - sbits))) return;
+  const uint64_t h = h0 << sbits;
+  const uint32_t ix = (uint32_t)(h >> (64 - kHllBits));
+  const uint64_t rest = (h << kHllBits) | (1ull << (kHllBits - 1 + sbits));
+  atomicMax(&s_reg[ix], (uint32_t)__clzll(rest) + 1);
+}
+
 // HyperLogLog registers of the canonical k-mers.  Windows whose hash has its
 // top `sbits` bits zero (a 2^-sbits sample chosen by key, so every
 // occurrence of a sampled key is sampled) update the registers; the estimate
@@ -750,22 +760,38 @@ __global__ __launch_bounds__(256) void k_hll(ReadsView rv, uint64_t r_begin, uin
         fwd = ((fwd << 2) | b) & kmask;
         rc = (rc >> 2) | ((uint64_t)(3u - b) << rsh);
         run = ((msk >> (31 - j)) & 1u) ? 0u : run + 1;
-        if (run >= (uint32_t)k) {
-          const uint64_t key = (canonical && rc < fwd) ? rc : fwd;
-          const uint64_t h0 = mix64(key ^ 0x5bd1e9955bd1e995ULL);
-          if (!(sbits && (h0 >> (64 - sbits)))) {
-            const uint64_t h = h0 << sbits;
-            const uint32_t ix = (uint32_t)(h >> (64 - kHllBits));
-            const uint64_t rest = (h << kHllBits) | (1ull << (kHllBits - 1 + sbits));
-            atomicMax(&s_reg[ix], (uint32_t)__clzll(rest) + 1);
-          }
-        }
+        if (run >= (uint32_t)k) hll_add(s_reg, (canonical && rc < fwd) ? rc : fwd, sbits);
         if (keys) mk.push(b, 32 * w + j);
       }
     }
     if (keys) {
       keys[r] = mk.key(L);
       idx[r] = (uint32_t)r;
+    }
+  }
+  __syncthreads();
+  for (int i = threadIdx.x; i < kHllRegs; i += blockDim.x)
+    if (s_reg[i]) atomicMax(&regs[i], s_reg[i]);
+}
+
+// The keys of a table's slots into the same registers: those of the reads and
+// the table together then estimate their union.  One block of 1,024 threads per
+// CU, four 16-byte loads in flight per thread.
+__global__ __launch_bounds__(1024) void k_hll_slots(TableView t, uint64_t n_slots, uint32_t sbits,
+                                                    uint32_t* __restrict__ regs) {
+  __shared__ uint32_t s_reg[kHllRegs];
+  for (int i = threadIdx.x; i < kHllRegs; i += blockDim.x) s_reg[i] = 0;
+  __syncthreads();
+  const ulonglong2* l2 = reinterpret_cast<const ulonglong2*>(t.slots);
+  const uint64_t n2 = n_slots / 2, stride = (uint64_t)gridDim.x * blockDim.x;  // whole buckets: n_slots % 8 == 0
+  for (uint64_t i0 = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i0 < n2; i0 += 4 * stride) {
+    ulonglong2 v[4];
+#pragma unroll
+    for (int u = 0; u < 4; u++) v[u] = i0 + u * stride < n2 ? l2[i0 + u * stride] : make_ulonglong2(0ull, 0ull);
+#pragma unroll
+    for (int u = 0; u < 4; u++) {
+      if (v[u].x) hll_add(s_reg, v[u].x & (t.occ - 1), sbits);
+      if (v[u].y) hll_add(s_reg, v[u].y & (t.occ - 1), sbits);
     }
   }
   __syncthreads();
@@ -2401,7 +2427,7 @@ int tk_reads_free(tk_reads* r) {
 
 // ---------------- table ----------------
 static int hll_estimate(tk_ctx* c, const tk_reads* r, uint64_t rb, uint64_t re, int k, int canonical,
-                        uint64_t windows, double* est);
+                        uint64_t windows, double* est, const tk_table* t = nullptr);
 
 int tk_estimate_distinct(tk_ctx* c, const tk_reads* r, int k, int canonical, double* est) {
   if (!c || !r || !est) return fail(TK_ERR_ARG, "NULL argument");
@@ -2449,10 +2475,11 @@ int tk_table_info(const tk_table* t, int* k, int* canonical, uint64_t* capacity,
   return TK_OK;
 }
 
-// HyperLogLog estimate of the distinct keys of reads [rb, re).  Large inputs
-// (>= 64M windows) update the registers from a 1/16 key sample.
+// HyperLogLog estimate of the distinct keys of reads [rb, re), and of table t's
+// keys with them (NULL: none).  Large inputs (>= 64M windows) update the
+// registers from a 1/16 key sample.
 static int hll_estimate(tk_ctx* c, const tk_reads* r, uint64_t rb, uint64_t re, int k, int canonical,
-                        uint64_t windows, double* est) {
+                        uint64_t windows, double* est, const tk_table* t) {
   void* p = nullptr;
   int rc = ensure_scratch(c, 0, kHllRegs * 4, &p);
   if (rc) return rc;
@@ -2490,6 +2517,8 @@ static int hll_estimate(tk_ctx* c, const tk_reads* r, uint64_t rb, uint64_t re, 
     }
   }
   if (keys && (rc = order_finish(c, rw, keys, order))) return rc;
+  if (t)
+    TK_LAUNCH(c, "hll_slots", std::max(c->num_cu, 1), 1024, 0, k_hll_slots, table_view(t), t->nb * 8, sbits, regs);
   std::vector<uint32_t> h(kHllRegs);
   TK_HIP(hipMemcpyAsync(h.data(), regs, kHllRegs * 4, hipMemcpyDeviceToHost, c->stream));
   TK_HIP(hipStreamSynchronize(c->stream));
@@ -2940,14 +2969,20 @@ static int count_resident(tk_ctx* c, tk_table* t, const tk_reads* r, const Reads
   if (!whole && cap_chunked < kResMinStreamWords) return kNotResident;  // before the table grows for it
   // the table's final regions must be known before words are grouped by them
   if ((double)(t->n_keys + windows) > 0.9 * (double)(t->nb * 8)) {
-    double est = 0;
+    const double limit = t->max_load * (double)(t->nb * 8);
+    double est = 0, want = 0;
     auto it = r->est.find(2 * t->k + t->canonical);  // the caller's own estimate of these reads
-    if (rb == 0 && re == r->n_reads && it != r->est.end())
-      est = it->second;
-    else if ((rc = hll_estimate(c, r, rb, re, t->k, t->canonical, windows, &est)))
-      return rc == TK_ERR_OOM ? kNotResident : rc;
-    const double want = (double)t->n_keys + 1.05 * est + 4096;
-    if (want > t->max_load * (double)(t->nb * 8)) {
+    const bool known = rb == 0 && re == r->n_reads && it != r->est.end();
+    if (known) want = (double)t->n_keys + 1.05 * it->second + 4096;
+    // without one, or when it would have a table grow for keys that it may hold
+    // already (the next part of a sample, the same reads again): from the reads
+    // and the table together
+    if (!known || (t->n_keys && want > limit)) {
+      rc = hll_estimate(c, r, rb, re, t->k, t->canonical, windows, &est, t->n_keys ? t : nullptr);
+      if (rc) return rc == TK_ERR_OOM ? kNotResident : rc;
+      want = !t->n_keys || est > limit ? 1.05 * est + 4096 : 0;
+    }
+    if (want > limit) {
       if ((rc = table_zero(c, t))) return rc;  // the rehash reads the old slots
       if ((rc = table_grow(c, t, (uint64_t)want))) return rc == TK_ERR_OOM ? kNotResident : rc;
       if (!resident_usable(c, t)) return kNotResident;
