@@ -155,22 +155,6 @@ __device__ __forceinline__ void window_at(const ReadsView& rv, uint64_t wbase,
   valid = (m >> (32 - k)) == 0u;
 }
 
-// As window_at, plus the window's non-ACGT mask: bit k-1-i set when base
-// pos+i is not ACGT (bit 0 = the window's last base).
-__device__ __forceinline__ void window_at_mask(const ReadsView& rv, uint64_t wbase, uint32_t pos, int k,
-                                               uint64_t& fwd, uint32_t& nmask) {
-  const uint64_t w = wbase + (pos >> 5);
-  const uint32_t o = pos & 31u;
-  const uint64_t hi = rv.codes[w];
-  const uint64_t lo = rv.codes[w + 1];
-  const uint32_t mhi = rv.nmask[w];
-  const uint32_t mlo = rv.nmask[w + 1];
-  const uint64_t x = o ? ((hi << (2 * o)) | (lo >> (64 - 2 * o))) : hi;
-  const uint32_t m = o ? ((mhi << o) | (mlo >> (32 - o))) : mhi;
-  fwd = x >> (64 - 2 * k);
-  nmask = m >> (32 - k);
-}
-
 // The words a lane needs for its two windows of a run of 128 (windows lane and
 // 64 + lane of a read whose words start at wb): words lane/32 .. lane/32 + 3.
 // Every lane loads its own (three 16-byte loads, one or two lines per wave),
@@ -367,139 +351,6 @@ __device__ __forceinline__ uint64_t slot_count(const TableView& t, uint64_t s) {
   if (f != t.cmax) return f;
   const uint64_t* o = ovf_find(t, s & t.kmo);
   return o ? *o : f;
-}
-
-// ---- LDS tables of 64-B buckets (eight slots in the global slot format) ----
-// Insert-or-add into an LDS table of nb buckets: `word` = tagged key | c <<
-// cshift.  From bucket b (wrapping at nb) each step reads one bucket, picks without
-// branching the slot holding the key or else the first empty one, and
-// issues a single atomic there: add c, or claim with CAS (a lost claim
-// rescans the same bucket).  Occupied slots stay a prefix of their bucket.
-// Returns 2 when a slot was claimed, 1 when added (old = previous slot
-// value), 0 when max_steps steps found no room.
-__device__ __forceinline__ int lds_bucket_add(uint64_t* tab, uint32_t b, uint32_t nb, uint64_t word,
-                                              uint64_t kmo, uint32_t cshift, uint32_t max_steps,
-                                              uint64_t& old) {
-  const uint64_t tagged = word & kmo;
-  const uint64_t add = (word >> cshift) << cshift;
-  for (uint32_t p = 0; p < max_steps; p++) {
-    uint64_t* line = tab + ((uint64_t)b << 3);
-    const ulonglong2* l2 = reinterpret_cast<const ulonglong2*>(line);
-    const ulonglong2 v0 = l2[0], v1 = l2[1], v2 = l2[2], v3 = l2[3];
-    const uint64_t sv[8] = {v0.x, v0.y, v1.x, v1.y, v2.x, v2.y, v3.x, v3.y};
-    int jm = 8, je = 8;
-#pragma unroll
-    for (int j = 7; j >= 0; j--) {
-      jm = (sv[j] & kmo) == tagged ? j : jm;
-      je = sv[j] == 0 ? j : je;
-    }
-    if (jm < 8) {
-      old = atomicAdd((unsigned long long*)&line[jm], (unsigned long long)add);
-      return 1;
-    }
-    if (je < 8) {
-      const uint64_t v = atomicCAS((unsigned long long*)&line[je], 0ull, (unsigned long long)word);
-      if (v == 0) return 2;
-      if ((v & kmo) == tagged) {
-        old = atomicAdd((unsigned long long*)&line[je], (unsigned long long)add);
-        return 1;
-      }
-      continue;  // another key took the slot: rescan this bucket
-    }
-    b = b + 1 == nb ? 0 : b + 1;
-  }
-  return 0;
-}
-
-// lds_bucket_add_khi reading each bucket in two halves: the second four
-// slots only when the first four hold neither the key nor an empty slot
-// (occupied slots form a prefix, so a half that ends in an empty slot ends
-// the bucket).  Same protocol and results.
-__device__ __forceinline__ int lds_bucket_add_khi_half(uint64_t* tab, uint32_t b, uint32_t nb, uint64_t word,
-                                                       uint32_t khi, uint32_t cshift, uint32_t max_steps,
-                                                       uint64_t& old) {
-  const uint32_t tlo = (uint32_t)word, thi = (uint32_t)(word >> 32) & khi;
-  const uint64_t add = (word >> cshift) << cshift;
-  for (uint32_t p = 0; p < max_steps; p++) {
-    uint64_t* line = tab + ((uint64_t)b << 3);
-    const uint4* l4 = reinterpret_cast<const uint4*>(line);
-    int jm = 8, je = 8;
-    {
-      const uint4 q0 = l4[0], q1 = l4[1];
-      const uint32_t lo[4] = {q0.x, q0.z, q1.x, q1.z};
-      const uint32_t hi[4] = {q0.y, q0.w, q1.y, q1.w};
-#pragma unroll
-      for (int j = 3; j >= 0; j--) {
-        jm = (lo[j] == tlo && (hi[j] & khi) == thi) ? j : jm;
-        je = hi[j] == 0 ? j : je;
-      }
-    }
-    if (jm == 8 && je == 8) {
-      const uint4 q2 = l4[2], q3 = l4[3];
-      const uint32_t lo[4] = {q2.x, q2.z, q3.x, q3.z};
-      const uint32_t hi[4] = {q2.y, q2.w, q3.y, q3.w};
-#pragma unroll
-      for (int j = 3; j >= 0; j--) {
-        jm = (lo[j] == tlo && (hi[j] & khi) == thi) ? j + 4 : jm;
-        je = hi[j] == 0 ? j + 4 : je;
-      }
-    }
-    if (jm < 8) {
-      old = atomicAdd((unsigned long long*)&line[jm], (unsigned long long)add);
-      return 1;
-    }
-    if (je < 8) {
-      const uint64_t v = atomicCAS((unsigned long long*)&line[je], 0ull, (unsigned long long)word);
-      if (v == 0) return 2;
-      if ((uint32_t)v == tlo && ((uint32_t)(v >> 32) & khi) == thi) {
-        old = atomicAdd((unsigned long long*)&line[je], (unsigned long long)add);
-        return 1;
-      }
-      continue;  // another key took the slot: rescan this bucket
-    }
-    b = b + 1 == nb ? 0 : b + 1;
-  }
-  return 0;
-}
-
-// lds_bucket_add for 2k >= 32: the key's low 32 bits are all of the slot's
-// low word and the occupied bit lies in the high word, so a slot matches
-// when its low word equals the key's and its masked high word the tagged
-// key's, and it is empty when its high word is zero.  khi = high word of
-// the key + occupied mask.
-__device__ __forceinline__ int lds_bucket_add_khi(uint64_t* tab, uint32_t b, uint32_t nb, uint64_t word,
-                                                  uint32_t khi, uint32_t cshift, uint32_t max_steps,
-                                                  uint64_t& old) {
-  const uint32_t tlo = (uint32_t)word, thi = (uint32_t)(word >> 32) & khi;
-  const uint64_t add = (word >> cshift) << cshift;
-  for (uint32_t p = 0; p < max_steps; p++) {
-    uint64_t* line = tab + ((uint64_t)b << 3);
-    const uint4* l4 = reinterpret_cast<const uint4*>(line);
-    const uint4 q0 = l4[0], q1 = l4[1], q2 = l4[2], q3 = l4[3];
-    const uint32_t lo[8] = {q0.x, q0.z, q1.x, q1.z, q2.x, q2.z, q3.x, q3.z};
-    const uint32_t hi[8] = {q0.y, q0.w, q1.y, q1.w, q2.y, q2.w, q3.y, q3.w};
-    int jm = 8, je = 8;
-#pragma unroll
-    for (int j = 7; j >= 0; j--) {
-      jm = (lo[j] == tlo && (hi[j] & khi) == thi) ? j : jm;
-      je = hi[j] == 0 ? j : je;
-    }
-    if (jm < 8) {
-      old = atomicAdd((unsigned long long*)&line[jm], (unsigned long long)add);
-      return 1;
-    }
-    if (je < 8) {
-      const uint64_t v = atomicCAS((unsigned long long*)&line[je], 0ull, (unsigned long long)word);
-      if (v == 0) return 2;
-      if ((uint32_t)v == tlo && ((uint32_t)(v >> 32) & khi) == thi) {
-        old = atomicAdd((unsigned long long*)&line[je], (unsigned long long)add);
-        return 1;
-      }
-      continue;  // another key took the slot: rescan this bucket
-    }
-    b = b + 1 == nb ? 0 : b + 1;
-  }
-  return 0;
 }
 
 // ---- LDS tables with an 8-bit tag per slot ----

@@ -380,20 +380,6 @@ __global__ __launch_bounds__(256) void k_read_words(const uint64_t* __restrict__
   }
 }
 
-__device__ __forceinline__ uint32_t base_code(uint8_t ch, uint32_t& bad) {
-  // A/a=0 C/c=1 G/g=2 T/t=3 ; everything else invalid
-  const uint8_t u = ch & 0xDF;  // upper-case letters
-  uint32_t c = 0;
-  bad = 0;
-  if (u == 'A') c = 0;
-  else if (u == 'C') c = 1;
-  else if (u == 'G') c = 2;
-  else if (u == 'T') c = 3;
-  else bad = 1;
-  if (ch < 'A') bad = 1;  // digits/punctuation whose low bits alias letters
-  return c;
-}
-
 // blk_read[b] = read holding word 256*b (thread per read; reads are
 // ordered, so every 256-word block start lies in exactly one read).
 __global__ void k_block_starts(const uint64_t* __restrict__ word_off, uint64_t n,
@@ -2080,14 +2066,8 @@ static uint32_t read_ticket_grab(const tk_ctx* ctx, uint64_t n_reads) {
   return v > 1024 ? 1024u : (uint32_t)v;
 }
 
-static int grid_for_waves(tk_ctx* ctx, uint64_t n_items, int waves_per_block) {
-  uint64_t want = ceil_div(n_items, (uint64_t)waves_per_block);
-  uint64_t cap = (uint64_t)std::max(ctx->num_cu, 1) * 32;
-  return (int)std::max<uint64_t>(1, std::min<uint64_t>(want, cap));
-}
-
-// LDS per wave for the per-read kernels: a value slab of `slab` u32 plus a
-// 64 x u64 lookup scratch; at most 64 KiB per block.  Returns waves per block.
+// LDS per wave for the per-read kernels: a value slab of `slab` u32 plus
+// kLookupScratch u64; at most 64 KiB per block.  Returns waves per block.
 static int slab_layout(uint32_t max_nwin, uint32_t* slab, int* wpb) {
   uint32_t s = std::max<uint32_t>(64, (max_nwin + 63) / 64 * 64);
   if ((uint64_t)s * 4 + 8 * kLookupScratch > 65536) return -1;

@@ -315,7 +315,7 @@ __device__ __forceinline__ void cache_put(const CountCache& c, uint64_t tagged, 
 
 // stats_read for a read of at most 128 windows, with the block's count
 // cache in front of the table: only keys the cache does not hold are looked
-// up (coop4_get reads no bucket for the others), and those are added to it.
+// up (the others' lanes load bucket 0 with them), and those are added to it.
 __device__ inline void stats_read_cached(const ReadsView& rv, uint64_t r, int k, int canonical,
                                          const TableView& t, const StatsParams& sp, const CountCache& cc,
                                          uint64_t* tmp, int lane, tk_read_stat* out) {
