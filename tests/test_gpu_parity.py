@@ -209,24 +209,51 @@ def test_count_resident_in_chunks(api, ctx, mode, monkeypatch):
     assert np.array_equal(gk, ok) and np.array_equal(gc, 2 * oc)
 
 
-@pytest.mark.parametrize("wpr", ["1", "2"])
-def test_count_resident_merge_windows_per_round(api, ctx, wpr, monkeypatch):
-    """The region-resident merge with one or two windows per thread between
-    its block barriers: homopolymer reads put a block's every window on one
-    key (the merge's per-flush occurrence bound, and counts past the slot's
-    count field), random ones fill its table to the load bound."""
-    say("count_resident_merge wpr", wpr)
-    monkeypatch.setenv("TK_MERGE_WPR", wpr)
+@pytest.mark.parametrize("region_kb,one_pass", [("64", True), ("4", False)])
+def test_count_resident_merge_runs_and_loads(api, ctx, region_kb, one_pass, monkeypatch):
+    """The region-resident merge: homopolymer reads put a block's every window
+    on one key (the merge's per-flush occurrence bound, and counts past the
+    slot's count field), random ones fill its table to the load bound.  Its
+    words sorted by region in one pass (at most 960 regions) or in two."""
+    say("count_resident_merge region_kb", region_kb)
     monkeypatch.setenv("TK_PARTITION", "0")
     monkeypatch.setenv("TK_ORDER", "1")
     monkeypatch.setenv("TK_ORDER_MIN_READS", "0")
     monkeypatch.setenv("TK_RESIDENT", "1")
-    monkeypatch.setenv("TK_REGION_KB", "4")
+    monkeypatch.setenv("TK_REGION_KB", region_kb)
     seqs = (random_reads(41, 30000, 25, 150, n_rate=0.002) + repetitive_reads(25, 6000)
             + ["A" * 150] * 3000 + ["ACG" * 50] * 500)
+    ctx.timing(True)
+    ctx.timing_reset()
     r, t, seq, off = _count(api, ctx, seqs, 25, True)
+    ctx.sync()
+    passes = ctx.kernel_time("count_scatter")[1]
+    ctx.timing(False)
+    assert (t.info()["capacity"] * 8 // (int(region_kb) << 10) <= 960) == one_pass
+    assert passes == (1 if one_pass else 2)
     ok, oc = O.count(seq, off, 25, True)
     assert oc.max() > 8064
+    gk, gc = t.dump()
+    assert np.array_equal(gk, ok) and np.array_equal(gc, oc)
+
+
+def test_count_resident_crowded_in_one_pass(api, ctx, monkeypatch):
+    """Crowded regions of a table that is sorted in one pass, whose words lie
+    in the other stream: 128-slot regions at load 0.86, of which some receive
+    more keys than they hold, added after the table grows."""
+    say("count_resident_crowded_one_pass")
+    monkeypatch.setenv("TK_ORDER_MIN_READS", "0")
+    monkeypatch.setenv("TK_RESIDENT", "1")
+    monkeypatch.setenv("TK_REGION_KB", "1")
+    seqs = random_reads(18, 900, 100, 150, n_rate=0.001)
+    ctx.timing(True)
+    ctx.timing_reset()
+    r, t, seq, off = _count(api, ctx, seqs, 25, True, expected=64, max_load=0.9)
+    ctx.sync()
+    launches = [ctx.kernel_time(n)[1] for n in ("count_scatter", "count_regions", "count_retry")]
+    ctx.timing(False)
+    assert launches[:2] == [1, 1] and launches[2] >= 1
+    ok, oc = O.count(seq, off, 25, True)
     gk, gc = t.dump()
     assert np.array_equal(gk, ok) and np.array_equal(gc, oc)
 
