@@ -124,8 +124,11 @@ struct BuffersInUse {
     bool any = false;
     for (int i = kSlotResA; i <= kSlotResMisc; i++) any = any || c->scratch[i].p;
     if (!any) return;
-    std::lock_guard<std::mutex> lk(g_idle_mu);
-    g_idle.push_back({c, std::this_thread::get_id(), t_cache});
+    try {
+      std::lock_guard<std::mutex> lk(g_idle_mu);
+      g_idle.push_back({c, std::this_thread::get_id(), t_cache});
+    } catch (...) {  // no host memory to list them: they stay with the context
+    }
   }
 };
 
