@@ -83,3 +83,59 @@ def test_batch_table_regions(api, ctx, monkeypatch, k, canonical, packed):
             a, z = int(ro[c]), int(ro[c + 1])
             assert np.array_equal(vo[a:z], want.astype(vo.dtype)), (rep, c)
     b.free()
+
+
+def _with_runs_of_empties(rng, k, runs):
+    """Contigs of 40 to 400 bases with runs of empty ones between them, and
+    reads from them."""
+    contigs = []
+    for n in runs:
+        contigs += ["".join(rng.choice(list("ACGT"), size=int(rng.integers(40, 400)))) for _ in range(20)] + [""] * n
+    contigs.append(contigs[0])
+    whole = [c for c in contigs if c]
+    return contigs, [whole[int(rng.integers(len(whole)))][:150] for _ in range(300)]
+
+
+@pytest.mark.parametrize("k", [25, 31])
+def test_runs_of_empty_contigs(api, ctx, k):
+    """The passes that go over packed contig words find each word's contig past
+    runs of empty ones, shorter and longer than they step over one by one: one
+    table, and a batch whose table has several regions."""
+    print("runs_of_empty_contigs", k, flush=True)
+    contigs, reads = _with_runs_of_empties(np.random.default_rng(6), k, [0, 1, 2, 3, 4, 5, 6, 7, 100, 1000] * 3)
+    seq, off = concat(reads)
+    bseq, boff = concat(contigs)
+    keys, cv = O.r2t_build(bseq, boff, np.arange(len(contigs)), k, True)
+    want = O.r2t_vote(seq, off, keys, cv, k, True)
+    r, b = api.Reads(ctx, seq, off), api.Reads(ctx, bseq, boff)
+    t = api.CTable(ctx, b, np.arange(len(contigs), dtype=np.uint32), k, True)
+    assert np.array_equal(t.vote(r), want.astype(api.R2T_VOTE_DTYPE))
+    n = len(reads)
+    batch = api.Batch(ctx, r, np.array([0, n], np.uint64), b, np.array([0, len(contigs)], np.uint64), k=k)
+    d_st, d_vo = api.DeviceBuffer(ctx, n * 32), api.DeviceBuffer(ctx, n * 12)
+    batch.run_d(d_st.ptr, d_vo.ptr)
+    vo = np.zeros(n, api.R2T_VOTE_DTYPE)
+    d_vo.download(vo)
+    assert np.array_equal(vo, want.astype(vo.dtype))
+    batch.free()
+
+
+def test_long_run_of_empty_contigs_is_stepped_over(api, ctx):
+    """A million empty sequences between two others cost the table build a
+    bisection, not a million steps of one lane."""
+    print("long_run_of_empty_contigs", flush=True)
+    contigs, reads = _with_runs_of_empties(np.random.default_rng(7), 25, [1_000_000, 0])
+    bseq, boff = concat(contigs)
+    b = api.Reads(ctx, bseq, boff)
+    comps = np.arange(len(contigs), dtype=np.uint32)
+    ctx.timing(True)
+    ctx.timing_reset()
+    t = api.CTable(ctx, b, comps, 25, True)
+    ctx.sync()
+    ms = ctx.kernel_time("ctable_build")[0]
+    ctx.timing(False)
+    seq, off = concat(reads)
+    keys, cv = O.r2t_build(bseq, boff, comps, 25, True)
+    assert np.array_equal(t.vote(api.Reads(ctx, seq, off)), O.r2t_vote(seq, off, keys, cv, 25, True).astype(api.R2T_VOTE_DTYPE))
+    print("ctable_build", ms, "ms", flush=True)
+    assert ms < 5  # 0.02; 84 step by step

@@ -301,7 +301,7 @@ struct ContigWalk {
     const words2 nx = *reinterpret_cast<const words2*>(cv.codes + w + 2);  // the arrays end in padding
     const uint32_t nmx = cv.nmask[w + 2], nmy = cv.nmask[w + 3];
     if (w < wend && wn <= w) {
-      do r++; while (cv.word_off[r + 1] <= w);
+      r = read_from(cv.word_off, cv.n_reads, r, w);
       wb = cv.word_off[r];
       wn = cv.word_off[r + 1];
       len = cv.len[r];

@@ -192,6 +192,23 @@ __device__ __forceinline__ uint64_t read_of_word(const uint64_t* __restrict__ wo
   return lo;
 }
 
+// The read holding word w, from a read r on whose first word is at or before
+// it: r or one of the next few, or by bisection past a run of empty reads.
+__device__ __forceinline__ uint64_t read_from(const uint64_t* __restrict__ word_off, uint64_t n_reads, uint64_t r,
+                                              uint64_t w) {
+  for (int i = 0; i < 4; i++) {
+    if (word_off[r + 1] > w) return r;
+    r++;
+  }
+  uint64_t hi = n_reads;
+  while (hi - r > 1) {
+    const uint64_t mid = r + ((hi - r) >> 1);
+    if (word_off[mid] <= w) r = mid;
+    else hi = mid;
+  }
+  return r;
+}
+
 // Forward k-mer at base o (< 32) of the word pair (hi, lo) with masks (mhi, mlo).
 __device__ __forceinline__ void pair_window(uint64_t hi, uint64_t lo, uint32_t mhi, uint32_t mlo, uint32_t o, int k,
                                             uint64_t& fwd, bool& valid) {

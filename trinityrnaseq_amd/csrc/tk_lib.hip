@@ -1968,7 +1968,7 @@ __global__ __launch_bounds__(256) void k_ctable_build(ReadsView rv, uint64_t n_w
     uint64_t r = read_of_word(rv.word_off, rv.n_reads, w0, lane);
     const uint64_t wend = std::min<uint64_t>(n_words, w0 + per);
     for (uint64_t w = w0 + (lane >> 5); w < wend; w += 2) {
-      while (rv.word_off[r + 1] <= w) r++;
+      r = read_from(rv.word_off, rv.n_reads, r, w);
       const uint64_t wb = rv.word_off[r];
       const uint64_t pos = (w - wb) * 32 + (lane & 31);
       if (pos + k <= rv.len[r]) {
