@@ -150,10 +150,12 @@ int tk_table_create(tk_ctx* ctx, int k, int canonical, uint64_t expected_distinc
 int tk_table_info(const tk_table* t, int* k, int* canonical, uint64_t* capacity,
                   uint64_t* device_bytes);
 /* Count every N-free window of reads (jellyfish count).  Accumulates.  Large
-   counts (>= 2^23 windows, and a third of the slots of a table that holds keys
-   already) group their merged keys by table region and count each region in
-   LDS, keeping two word streams as context scratch (freed by tk_ctx_free);
-   others add merged keys to the table with atomics. */
+   counts (>= 2^23 windows, a third of the slots of a table that holds keys
+   already and a seventh of a new one's, a quarter from 2^28 windows on) group
+   their merged keys by table region and count each region in LDS, keeping two
+   word streams as context scratch (given back when another allocation needs
+   the memory, and by tk_ctx_free); others add merged keys to the table with
+   atomics. */
 int tk_count(tk_ctx* ctx, tk_table* t, const tk_reads* reads);
 /* Number of keys whose count lies in [min_count, max_count]. */
 int tk_table_dump_size(tk_ctx* ctx, tk_table* t, uint32_t min_count, uint32_t max_count,

@@ -264,13 +264,16 @@ def test_count_resident_crowded_in_one_pass(api, ctx, monkeypatch):
     (66577, 1 << 22, True, True),     # onto keys, one slot per window
     (66577, 12_000_000, True, True),  # 2.9 slots per window
     (66577, 13_000_000, True, False),  # 3.1
-    (66577, 13_000_000, False, True),  # the same size, empty: written once either way
+    (66577, 13_000_000, False, True),  # the same size, new
+    (66577, 29_000_000, False, True),  # new, 6.9 slots per window
+    (66577, 30_000_000, False, False),  # 7.2
 ])
 def test_count_chooses_regions_by_cost(api, ctx, n_reads, expected, prefill, resident, monkeypatch):
     """The default choice of the region-resident passes: from 2^23 windows on,
-    and, for a table that holds keys already, up to three slots per window (the
-    passes read and write such a table again wherever a word falls).  Either
-    way the counts are the oracle's."""
+    up to three slots per window of a table that holds keys already (the passes
+    read and write it again wherever a word falls) and seven of a new one
+    (which they write more slowly than it is cleared).  Either way the counts
+    are the oracle's."""
     say("count_choice", n_reads, expected, prefill)
     from trinityrnaseq_amd import synth
     monkeypatch.delenv("TK_RESIDENT", raising=False)

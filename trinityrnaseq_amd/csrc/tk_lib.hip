@@ -2714,9 +2714,14 @@ static bool resident_enabled(uint64_t windows) {
 // 9.59 with regions, 756 M windows added to 8 / 16 / 64 GB 19.9 / 20.0 / 20.1 and
 // 16.0 / 20.2 / 50.3.  The two cost the same at 4.4 slots per window for 10 M
 // windows, 4.1 for 30 M, 4.0 for 76 M, 3.1 for 252 M and 2.8 for 756 M.
+// A new table not yet cleared is written whole either way, by the region pass
+// at 0.39 ms per GB, cleared for the atomics at 0.19: the same cost at 8, 7.5,
+// 7.7, 6.8 and 4.6 slots per window (30 M windows into 0.3 / 1.8 / 5.4 GB: 1.53 /
+// 1.66 / 2.31 ms with atomics, 1.12 / 1.72 / 3.49 with regions).
 constexpr uint64_t kResSlotsPerWindow = 3;
+static uint64_t res_new_slots_per_window(uint64_t windows) { return windows < (1ull << 28) ? 7 : 4; }
 static bool resident_pays(const tk_table* t, const tk_reads* r, uint64_t windows) {
-  if (!t->n_keys) return true;  // an empty table is written once either way
+  if (!t->n_keys && t->zero_pending) return t->nb * 8 <= res_new_slots_per_window(windows) * windows;
   // regions that can get a word: no more than the reads have distinct keys
   double keys = (double)windows;
   const auto it = r->est.find(2 * t->k + t->canonical);
