@@ -468,6 +468,37 @@ def test_table_grows_in_place_of_the_streams(api, monkeypatch):
         r.free()
 
 
+def test_crowded_table_grows_in_place_of_a_stream(api, monkeypatch):
+    """Crowded regions (as above, sorted in one pass) whose table finds no room
+    to grow beside both streams: all but the one that holds the words goes back."""
+    say("crowded_grow_beside_streams")
+    monkeypatch.setenv("TK_ORDER_MIN_READS", "0")
+    monkeypatch.setenv("TK_RESIDENT", "1")
+    monkeypatch.setenv("TK_REGION_KB", "1")
+    seqs = random_reads(18, 900, 100, 150, n_rate=0.001)
+    seq, off = concat(seqs)
+    ok, oc = O.count(seq, off, 25, True)
+    with api.Context(0) as c:
+        r = api.Reads(c, seq, off)
+        first = api.Table(c, 25, True, 64, 0.9)
+        first.count(r)  # the context has its buffers now
+        first.free()
+        t = api.Table(c, 25, True, 64, 0.9)
+        held = api.device_bytes_in_use()
+        # the table the estimate asks for fits (0.9 MB), the one after it (1.6 MB) does not
+        monkeypatch.setenv("TK_DEVICE_ALLOC_LIMIT", str(held + 1_800_000))
+        c.timing(True)
+        t.count(r)
+        c.sync()
+        monkeypatch.delenv("TK_DEVICE_ALLOC_LIMIT")
+        assert c.kernel_time("count_retry")[1] >= 1
+        assert api.device_bytes_in_use() < held - (64 << 20)
+        gk, gc = t.dump()
+        assert np.array_equal(gk, ok) and np.array_equal(gc, oc)
+        t.free()
+        r.free()
+
+
 @pytest.mark.parametrize("resident", ["1", "0"])
 def test_count_reused_blocks(api, ctx, resident, monkeypatch):
     """With the thread's block reuse on, each table takes the block of the
