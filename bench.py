@@ -54,19 +54,19 @@ VOTE_B_PER_WIN, VOTE_B_PER_READ = 64.375, 24.0
 # 5.04 G windows, counters calibrated against kernels of the same access shape), from
 # profiles/large_pe_20M_pairs_count_stats.md.  The counters cannot be read inside this
 # process, so the profiled figures are carried here for roofline.traffic.
-TRAFFIC_B_PER_WIN = {"count": (121.5 + 83.4) / 5.04, "stats": (143.49 + 1.61) / 5.04}
+TRAFFIC_B_PER_WIN = {"count": (121.5 + 83.4) / 5.04, "stats": (138.10 + 1.61) / 5.04}
 # The same for the stressed sample's kernels (37.8 G windows per step), from
 # profiles/stress_150M_pairs_trace.md: FETCH_SIZE + WRITE_SIZE of one job at
 # face value (their random 64-B line reads read as 64 B each, atomics as 32 B
 # of WRITE_SIZE).
-STRESS_TRAFFIC_B_PER_WIN = {"count": (880.30 + 574.82) / 37.8, "stats": (861.49 + 12.01) / 37.8,
-                            "vote": (790.17 + 14.40) / 37.8, "count_merge": (87.79 + 115.15) / 37.8,
-                            "count_scatter": (130.83 + 307.42) / 37.8, "count_hist": (116.33 + 14.80) / 37.8,
-                            "count_regions": (103.86 + 17.54 + 129.94 + 64.96) / 37.8}
+STRESS_TRAFFIC_B_PER_WIN = {"count": (880.30 + 574.82) / 37.8, "stats": (833.72 + 12.02) / 37.8,
+                            "vote": (876.87 + 14.40) / 37.8, "count_merge": (90.69 + 119.34) / 37.8,
+                            "count_scatter": (134.82 + 316.69) / 37.8, "count_hist": (119.57 + 15.19) / 37.8,
+                            "count_regions": (104.29 + 18.83 + 129.94 + 64.96) / 37.8}
 
 
 # every kernel name the library times (TK_LAUNCH / timing names)
-KERNEL_NAMES = ["pack", "read_words", "hll", "sort_pairs", "minimizer", "count", "count_merge", "count_hist",
+KERNEL_NAMES = ["pack", "read_words", "hll", "hll_slots", "sort_pairs", "minimizer", "count", "count_merge", "count_hist",
                 "count_scatter", "count_bounds", "count_regions", "count_retry", "ovf_fold", "ovf_rehash", "rehash",
                 "stats", "select", "select_flags", "scan_u32", "scan_u64", "windows", "gather_stats", "prune",
                 "ctable_build", "vote", "dump", "dump_bins", "dump_count", "histo", "tickets"]

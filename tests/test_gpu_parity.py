@@ -631,7 +631,7 @@ def test_per_read_passes_ticket_modes(api, ctx, small_se, grab, pipe, monkeypatc
 @pytest.mark.parametrize("k,canonical", [(31, True), (31, False), (13, True), (1, True), (20, False)])
 def test_pipelined_scoring_k_and_strand(api, ctx, k, canonical, monkeypatch):
     """The software-pipelined scoring kernel (reads of at most 128 windows,
-    their code words spread over lanes 0-5) for other k and strand-specific
+    every lane loading the code words of its own) for other k and strand-specific
     counts, reads of every length up to 127 + k bases (128 windows) with
     Ns, in locality order, against the oracle."""
     say("pipelined scoring k", k, "canonical", canonical)

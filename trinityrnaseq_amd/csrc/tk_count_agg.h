@@ -21,10 +21,10 @@ constexpr int kReadsPerBlock = 64;
 // occurrences, through the cooperative four-lane add.  Needs cmax >= kMaxRun
 // (k <= 25), so neither the LDS word nor one global add carries more than once.
 //
-// The merge is bound by vector instruction issue (69% of the cycles with the
-// bucketed table and one window per lane and barrier it had before: a wave
-// ran every probe step until its unluckiest lane was done, 222 instructions
-// per 64 windows).  So the lanes run free of each other: a step probes one
+// The merge is bound by vector instruction issue (70% of the cycles, 125
+// instructions per 64 windows; 69% and 222 with the bucketed table and two
+// windows per lane and barrier it had before, where a wave ran every probe step
+// until its unluckiest lane was done).  So the lanes run free of each other: a step probes one
 // slot per lane (a CAS of the window's word; slots are single)
 // and a lane whose window is in rolls to its next one in the same step, about
 // 1.5 steps per window whatever the others need.  Four threads per read, each

@@ -765,7 +765,8 @@ __global__ __launch_bounds__(256) void k_hll(ReadsView rv, uint64_t r_begin, uin
 
 // The keys of a table's slots into the same registers: those of the reads and
 // the table together then estimate their union.  One block of 1,024 threads per
-// CU, four 16-byte loads in flight per thread.
+// CU, four 16-byte loads in flight per thread: bound by the reading of the table
+// (3.2 GB in 0.59 ms, 5.7 TB/s, before a region pass of 3.7 ms).
 __global__ __launch_bounds__(1024) void k_hll_slots(TableView t, uint64_t n_slots, uint32_t sbits,
                                                     uint32_t* __restrict__ regs) {
   __shared__ uint32_t s_reg[kHllRegs];
@@ -1795,13 +1796,13 @@ __device__ __forceinline__ void piped_reads(const ReadsView& rv, uint32_t* ticke
   }
 }
 
-// The scoring pass for reads of at most 128 * CH windows.  Bound by the table
-// lines that miss L2 (44.7 G/s of the 47-49 G/s such lines reach: 4 M pairs,
-// 670 M of 1,008 M lookups miss) once the reads are many, by instruction issue
-// below that.  Eight lookups in flight per lane: with four and the registers
-// for seven waves per SIMD instead of four, 8.6 instead of 6.75 ms for 2 M
-// pairs.  With values in registers, DPP reductions and the LDS exchange of
-// coop_lookup (before: 1.5x the vector instructions): 200 k 76-nt reads
+// The scoring pass for reads of at most 128 * CH windows.  Bound by its table
+// lookups once the reads are many (20 M pairs: 2.86 G lines hit L2, 2.21 G miss;
+// 61 of the 66.7 ms at the 186 and 48.7 G/s that such lines reach one after the
+// other, vector issue 34%), by instruction issue below that.  Eight lookups in
+// flight per lane: with four and the registers for seven waves per SIMD instead
+// of four, 8.6 instead of 6.75 ms for 2 M pairs.  With values in registers, DPP reductions and the LDS exchange of
+// coop_lookup (before: 2.3x the vector instructions): 200 k 76-nt reads
 // 477 -> 362 us, 2 M pairs 7.31 -> 6.75 ms, 20 M pairs 68.3 -> 66.9 ms.
 template <int CH>
 __global__ __launch_bounds__(256, 4) void k_stats_pipe(ReadsView rv, int k, int canonical, TableView t,
@@ -2031,8 +2032,10 @@ __global__ __launch_bounds__(256, 6) void k_vote_pipe(ReadsView rv, int k, int c
 // per_cu; 0 = one block per wpb reads) blocks per CU.  Fewer reads in flight
 // keep a locus' lines in L2, more hide the misses: the passes over reads of at
 // most 128 windows are the same from 4 to 128 (2 M pairs: 6.45 to 6.75 ms; 7.70 at
-// 2), the vote is fastest at 5 (6 M reads: 9.06 ms; 9.40 at 128), reads of
-// 129 to 256 windows at 3 (1.2 M 250-nt reads: 3.48 ms; 3.82 at 4, 4.00 at 128).
+// 2).  The vote takes 5 (at 3 / 5 / 128: 0.5 M reads 1.12 / 1.12 / 1.32 ms, 6 M
+// 10.9 / 10.2 / 10.6, 16 M 27.2 / 24.9 / 25.3), reads of 129 to 256 windows 3 (at 3 /
+// 4 / 128: 0.2 M reads of 250 nt 0.85 / 0.85 / 1.01 ms, 1.2 M 3.88 / 4.22 / 4.38, 4 M
+// 11.80 / 11.85 / 12.03; of 200 nt 1.2 M 3.09 / 3.27 / 3.43, 4 M 9.65 / 9.35 / 9.55).
 static int per_read_grid(tk_ctx* ctx, uint64_t n_reads, int wpb, uint64_t per_cu = 128) {
   if (const char* e = getenv("TK_READ_BLOCKS_PER_CU")) per_cu = strtoull(e, nullptr, 10);
   const uint64_t want = ceil_div(n_reads, (uint64_t)wpb);
