@@ -300,6 +300,27 @@ def test_count_chooses_regions_by_cost(api, ctx, n_reads, expected, prefill, res
     r.free()
 
 
+def test_count_grows_a_new_table_and_takes_regions(api, ctx, monkeypatch):
+    """A new table that the estimate has grown before the passes (and so
+    cleared): 3.6 slots per window are still few for a table without keys."""
+    say("count_grown_choice")
+    from trinityrnaseq_amd import synth
+    monkeypatch.delenv("TK_RESIDENT", raising=False)
+    tx = synth.large_transcriptome(1003, 2000)
+    seq, off = synth.se_reads(tx, 66577, 150, seed=21)
+    seq = seq.tobytes()
+    ok, oc = O.count(seq, off, 25, True)
+    r = api.Reads(ctx, seq, off)
+    t = api.Table(ctx, 25, True, 64, 1.05 * len(ok) / (3.6 * r.windows(25)))
+    t.count(r)
+    assert 3.2 < t.info()["capacity"] / r.windows(25) < 4
+    assert ctx.count_words() > 0
+    gk, gc = t.dump()
+    assert np.array_equal(gk, ok) and np.array_equal(gc, oc)
+    t.free()
+    r.free()
+
+
 @pytest.mark.parametrize("estimated", [True, False])
 def test_count_again_keeps_the_table(api, ctx, estimated, monkeypatch):
     """A table made for a sample's keys does not grow when the region passes

@@ -2720,17 +2720,21 @@ static bool resident_enabled(uint64_t windows) {
 // A new table not yet cleared is written whole either way, by the region pass
 // at 0.39 ms per GB, cleared for the atomics at 0.19: the same cost at 8, 7.5,
 // 7.7, 6.8 and 4.6 slots per window (30 M windows into 0.3 / 1.8 / 5.4 GB: 1.53 /
-// 1.66 / 2.31 ms with atomics, 1.12 / 1.72 / 3.49 with regions).
-constexpr uint64_t kResSlotsPerWindow = 3;
-static uint64_t res_new_slots_per_window(uint64_t windows) { return windows < (1ull << 28) ? 7 : 4; }
+// 1.66 / 2.31 ms with atomics, 1.12 / 1.72 / 3.49 with regions).  One that is
+// empty and cleared (it was grown for this count) costs the writing alone.
+static uint64_t res_slots_per_window(const tk_table* t, uint64_t windows) {
+  if (t->n_keys) return 3;
+  return t->zero_pending && windows < (1ull << 28) ? 7 : 4;
+}
 static bool resident_pays(const tk_table* t, const tk_reads* r, uint64_t windows) {
-  if (!t->n_keys && t->zero_pending) return t->nb * 8 <= res_new_slots_per_window(windows) * windows;
-  // regions that can get a word: no more than the reads have distinct keys
-  double keys = (double)windows;
-  const auto it = r->est.find(2 * t->k + t->canonical);
-  if (it != r->est.end()) keys = std::min(keys, 1.05 * it->second);
-  const double regions = std::min((double)(t->nb >> t->rbits), keys);
-  return regions * (double)(8ull << t->rbits) <= (double)kResSlotsPerWindow * (double)windows;
+  double regions = (double)(t->nb >> t->rbits);
+  if (!t->zero_pending) {  // regions that can get a word: no more than the reads have distinct keys
+    double keys = (double)windows;
+    const auto it = r->est.find(2 * t->k + t->canonical);
+    if (it != r->est.end()) keys = std::min(keys, 1.05 * it->second);
+    regions = std::min(regions, keys);
+  }
+  return regions * (double)(8ull << t->rbits) <= (double)res_slots_per_window(t, windows) * (double)windows;
 }
 
 // Most words in each stream of a count below kResLargeWindows windows: their
@@ -2878,8 +2882,8 @@ constexpr int kNotResident = -1000;
 struct ResSort {
   uint32_t R, F, C, fs = 0;
   bool one_pass;
-  uint64_t ns2_max, nh1, nh2, nh_max;                           // slices of the second pass, histogram words
-  uint64_t hb_off, m_off, rs_off, cs_off, misc_bytes;           // tables of kSlotResMisc, after the slices
+  uint64_t ns2_max, nh1, nh2, nh_max;                  // slices of the second pass, histogram words
+  uint64_t hb_off, m_off, rs_off, cs_off, misc_bytes;  // tables of kSlotResMisc, after the slices
   ResSort(const tk_table* t, uint64_t ns1) {
     R = (uint32_t)(t->nb >> t->rbits);
     one_pass = R <= kResOnePass;
@@ -2960,7 +2964,7 @@ static int count_resident(tk_ctx* c, tk_table* t, const tk_reads* r, const Reads
   if (!whole && cap_chunked < kResMinStreamWords) return kNotResident;  // before the table grows for it
   // the table's final regions must be known before words are grouped by them
   if ((double)(t->n_keys + windows) > 0.9 * (double)(t->nb * 8)) {
-    const double limit = t->max_load * (double)(t->nb * 8);
+    const double slots = (double)(t->nb * 8), limit = t->max_load * slots;
     double est = 0, want = 0;
     auto it = r->est.find(2 * t->k + t->canonical);  // the caller's own estimate of these reads
     const bool known = rb == 0 && re == r->n_reads && it != r->est.end();
@@ -2971,7 +2975,8 @@ static int count_resident(tk_ctx* c, tk_table* t, const tk_reads* r, const Reads
     if (!known || (t->n_keys && want > limit)) {
       rc = hll_estimate(c, r, rb, re, t->k, t->canonical, windows, &est, t->n_keys ? t : nullptr);
       if (rc) return rc == TK_ERR_OOM ? kNotResident : rc;
-      want = !t->n_keys || est > limit ? 1.05 * est + 4096 : 0;
+      // no margin for the estimate's error but where the slots themselves would run out
+      want = !t->n_keys || 1.05 * est > std::min(1.05 * limit, 0.9 * slots) ? 1.05 * est + 4096 : 0;
     }
     if (want > limit) {
       if ((rc = table_zero(c, t))) return rc;  // the rehash reads the old slots
